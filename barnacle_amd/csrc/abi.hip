@@ -1445,10 +1445,11 @@ int bn_first_hit(bn_ctx* ctx, int32_t scene, const bn_pt_params* p, int32_t samp
         c->out_b.ensure(n * 4);
         c->out_c.ensure(n * 4);
         c->ctl.ensure(sizeof(bnd::Ctl));
-        hip_check(hipMemsetAsync(c->ctl.p, 0, sizeof(bnd::Ctl), c->stream), "memset ctl");
+        const bnd::Buffers B = buffers(c);
+        bnd::launch_reset((bnd::Ctl*)c->ctl.p, 0, B.fetch_seg, c->stream);
         bnd::launch_first_hit(s.dev, p->width, p->height, sample_id, p->spp, p->frame_id, (int*)c->out_a.p,
                               (int*)c->out_b.p, (float*)c->out_c.p, (uint32_t*)c->spill.p, c->spill_stride,
-                              &((bnd::Ctl*)c->ctl.p)->fetch[0], grid_trace(c), c->stream);
+                              B.fetch_seg, bnd::kFetchSegs, c->stack_k, grid_trace(c), c->stream);
         hip_check(hipGetLastError(), "kernel launch");
         hip_check(hipMemcpyAsync(inst, c->out_a.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
         hip_check(hipMemcpyAsync(prim, c->out_b.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");

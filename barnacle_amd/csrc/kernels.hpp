@@ -56,7 +56,6 @@ struct Ctl {
     uint32_t q_count[2];      // active queues (this iteration, next iteration)
     uint32_t bin_count[kBins];
     uint32_t sh_count;
-    uint32_t fetch[4];
     uint32_t free_count[2];   // free-slot lists (read by this iteration's regen, filled for the next)
     uint32_t next_pid;        // next path id of the round to issue (may run past the end)
     uint32_t pad;
@@ -195,7 +194,10 @@ void launch_trace_closest(bool count, const DevScene& S, const PathBuf& P, Ctl* 
 void launch_trace_shadow(bool count, const DevScene& S, const PathBuf& P, Ctl* ctl, const uint32_t* shq,
                          const Buffers& B, uint32_t refill, int grid, hipStream_t st, int par = -1,
                          uint32_t* spill = nullptr);
+// fetch: `segs` zeroed counters, kSegStride words apart; stack_k: LDS stack
+// window (16 or 32 entries, the rest in spill).
 void launch_first_hit(const DevScene& S, int w, int h, int sample_id, int spp, int frame_id, int* inst, int* prim,
-                      float* t, uint32_t* spill, size_t spill_stride, uint32_t* fetch, int grid, hipStream_t st);
+                      float* t, uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs, int stack_k, int grid,
+                      hipStream_t st);
 
 }  // namespace bnd

@@ -277,7 +277,6 @@ __global__ void k_reset(Ctl* ctl, int nxt, uint32_t* fetch_seg, int par) {
         ctl->q_count[nxt] = 0;
         ctl->free_count[nxt] = 0;
     }
-    if (i < 4) ctl->fetch[i] = 0;
 }
 
 // ------------------------------------------------------------ trace closest
@@ -286,11 +285,57 @@ __global__ void k_reset(Ctl* ctl, int nxt, uint32_t* fetch_seg, int par) {
 // queue once at least `refill` of them are idle.  The queue is cut into
 // segments with one fetch counter each (a counter serialises its atomics, so
 // one shared counter would cap the whole GPU at one refill per ~11 ns): a
-// wave starts on its own segment and moves on when that one runs dry.
+// wave starts on its own segment and moves on when that one runs dry, to the
+// next segment with rays left.  A queue that the grid's lanes hold at once is
+// dealt out without counters.
 struct SegFetch {
     uint32_t* ctr;    // segs counters, kSegStride words apart, zero at launch
     int segs;
 };
+
+// Rays per wave of a queue that the grid's lanes hold at once, 0 for a longer
+// one: fewer than 64 when that fills less than kSpreadWaves waves (a wave's
+// step runs the code of every item kind its lanes hold, so waves with fewer
+// rays take shorter steps).  A frame of 31k paths and eight bounces takes
+// 1.38 ms with 2048 or 3072 waves, 1.46 with 1024, 1.53 with 512; 4096 and
+// more cost Metropolis rendering 5-10%, whose two traversals share the GPU.
+constexpr uint32_t kSpreadWaves = 2048;
+__device__ __forceinline__ uint32_t dealt_rays(uint32_t count, uint32_t n_waves) {
+    if (count > n_waves * 64u) return 0;
+    const uint32_t spread = min(n_waves, kSpreadWaves);
+    return min(64u, (count + spread - 1) / spread);
+}
+// A segment with rays left, -1 if there is none: every lane reads the counters
+// of two segments, one memory round trip for all of them (a wave that read one
+// counter after the other spent 128 round trips, 0.1 ms, at the end of every
+// launch).  Waves pick different ones (`pick`, a number of the wave's), so
+// that the waves of the segments that run dry first spread over the others
+// (all of them moving on to the same one serialised on its counter: a
+// config-3 step takes 53.2 ms instead of 61.2).
+__device__ __forceinline__ int next_segment(const SegFetch& F, uint32_t pick, uint32_t seg_len, uint32_t count) {
+    constexpr int N = kFetchSegs / 64;
+    const int lane = opaque((int)lane_id());
+    bool some[N];
+    uint32_t rank[N], n = 0;
+    for (int j = 0; j < N; ++j) {
+        const int k = lane + 64 * j;
+        some[j] = false;
+        if (k < F.segs) {
+            const uint32_t lo = (uint32_t)k * seg_len;
+            some[j] = lo + __hip_atomic_load(F.ctr + (size_t)k * kSegStride, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT) < min(count, lo + seg_len);
+        }
+        const uint64_t m = __ballot(some[j]);
+        rank[j] = n + mbcnt(m);
+        n += (uint32_t)__popcll(m);
+    }
+    const uint32_t want = __umulhi(pick, n);
+    for (int j = 0; j < N; ++j) {
+        const uint64_t m = __ballot(some[j] && rank[j] == want);
+        if (m) return 64 * j + __ffsll((unsigned long long)m) - 1;
+    }
+    return -1;
+}
 
 template <bool ANY, bool COUNT, int K, typename Setup, typename Init, typename Done>
 __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uint32_t* stk, uint32_t* spill,
@@ -301,30 +346,40 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
     tr.st = LaneStack<K>{stk + threadIdx.x, (int)blockDim.x, spill + gid, spill_stride, 0};
     tr.clear();
     setup(tr);
+    // wave-uniform values are kept in scalar registers
+    const uint32_t wave = uniform(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    const uint32_t n_waves = gridDim.x * (blockDim.x >> 6);
+    const uint32_t dealt = dealt_rays(count, n_waves);
     const uint32_t seg_len = (count + (uint32_t)F.segs - 1) / (uint32_t)F.segs;
-    int seg = (int)((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % (uint32_t)F.segs);
-    int tried = 0;
-    bool active = false, more = count > 0;
+    int seg = (int)uniform(wave % (uint32_t)F.segs);
+    bool active = false, more = dealt ? wave * dealt < count : count > 0;
     uint32_t item = 0;
     for (;;) {
         const uint64_t idle = __ballot(!active);
         const uint32_t n_idle = (uint32_t)__popcll(idle);
         if (more && n_idle >= refill) {
-            const uint32_t lo = (uint32_t)seg * seg_len;
-            const uint32_t hi = min(count, lo + seg_len);
-            uint32_t* c = F.ctr + (size_t)seg * kSegStride;
-            uint32_t b = 0;
-            if (lane_id() == 0) {
-                const uint32_t seen = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                b = lo + seen < hi ? atomicAdd(c, n_idle) : seg_len;
-            }
-            b = __shfl(b, 0);
-            // idle lanes take [start, start + n_idle) clipped to the segment;
-            // each lane bounds its own item (start may lie past hi)
-            const uint32_t start = lo + b;
-            if (start + n_idle >= hi) {
-                seg = seg + 1 == F.segs ? 0 : seg + 1;
-                if (++tried >= F.segs) more = false;
+            uint32_t start, hi;
+            if (dealt) {
+                start = wave * dealt;
+                hi = min(count, start + dealt);
+                more = false;
+            } else {
+                const uint32_t lo = (uint32_t)seg * seg_len;
+                hi = min(count, lo + seg_len);
+                uint32_t* c = F.ctr + (size_t)seg * kSegStride;
+                uint32_t b = 0;
+                if (lane_id() == 0) {
+                    const uint32_t seen = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    b = lo + seen < hi ? atomicAdd(c, n_idle) : seg_len;
+                }
+                b = uniform(b);
+                // idle lanes take [start, start + n_idle) clipped to the
+                // segment; each lane bounds its own item (start may lie past hi)
+                start = lo + b;
+                if (start + n_idle >= hi) {
+                    seg = next_segment(F, wave * 0x9e3779b9u, seg_len, count);
+                    more = seg >= 0;
+                }
             }
             if (!active) {
                 const uint32_t i = start + mbcnt(idle);
@@ -1246,16 +1301,17 @@ __global__ void k_shade_direct(Work<false> W, PathBuf P, Ctl* ctl, const uint32_
 }
 
 // First hit of one sample per pixel: (instance, primitive, t) in pixel order.
-__global__ __launch_bounds__(256) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
+template <int K>
+__global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
                                                    int frame_id, int* out_inst, int* out_prim, float* out_t,
-                                                   uint32_t* spill, size_t spill_stride, uint32_t* fetch) {
-    __shared__ uint32_t stk[kStackK * 256];
+                                                   uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs) {
+    __shared__ uint32_t stk[K * 256];
     const uint32_t n = (uint32_t)width * (uint32_t)height;
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, false, kStackK>(
-        SegFetch{fetch, 1}, n, stk, spill, spill_stride, 16u, tc,
-        [&](Traversal<kStackK>& tr) { tr.G.set(S); },
-        [&](Traversal<kStackK>& tr, uint32_t p) {
+    persistent_trace<false, false, K>(
+        SegFetch{fetch, segs}, n, stk, spill, spill_stride, 16u, tc,
+        [&](Traversal<K>& tr) { tr.G.set(S); },
+        [&](Traversal<K>& tr, uint32_t p) {
             const int x = (int)(p % (uint32_t)width), y = (int)(p / (uint32_t)width);
             uint32_t rng = xxhash3((uint32_t)x, (uint32_t)y, (uint32_t)(frame_id * spp + sample_id));
             V2 uPix, uLens;
@@ -1264,7 +1320,7 @@ __global__ __launch_bounds__(256) void k_first_hit(DevScene S, int width, int he
             tr.start(camera_ray(S, x, y, uPix, uLens), kInf, S.exact_only != 0);
             tr.take_tlas_root();
         },
-        [&](Traversal<kStackK>& tr, uint32_t p, bool fin, bool) {
+        [&](Traversal<K>& tr, uint32_t p, bool fin, bool) {
             if (fin) {
                 out_inst[p] = tr.hit_inst;
                 out_prim[p] = tr.hit_prim;
@@ -1548,9 +1604,14 @@ void launch_trace_shadow(bool count, const DevScene& S, const PathBuf& P, Ctl* c
     launch_shadow_t<false>(count, B.stack_k, W, P, ctl, shq, nullptr, B, refill, grid, st, par, spill);
 }
 void launch_first_hit(const DevScene& S, int w, int h, int sample_id, int spp, int frame_id, int* inst, int* prim,
-                      float* t, uint32_t* spill, size_t spill_stride, uint32_t* fetch, int grid, hipStream_t st) {
-    hipLaunchKernelGGL(k_first_hit, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst, prim, t,
-                       spill, spill_stride, fetch);
+                      float* t, uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs, int stack_k, int grid,
+                      hipStream_t st) {
+    if (stack_k == 16)
+        hipLaunchKernelGGL(k_first_hit<16>, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst,
+                           prim, t, spill, spill_stride, fetch, segs);
+    else
+        hipLaunchKernelGGL(k_first_hit<32>, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst,
+                           prim, t, spill, spill_stride, fetch, segs);
 }
 
 }  // namespace bnd

@@ -81,7 +81,7 @@ void first_hit_noalloc(Ctx* c, SceneRec& s, const bn_pt_params& p, int sample_id
     // before they are read
     hip_check(hipMemsetAsync(fetch, 0, kNoAllocHdr * 4, st), "memset scratch counter");
     bnd::launch_first_hit(s.dev, p.width, p.height, sample_id, p.spp, p.frame_id, out_inst, out_prim, out_t, spill,
-                          kNoAllocLanes, fetch, kNoAllocBlocks, st);
+                          kNoAllocLanes, fetch, 1, bnd::kStackK, kNoAllocBlocks, st);
     hip_check(hipGetLastError(), "kernel launch");
     hip_check(hipMemcpyAsync(inst, out_inst, n * 4, hipMemcpyDeviceToHost, st), "D2H");
     hip_check(hipMemcpyAsync(prim, out_prim, n * 4, hipMemcpyDeviceToHost, st), "D2H");

@@ -7,6 +7,14 @@
 namespace bnd {
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
+// A value every lane of the wave holds (lane 0's), in a scalar register.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+// v, computed anew where it is used: what is derived from it is not kept in
+// registers across a loop.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
 // Lanes below this one whose bit is set in m.
 __device__ __forceinline__ uint32_t mbcnt(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
