@@ -954,6 +954,11 @@ void autotune(Ctx* c, const bn_batch_item* items, int n, int flags, bn_tune_resu
     }
 }
 
+// Chain mutations per launch of the one-wave-per-chain kernel: a launch waits
+// for its slowest chain (1024 chains: 63.5 ms with 128 mutations a launch, 57.8
+// with 1024), but should not last much longer than 0.2 s.
+constexpr int64_t kMltLaunch = 1 << 20;
+
 // PSSMLTIntegrator.Render (Extensions/Integrator/PSSMLT.fs:379-414): the
 // bootstrap paths and the chains run as wavefronts on the device; the mean
 // bootstrap luminance B (Array.average, sequential) and the bootstrap alias
@@ -1072,7 +1077,14 @@ void render_pssmlt(Ctx* c, SceneRec& sc, const bn_mlt_params& p, float* film_hos
             bnd::launch_mlt_chain_init(M, dp, (const float*)c->m_aprob.p, (const int*)c->m_aidx.p, c0, n, s);
             run_paths(false, c0, n);                                 // replay of the bootstrap path
             bnd::launch_mlt_replay_done(P, M, dp, c0, n, s);
-            for (int m = 0; m < mpc; ++m) {
+            const bool waves = n <= c->mlt_wave_chains && p.max_depth <= bnd::kMltWaveDepth;
+            const int per = (int)std::max<int64_t>(64, kMltLaunch / std::max(n, 1024));
+            for (int m = 0; waves && m < mpc; m += per) {
+                Timed tm(T, "mlt_wave_chains", s);
+                bnd::launch_mlt_wave_chains(sc.dev, M, dp, (float*)c->film.p, BF, n, std::min(per, mpc - m),
+                                            p.max_depth, p.rr_depth, 4 * c->n_cu, (int)(c->spill_stride / 64), s);
+            }
+            for (int m = 0; !waves && m < mpc; ++m) {
                 run_paths(false, c0, n);
                 { Timed tm(T, "mlt_accept", s); bnd::launch_mlt_accept(P, M, dp, (float*)c->film.p, n, s); }
             }
@@ -1515,6 +1527,9 @@ extern "C" int bn_set_option(bn_ctx* ctx, const char* key, int64_t value) {
         } else if (k == "overlap_shadow") {
             if (value < 0 || value > 1) throw Error(BN_E_INVALID, "overlap_shadow must be 0 or 1");
             c->overlap_shadow = value != 0;
+        } else if (k == "mlt_wave_chains") {
+            if (value < 0 || value > ((int64_t)1 << 26)) throw Error(BN_E_INVALID, "mlt_wave_chains out of range");
+            c->mlt_wave_chains = (int)value;
         } else if (k == "bvh_small") {
             if (value < 128 || value > 512) throw Error(BN_E_INVALID, "bvh_small must be in [128, 512]");
             c->bvh_small = (int)value;

@@ -10,6 +10,7 @@
 #include "kernels.hpp"
 #include "kernels_mlt.hpp"
 #include "shading.hpp"
+#include "traverse.hpp"
 #include "wave.hpp"
 
 namespace bnd {
@@ -51,6 +52,18 @@ __device__ __forceinline__ float erf_inv(float x) {
     p = fmaf(p, w, 0.00943887047f);
     p = fmaf(p, w, 1.00167406f);
     return fmaf(p, w, 2.83297682f) * x;
+}
+
+// The catch-up mutation of a sample over n small steps (PSSMLT.fs:106-135):
+// Gaussian in one draw, Kelemen one term per step.
+__device__ __forceinline__ float gaussian_step(float u, float sigma, int n, float v) {
+    const float ns = sqrtf(2.0f) * erf_inv(fmaf(2.0f, u, -1.0f));
+    return fmaf(ns, sigma * sqrtf((float)n), v);
+}
+__device__ __forceinline__ float kelemen_term(float u, float a, float eps_max) {
+    const float u1 = u - 0.5f;
+    const float u2 = u1 < 0.0f ? 1.0f + 2.0f * u1 : 2.0f * u1;
+    return copysignf(eps_max * exp_f(-a * u2), u1);
 }
 
 // MLTSampler of one chain (PSSMLT.fs:35-150), loaded into registers for one
@@ -110,16 +123,12 @@ struct ChainSampler {
         } else {
             float val;
             if (M->strategy == 0) {
-                const float ns = sqrtf(2.0f) * erf_inv(fmaf(2.0f, lcg(inner), -1.0f));
-                const float es = M->sigma * sqrtf((float)(cur - lm));
-                val = fmaf(ns, es, v);
+                val = gaussian_step(lcg(inner), M->sigma, cur - lm, v);
             } else {
                 val = v;
                 const float a = log_f(M->eps_max / M->eps_min);
                 for (int k = lm; k <= cur - 1; ++k) {
-                    const float u1 = lcg(inner) - 0.5f;
-                    const float u2 = u1 < 0.0f ? 1.0f + 2.0f * u1 : 2.0f * u1;
-                    val = val + copysignf(M->eps_max * exp_f(-a * u2), u1);
+                    val = val + kelemen_term(lcg(inner), a, M->eps_max);
                 }
             }
             v = val - floorf(val);
@@ -194,6 +203,49 @@ __global__ __launch_bounds__(256) void k_mlt_start(DevScene S, PathBuf P, MltBuf
     }
 }
 
+// NEE set-up, BSDF sampling and Russian roulette of one vertex from its seven
+// primary samples (PSSMLT.fs:199-243).
+struct MltVertex {
+    bool shadow, cont;                // casts a shadow ray / the path continues
+    V3 sh_d, nee_a, nee_b;            // shadow ray from g.p, factors of its NEE term
+    float sh_t;
+    V3 d, beta;                       // continuing ray from g.p
+    float pdf;
+};
+__device__ __forceinline__ void mlt_scatter(const DevScene& S, const Ray& r, const Geom& g, int mat, V3 beta,
+                                            float uLight, V2 uEmit, float uLobe, V2 uBSDF, float uRR, int depth,
+                                            int max_depth, int rr_depth, MltVertex& v) {
+    const Mat m = load_mat(S, mat);
+    const V3 wo_l = to_local(g, -r.d);
+    const LightSample ls = light_sample(S, g.p, uLight, uEmit);
+    v.shadow = false;
+    v.cont = false;
+    if (ls.pdf != 0.0f) {
+        const BSDF e = mat_eval(m, wo_l, to_local(g, ls.wi));
+        const float dist = length(ls.p - g.p);
+        v.sh_t = dist - 1e-3f;
+        v.sh_d = ls.wi;
+        v.nee_a = beta * e.f;
+        v.nee_b = ls.L * rcp_e(e.pdf + ls.pdf);
+        v.shadow = true;
+    }
+    V3 wi_l;
+    const BSDF bs = mat_sample(m, wo_l, uLobe, uBSDF, wi_l);
+    if (bs.pdf != 0.0f) {
+        v.d = to_world(g, wi_l);
+        beta = beta * bs.f * rcp_e(bs.pdf);
+        v.cont = true;
+        if (depth >= rr_depth) {
+            const float q = min_n(1.0f, max_n(beta.x, max_n(beta.y, beta.z)));
+            if (uRR < q) beta = beta * rcp_e(q);
+            else v.cont = false;
+        }
+        v.beta = beta;
+        v.pdf = bs.pdf;
+    }
+    v.cont = v.cont && depth + 1 < max_depth;
+}
+
 // PSSMLTIntegrator.Li after a closest hit (PSSMLT.fs:184-243): emission with
 // MIS, then seven primary samples drawn for every hit, then NEE set-up, BSDF
 // sampling and Russian roulette.  The NEE term is applied by trace_shadow.
@@ -244,34 +296,21 @@ __global__ __launch_bounds__(256) void k_shade_mlt(DevScene S, PathBuf P, MltBuf
             const float uRR = smp.ensure(s0 + 6, rs[6]);
             smp.store();
             if (info.z >= 0) {
-                const Mat m = load_mat(S, info.z);
-                const V3 wo_l = to_local(g, -r.d);
-                const LightSample ls = light_sample(S, g.p, uLight, uEmit);
-                if (ls.pdf != 0.0f) {
-                    const BSDF e = mat_eval(m, wo_l, to_local(g, ls.wi));
-                    const float dist = length(ls.p - g.p);
-                    P.sh_o[slot] = f4(g.p, dist - 1e-3f);
-                    P.sh_d[slot] = f4(ls.wi, 0.0f);
-                    P.nee_a[slot] = f4(beta * e.f, 0.0f);
-                    P.nee_b[slot] = f4(ls.L * rcp_e(e.pdf + ls.pdf), 0.0f);
-                    shadow = true;
+                MltVertex v;
+                mlt_scatter(S, r, g, info.z, beta, uLight, uEmit, uLobe, uBSDF, uRR, depth, max_depth, rr_depth, v);
+                shadow = v.shadow;
+                cont = v.cont;
+                if (shadow) {
+                    P.sh_o[slot] = f4(g.p, v.sh_t);
+                    P.sh_d[slot] = f4(v.sh_d, 0.0f);
+                    P.nee_a[slot] = f4(v.nee_a, 0.0f);
+                    P.nee_b[slot] = f4(v.nee_b, 0.0f);
                 }
-                V3 wi_l;
-                const BSDF bs = mat_sample(m, wo_l, uLobe, uBSDF, wi_l);
-                if (bs.pdf != 0.0f) {
-                    const V3 wi = to_world(g, wi_l);
-                    beta = beta * bs.f * rcp_e(bs.pdf);
-                    cont = true;
-                    if (depth >= rr_depth) {
-                        const float q = min_n(1.0f, max_n(beta.x, max_n(beta.y, beta.z)));
-                        if (uRR < q) beta = beta * rcp_e(q);
-                        else cont = false;
-                    }
+                if (cont) {
                     P.o[slot] = f4(g.p, 0.0f);
-                    P.d[slot] = f4(wi, bs.pdf);
-                    P.beta[slot] = f4(beta, 0.0f);
+                    P.d[slot] = f4(v.d, v.pdf);
+                    P.beta[slot] = f4(v.beta, 0.0f);
                 }
-                cont = cont && depth + 1 < max_depth;
             }
             P.L[slot] = f4(L, 0.0f);
         }
@@ -365,6 +404,213 @@ __global__ void k_mlt_accept(PathBuf P, MltBuf M, MltParamsDev p, float* film, i
     M.state[i] = st;
 }
 
+// ------------------------------------------------- one wave per chain
+// Few chains leave the wavefront above latency-bound: each of a mutation's
+// bounces is six launches for a handful of waves.  Here a wave owns a chain
+// and runs its mutations one after the other without leaving the kernel.  All
+// lanes hold the path (the same values: no divergence, one memory
+// transaction); what a mutation does many times over is spread over them: the
+// samples of a vertex are mutated side by side, eight lanes each, and a
+// rejection restores 64 samples at a time.  The primary samples live in LDS
+// for the launch.
+//
+// The draws of a sample depend on its own record only through their number, so
+// every sample's first random state is known from a prefix sum, by skipping
+// the LCG ahead; terms are added in the reference's order, so a chain's
+// trajectory is that of the wavefront, bit for bit.
+__device__ __forceinline__ uint32_t lcg_skip(uint32_t s, uint32_t n) {
+    uint32_t a = 0x000343fdu, c = 0x00269ec3u;               // s -> a*s + c, squared step by step
+    while (__ballot(n != 0) != 0) {
+        if (n & 1) s = a * s + c;
+        c = (a + 1u) * c;
+        a = a * a;
+        n >>= 1;
+    }
+    return s;
+}
+template <int LANE>
+__device__ __forceinline__ float group_lane(float v) {       // lane LANE of each group of eight
+    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (LANE << 5) | 0x18));
+}
+struct WaveChain {
+    const MltBuf& M;
+    float4* xs;             // LDS: the chain's records
+    float log_ratio;        // ln(eps_max / eps_min)
+    uint32_t inner;
+    int cur, last_large, init;
+    bool large;
+    // EnsureReady of samples [s0, s0 + N), N <= 8, in order; group g of eight
+    // lanes holds sample s0 + g.  Returns the lane's group's value.
+    __device__ __forceinline__ float ensure(int s0, int N) {
+        const int lane = (int)lane_id(), g = lane >> 3, q = lane & 7;
+        const int i = s0 + g;
+        const bool mine = g < N;
+        float v = 0.0f;
+        int lm = 0;
+        if (mine && i < init) {
+            const float4 r = xs[i];
+            v = r.x; lm = __float_as_int(r.z);
+        }
+        const bool stale = lm < last_large;                  // catch up with the last large step first
+        lm = stale ? last_large : lm;
+        const int steps = large || M.strategy == 0 ? 1 : max(cur - lm, 0);
+        const uint32_t draws = mine ? (uint32_t)((stale ? 1 : 0) + steps) : 0u;
+        uint32_t before = 0, total = 0;
+        for (int k = 0; k < N; ++k) {
+            const uint32_t d = (uint32_t)__builtin_amdgcn_readlane((int)draws, 8 * k);
+            if (k < g) before += d;
+            total += d;
+        }
+        uint32_t rng = lcg_skip(inner, before);
+        inner = lcg_skip(inner, total);
+        if (mine && stale) v = lcg(rng);
+        const float vb = v;
+        const int mb = lm;
+        if (large) {
+            v = lcg(rng);
+        } else {
+            float val = v;
+            if (M.strategy == 0) {
+                val = gaussian_step(lcg(rng), M.sigma, cur - lm, v);
+            } else {
+                // lane q computes terms q, q + 8, ... of its group's sample
+                for (int k = 0; k < q; ++k) (void)lcg(rng);
+                for (int k = 0; __ballot(mine && k < steps) != 0; k += 8) {
+                    uint32_t r = rng;
+                    const float t = kelemen_term(lcg(r), log_ratio, M.eps_max);
+                    for (int j = 0; j < 8; ++j) (void)lcg(rng);
+                    const int left = steps - k;
+                    float u;
+                    u = group_lane<0>(t); val = left > 0 ? val + u : val;
+                    u = group_lane<1>(t); val = left > 1 ? val + u : val;
+                    u = group_lane<2>(t); val = left > 2 ? val + u : val;
+                    u = group_lane<3>(t); val = left > 3 ? val + u : val;
+                    u = group_lane<4>(t); val = left > 4 ? val + u : val;
+                    u = group_lane<5>(t); val = left > 5 ? val + u : val;
+                    u = group_lane<6>(t); val = left > 6 ? val + u : val;
+                    u = group_lane<7>(t); val = left > 7 ? val + u : val;
+                }
+            }
+            v = val - floorf(val);
+        }
+        if (mine && q == 0) xs[i] = make_float4(v, vb, __int_as_float(cur), __int_as_float(mb));
+        wave_sync();
+        init = max(init, s0 + N);
+        return v;
+    }
+    __device__ __forceinline__ float of(float v, int g) const {     // group g's value, in every lane
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 8 * g));
+    }
+};
+
+constexpr int kMltWaveK = 16;
+// `mutations` mutations of each of the chains [0, n) (PSSMLT.fs:333-373).
+// WAVES per SIMD: alone on its SIMD a wave may use every register; where there
+// are more chains than SIMDs four waves share one, at 128 VGPRs, with spills
+// (1024 chains: 63.5 ms alone, 67.9 ms with four; 16384: 47.1 and 36.6 ms).
+template <int WAVES>
+__global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBuf M, MltParamsDev p, float* film,
+                                                           uint32_t* spill, size_t spill_stride, int n,
+                                                           int mutations, int nx, int max_depth, int rr_depth) {
+    extern __shared__ float4 xs[];
+    __shared__ uint32_t stk[kMltWaveK * 64];
+    const int lane = (int)lane_id();
+    Traversal<kMltWaveK> tr;
+    tr.st = LaneStack<kMltWaveK>{stk + lane, 64, spill + (size_t)blockIdx.x * 64 + lane, spill_stride, 0};
+    tr.clear();
+    tr.G.set(S);
+    // a whole traversal of one ray, the same in every lane
+    auto trace = [&](const Ray& r, float tmax, bool any) {
+        tr.start(r, tmax, S.exact_only != 0);
+        tr.take_tlas_root();
+        if (!(tmax == tmax)) tr.empty();
+        bool found = false;
+        while (tr.step_fast(any, found)) {}
+        if (any) tr.clear();
+        return found;
+    };
+    for (int c = blockIdx.x; c < n; c += gridDim.x) {
+        WaveChain smp{M, xs, log_f(M.eps_max / M.eps_min), M.inner[c]};
+        int4 st = M.state[c];
+        smp.cur = st.x; smp.last_large = st.y; smp.init = st.z; smp.large = st.w != 0;
+        for (int k = lane; k < nx; k += 64)
+            xs[k] = k < smp.init ? M.xs[(size_t)k * M.cap + c] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        wave_sync();
+        uint32_t outer = M.outer[c];
+        float4 lc = M.Lcur[c];
+        V3 rad = xyz(M.rad[c]);
+        int pix_cur = M.pix_cur[c], accepted = M.accepted[c];
+        for (int m = 0; m < mutations; ++m) {
+            // StartIteration and the camera ray (PSSMLT.fs:58-61, 333-345)
+            smp.large = smp.cur == 0 || lcg(smp.inner) < p.large_step_prob;
+            smp.cur = smp.cur + 1;
+            const float u = smp.ensure(0, 4);
+            const float upx = smp.of(u, 0) * (float)p.width, upy = smp.of(u, 1) * (float)p.height;
+            const int ix = min(p.width - 1, sat_int(upx)), iy = min(p.height - 1, sat_int(upy));
+            Ray r = camera_ray(S, ix, iy, V2{upx - (float)ix, upy - (float)iy}, V2{smp.of(u, 2), smp.of(u, 3)});
+            const int pix_new = iy * p.width + ix;
+            V3 L = mk(0, 0, 0), beta = mk(1, 1, 1);
+            float prev_pdf = 0.0f;
+            for (int depth = 0; depth < max_depth; ++depth) {
+                trace(r, kInf, false);
+                if (tr.hit_inst < 0) break;
+                const Geom g = hit_geometry(S, r, tr.hit_inst, tr.hit_prim, tr.t);
+                const int4 info = S.insts[tr.hit_inst].info;
+                if (info.w >= 0) {
+                    V3 Le;
+                    float lpdf;
+                    light_eval(S, tr.hit_inst, r.o, g, Le, lpdf);
+                    const float w = depth == 0 ? 1.0f : prev_pdf * rcp_e(lpdf + prev_pdf);
+                    L = fma3(beta, Le * w, L);
+                }
+                const float s = smp.ensure(4 + 7 * depth, 7);
+                if (info.z < 0) break;
+                MltVertex v;
+                mlt_scatter(S, r, g, info.z, beta, smp.of(s, 0), V2{smp.of(s, 1), smp.of(s, 2)}, smp.of(s, 3),
+                            V2{smp.of(s, 4), smp.of(s, 5)}, smp.of(s, 6), depth, max_depth, rr_depth, v);
+                if (v.shadow && !trace({g.p, v.sh_d}, v.sh_t, true)) L = fma3(v.nee_a, v.nee_b, L);
+                if (!v.cont) break;
+                r = {g.p, v.d};
+                beta = v.beta;
+                prev_pdf = v.pdf;
+            }
+            const V3 Ln = L * rcp_e(1.0f);
+            const float yn = luminance(Ln), y = lc.w;
+            const V3 Lc = xyz(lc);
+            const float a = min_n(1.0f, yn / y);
+            const float w_old = (1.0f - a) / fmaf(y, p.inv_b, p.large_step_prob);
+            rad = rad + w_old * Lc;
+            const float w_new = (a + (smp.large ? 1.0f : 0.0f)) / fmaf(yn, p.inv_b, p.large_step_prob);
+            if (lcg(outer) < a) {
+                ++accepted;
+                if (lane == 0) film_add(film, p, pix_cur, rad * p.inv_eff);
+                rad = w_new * Ln;
+                pix_cur = pix_new;
+                lc = f4(Ln, yn);
+                if (smp.large) smp.last_large = smp.cur;         // Accept()
+            } else {
+                if (a > 0.0f && lane == 0) film_add(film, p, pix_new, (w_new * p.inv_eff) * Ln);
+                for (int k = lane; k < smp.init; k += 64) {      // Reject()
+                    const float4 q = xs[k];
+                    xs[k] = make_float4(q.y, q.y, q.w, q.w);
+                }
+                wave_sync();
+                smp.cur = smp.cur - 1;
+            }
+        }
+        for (int k = lane; k < smp.init; k += 64) M.xs[(size_t)k * M.cap + c] = xs[k];
+        if (lane == 0) {
+            M.inner[c] = smp.inner;
+            M.state[c] = make_int4(smp.cur, smp.last_large, smp.init, smp.large ? 1 : 0);
+            M.outer[c] = outer;
+            M.Lcur[c] = lc;
+            M.rad[c] = f4(rad, 0.0f);
+            M.pix_cur[c] = pix_cur;
+            M.accepted[c] = accepted;
+        }
+    }
+}
+
 // Final Film.Accumulate of a chain (PSSMLT.fs:375).
 __global__ void k_mlt_finish(MltBuf M, MltParamsDev p, float* film, int* accepted_out, int c0, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -408,6 +654,19 @@ void launch_mlt_accept(const PathBuf& P, const MltBuf& M, const MltParamsDev& p,
 void launch_mlt_finish(const MltBuf& M, const MltParamsDev& p, float* film, int* accepted, int c0, int n,
                        hipStream_t st) {
     hipLaunchKernelGGL(k_mlt_finish, dim3(blocks(n)), dim3(256), 0, st, M, p, film, accepted, c0, n);
+}
+
+void launch_mlt_wave_chains(const DevScene& S, const MltBuf& M, const MltParamsDev& p, float* film, const Buffers& B,
+                            int n, int mutations, int max_depth, int rr_depth, int n_simd, int grid,
+                            hipStream_t st) {
+    const int nx = 4 + 7 * max_depth;
+    const size_t lds = (size_t)nx * sizeof(float4);
+    if (n <= n_simd)
+        hipLaunchKernelGGL(k_mlt_wave_chains<1>, dim3(min(n, grid)), dim3(64), lds, st, S, M, p, film, B.spill,
+                           B.spill_stride, n, mutations, nx, max_depth, rr_depth);
+    else
+        hipLaunchKernelGGL(k_mlt_wave_chains<4>, dim3(min(n, grid)), dim3(64), lds, st, S, M, p, film, B.spill,
+                           B.spill_stride, n, mutations, nx, max_depth, rr_depth);
 }
 
 }  // namespace bnd

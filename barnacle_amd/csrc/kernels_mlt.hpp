@@ -38,6 +38,13 @@ void launch_shade_mlt(bool fresh, const DevScene& S, const PathBuf& P, const Mlt
 void launch_mlt_boot_done(const PathBuf& P, float* weights, int id0, int n, hipStream_t st);
 void launch_mlt_replay_done(const PathBuf& P, const MltBuf& M, const MltParamsDev& p, int c0, int n, hipStream_t st);
 void launch_mlt_accept(const PathBuf& P, const MltBuf& M, const MltParamsDev& p, float* film, int n, hipStream_t st);
+// `mutations` mutations of each chain [0, n), one wave per chain, at most
+// `grid` waves (the spill area holds 64 lanes each).  The chain's records must
+// fit its LDS: max_depth <= kMltWaveDepth.
+constexpr int kMltWaveDepth = 256;
+void launch_mlt_wave_chains(const DevScene& S, const MltBuf& M, const MltParamsDev& p, float* film, const Buffers& B,
+                            int n, int mutations, int max_depth, int rr_depth, int n_simd, int grid,
+                            hipStream_t st);
 void launch_mlt_finish(const MltBuf& M, const MltParamsDev& p, float* film, int* accepted, int c0, int n,
                        hipStream_t st);
 

@@ -397,7 +397,7 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
         // Every lane steps: an idle lane's cleared state has no item, so its
         // step does nothing (and keeps the loop free of a per-lane branch).
         bool found = false;
-        const bool going = COUNT ? tr.template step<ANY, COUNT>(tc, found) : tr.template step_fast<ANY>(found);
+        const bool going = COUNT ? tr.template step<ANY, COUNT>(tc, found) : tr.step_fast(ANY, found);
         const bool fin = active && !going;
         if (__ballot(fin) != 0) {
             done(tr, item, fin, found);

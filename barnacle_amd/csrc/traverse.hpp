@@ -268,14 +268,13 @@ struct Traversal {
     }
 
     // One triangle of the current BLAS leaf.  Returns false on an any-hit.
-    template <bool ANY>
-    __device__ __forceinline__ bool do_tri(bool& found) {
+    __device__ __forceinline__ bool do_tri(bool any, bool& found) {
         const int idx = bl_cur++;
         const Tri tr = load_tri(G.tris, idx);
         if (!box_tri(tr)) return true;
         float tt;
         if (tri_hit(tr, co, cd, t, tt)) {
-            if (ANY) { found = true; return false; }
+            if (any) { found = true; return false; }
             t = tt;
             hit_inst = cur_inst;
             hit_prim = idx - tri_base;
@@ -285,8 +284,7 @@ struct Traversal {
 
     // One instance of the current TLAS leaf: a sphere is intersected, a mesh
     // BLAS is entered.  Returns false on an any-hit.
-    template <bool ANY>
-    __device__ __forceinline__ bool do_inst(bool& found) {
+    __device__ __forceinline__ bool do_inst(bool any, bool& found) {
         const int idx = tl_cur++;
         const DevInst& I = G.insts[idx];
         if (!box(xyz(I.lo), xyz(I.hi))) return true;
@@ -307,7 +305,7 @@ struct Traversal {
             float tt;
             int br;
             if (sphere_hit(I.lo.w, oo, od, t, tt, br)) {
-                if (ANY) { found = true; return false; }
+                if (any) { found = true; return false; }
                 t = tt;
                 hit_inst = idx;
                 hit_prim = br;
@@ -336,12 +334,11 @@ struct Traversal {
     // One item of the fast traversal (all lanes of a wave advance together,
     // whatever kind of item each has: measured faster than advancing only the
     // lanes of the most common kind).  Returns false when the traversal has
-    // finished or an any-hit query found its hit.
-    template <bool ANY>
-    __device__ __forceinline__ bool step_fast(bool& found) {
+    // finished or an any-hit query (`any`, per lane) found its hit.
+    __device__ __forceinline__ bool step_fast(bool any, bool& found) {
         const int kind = next_kind();
-        if (kind == kItemTri) return do_tri<ANY>(found);
-        if (kind == kItemInst) return do_inst<ANY>(found);
+        if (kind == kItemTri) return do_tri(any, found);
+        if (kind == kItemInst) return do_inst(any, found);
         if (kind == kItemTNode) { do_node(); return true; }
         return false;
     }
