@@ -425,6 +425,7 @@ void check_pt_params(const bn_pt_params& p) {
 }
 
 constexpr int kIterBlock = 8;     // iterations between two drain checks (even)
+constexpr int kMaxGraphIters = 64;  // longest round captured whole
 constexpr size_t kMaxGraphs = 64;  // captured graphs kept per context
 
 // Paths per round.  By default a round holds no more paths than there are
@@ -433,33 +434,42 @@ constexpr size_t kMaxGraphs = 64;  // captured graphs kept per context
 // costs more in uncoalesced path-state access than it saves in bounce tails.
 size_t window_paths(const Ctx* c) { return c->window_paths ? c->window_paths : c->chunk_slots; }
 
+// Iterations after which every path of a round that starts them all at once
+// has retired (slot rounds take an even number).
+int round_iterations(bnd::Integrator kind, const bnd::Buffers& B, int max_depth) {
+    return bnd::compact_round(kind, B) ? std::max(max_depth, 1) : std::max((max_depth + 1) / 2 * 2, 2);
+}
+
 // One round: its paths stream through L.n_slots slots until every path has
-// retired, checked on the host after every block of kIterBlock iterations
-// (a captured graph of one block when `block` is set).
+// retired.  When they all start at once their iterations run back to back;
+// else the host looks after every block of kIterBlock iterations.  `block`: a
+// captured graph of the round's iterations, or of one block.
 void run_round(Ctx* c, bool batch, bnd::Integrator kind, const bnd::Launch& L, const bnd::PathBuf& P, bnd::Ctl* ctl,
                const bnd::Buffers& B, uint32_t n_paths, int max_depth, bool count, Hook* hook,
                hipGraphExec_t block) {
     hipStream_t s = L.stream;
-    bnd::enqueue_round_begin(batch, L, P, ctl, B, hook);
+    if (L.at_once) {
+        // Every path starts in the first iteration and retires within
+        // max_depth iterations: no need to look whether the round has drained.
+        if (block) {
+            Timed t(c->timer, "round", s);
+            hip_check(hipGraphLaunch(block, s), "graph launch");
+        } else {
+            bnd::enqueue_round_begin(kind, L, P, ctl, B, hook);
+            bnd::enqueue_iterations(batch, kind, L, P, ctl, B, round_iterations(kind, B, max_depth), count, hook);
+        }
+        bnd::enqueue_round_end(batch, kind, L, P, ctl, B, hook);
+        return;
+    }
+    bnd::enqueue_round_begin(kind, L, P, ctl, B, hook);
     // every path needs at most max_depth + 1 iterations once it has a slot
     const int64_t limit = ((int64_t)n_paths / L.n_slots + 2) * (int64_t)(max_depth + 2) * 2 + 4 * kIterBlock;
     int64_t iters = 0;
-    // A round whose paths all fit its slots issues every path in its first
-    // iteration, and a path retires within max_depth iterations of its
-    // issue: the first check waits until then (the iterations in between run
-    // back to back, with no host synchronisation between blocks).
-    const bool all_at_once = n_paths <= L.n_slots;
     for (;;) {
-        int n = kIterBlock;
-        if (iters == 0 && all_at_once)
-            n = std::max(kIterBlock, block ? (max_depth + kIterBlock - 1) / kIterBlock * kIterBlock
-                                           : (max_depth + 1) / 2 * 2);
+        const int n = kIterBlock;
         if (block) {
-            for (int r = 0; r < n / kIterBlock; ++r) {
-                c->timer.begin("iteration_block", s);
-                hip_check(hipGraphLaunch(block, s), "graph launch");
-                c->timer.end(s);
-            }
+            Timed t(c->timer, "iteration_block", s);
+            hip_check(hipGraphLaunch(block, s), "graph launch");
         } else {
             bnd::enqueue_iterations(batch, kind, L, P, ctl, B, n, count, hook);
         }
@@ -498,8 +508,9 @@ void render_frames(Ctx* c, SceneRec& sc, const bn_pt_params& p, bnd::Integrator 
     c->film.ensure(film_n * 4);
     c->ctl.ensure(sizeof(bnd::Ctl));
     c->stats.ensure(8 * sizeof(unsigned long long));
-    hip_check(hipMemsetAsync(c->film.p, 0, film_n * 4, s), "memset film");
-    hip_check(hipMemsetAsync(c->stats.p, 0, 8 * sizeof(unsigned long long), s), "memset stats");
+    // the first samples start the film; without any it is black
+    if (p.spp <= 0) hip_check(hipMemsetAsync(c->film.p, 0, film_n * 4, s), "memset film");
+    if (stats) hip_check(hipMemsetAsync(c->stats.p, 0, 8 * sizeof(unsigned long long), s), "memset stats");
     bn_trace_stats acc{};
     bnd::PathBuf P = path_buf(c);
     bnd::Ctl* ctl = (bnd::Ctl*)c->ctl.p;
@@ -526,6 +537,7 @@ void render_frames(Ctx* c, SceneRec& sc, const bn_pt_params& p, bnd::Integrator 
         it.ns = std::min(ns, p.spp - s0);
         it.path_count = it.ns * it.p_pad;
         L.item = it;
+        L.at_once = (size_t)it.path_count <= slots;
         run_round(c, false, kind, L, P, ctl, B, (uint32_t)it.path_count, it.max_depth, stats != nullptr, &hook,
                   nullptr);
     }
@@ -612,7 +624,6 @@ void backward_pt(Ctx* c, SceneRec& sc, const bn_pt_params& p, const float* d_fil
     c->a_gmat.ensure((size_t)std::max(1, n_mat) * 16);
     c->a_glight.ensure((size_t)std::max(1, n_light) * 16);
     c->a_dfilm.upload(d_film, film_n * 4, s);
-    hip_check(hipMemsetAsync(c->film.p, 0, film_n * 4, s), "memset film");
     hip_check(hipMemsetAsync(c->a_gmat.p, 0, (size_t)std::max(1, n_mat) * 16, s), "memset gradients");
     hip_check(hipMemsetAsync(c->a_glight.p, 0, (size_t)std::max(1, n_light) * 16, s), "memset gradients");
     bnd::PathBuf P = path_buf(c);
@@ -654,6 +665,7 @@ void backward_pt(Ctx* c, SceneRec& sc, const bn_pt_params& p, const float* d_fil
         it.ns = std::min(ns, p.spp - s0);
         it.path_count = it.ns * it.p_pad;
         L.item = it;
+        L.at_once = (size_t)it.path_count <= slots;
         if (!cached)
             run_round(c, false, bnd::Integrator::Path, L, P, ctl, B, (uint32_t)it.path_count, it.max_depth, false,
                       &hook, nullptr);
@@ -719,7 +731,9 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
     c->b_scenes.upload(scenes.data(), scenes.size() * sizeof(bnd::DevScene), s);
     c->b_items.ensure((size_t)n * sizeof(bnd::RoundItem));
     c->b_hdr.ensure(sizeof(bnd::RoundHeader));
-    hip_check(hipMemsetAsync(c->film.p, 0, film_total * 4, s), "memset film");
+    // an item's first samples start its film; without any it is black
+    if (std::any_of(base.begin(), base.end(), [](const bnd::RoundItem& it) { return it.spp <= 0; }))
+        hip_check(hipMemsetAsync(c->film.p, 0, film_total * 4, s), "memset film");
     bnd::PathBuf P = path_buf(c);
     bnd::Ctl* ctl = (bnd::Ctl*)c->ctl.p;
     bnd::Launch L{};
@@ -735,15 +749,19 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
     L.stream = s;
     L.n_slots = (uint32_t)slots;
     const bnd::Buffers B = buffers(c);
-    // One captured block of iterations per trace binding: per ray (mixed
-    // rounds), or one scene's geometry in the launch arguments (rounds over
-    // one scene; keyed by everything of the scene that the trace kernels read).
-    auto block_graph = [&](const bnd::Launch& Lr) -> hipGraphExec_t {
-        if (!c->use_graph) return nullptr;
+    // Captured iterations, all of the round's or one block of them, per trace
+    // binding: per ray (mixed rounds), or one scene's geometry in the launch
+    // arguments (rounds over one scene; keyed by everything of the scene that
+    // the trace kernels read).
+    auto block_graph = [&](const bnd::Launch& Lr, int depth) -> hipGraphExec_t {
+        const bool whole = Lr.at_once && bnd::compact_round(bnd::Integrator::Path, B);
+        const int n = whole ? round_iterations(bnd::Integrator::Path, B, depth) : kIterBlock;
+        if (!c->use_graph || n > kMaxGraphIters || (Lr.at_once && !whole)) return nullptr;
         std::string key = "block:" + std::to_string(L.grid_trace) + ":" + std::to_string(L.refill) + ":" +
                           std::to_string(B.stack_k) + ":" + std::to_string(L.n_slots) + ":" +
                           std::to_string((uintptr_t)c->b_items.p) + ":" + std::to_string((uintptr_t)c->b_scenes.p) +
-                          ":" + std::to_string((uintptr_t)c->L_out.p) + ":" + std::to_string((int)L.octant_order) + ":" + std::to_string(L.skip_dark);
+                          ":" + std::to_string((uintptr_t)c->L_out.p) + ":" + std::to_string((int)L.octant_order) + ":" + std::to_string(L.skip_dark) +
+                          ":" + std::to_string(whole ? n : 0) + ":" + std::to_string(Lr.stream2 != nullptr);
         if (Lr.uniform) {
             const bnd::DevScene& d = Lr.scene;
             for (const void* q : {(const void*)d.tlas, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
@@ -756,7 +774,7 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
             if (c->graphs.size() >= kMaxGraphs) c->graphs.clear();   // no earlier round's graph is in flight
             hipGraph_t g;
             hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
-            bnd::enqueue_iterations(true, bnd::Integrator::Path, Lr, P, ctl, B, kIterBlock, false, nullptr);
+            bnd::enqueue_iterations(true, bnd::Integrator::Path, Lr, P, ctl, B, n, false, nullptr);
             hip_check(hipStreamEndCapture(s, &g), "end capture");
             hipGraphExec_t e;
             hip_check(hipGraphInstantiate(&e, g, nullptr, nullptr, 0), "graph instantiate");
@@ -841,13 +859,14 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
         hip_check(hipMemcpyAsync(c->b_hdr.p, &h, sizeof(h), hipMemcpyHostToDevice, s), "round header");
         L.scene = scenes[k0];
         scene_rounds += L.uniform;
-        // A large round over one scene runs eagerly with its shadow rays on the
-        // second stream (as a plain frame does); other rounds replay a graph.
-        const bool overlap = c->overlap_shadow && L.uniform && path >= (1 << 20);
-        L.stream2 = overlap ? c->stream2 : nullptr;
+        L.at_once = (size_t)path <= slots;
+        // The shadow rays run on the second stream (as in a plain frame).  A
+        // large round over one scene runs eagerly; other rounds replay a graph.
+        const bool eager = c->overlap_shadow && L.uniform && path >= (1 << 20);
+        L.stream2 = c->overlap_shadow && (eager || L.at_once) ? c->stream2 : nullptr;
         L.ev_shade = c->ev_shade;
         L.ev_shadow = c->ev_shadow;
-        const hipGraphExec_t exec = overlap ? nullptr : block_graph(L);
+        const hipGraphExec_t exec = eager ? nullptr : block_graph(L, round_depth);
         used_graph = used_graph || exec;
         run_round(c, true, bnd::Integrator::Path, L, P, ctl, B, (uint32_t)path, round_depth, false, &hook, exec);
         hip_check(hipStreamSynchronize(s), "round");

@@ -93,6 +93,7 @@ struct Launch {
     const DevScene* scenes;   // batch mode (device)
     uint32_t n_pix;           // plain mode
     uint32_t n_slots;         // path slots in flight
+    bool at_once;             // every path of the round fits a slot: all start in the first iteration
     int grid_trace, grid_shade;
     // Batch mode: every item of the round traces the geometry of `scene`, so
     // its compact rounds launch the single-scene trace kernels (the scene
@@ -171,9 +172,13 @@ struct LaunchHook {
 // appends new paths after the continuing ones, shading moves the continuing
 // paths to the other copy and retires the ended ones by path id.
 //   iterations: n (even) x [regen, prep, trace_closest, shade, trace_shadow]
+//   (a round whose paths all start at once: regen, then n x [trace_closest,
+//   shade, trace_shadow])
 enum class Integrator { Path, Normal, Adjoint, Direct };
-void enqueue_round_begin(bool batch, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,
+bool compact_round(Integrator kind, const Buffers& B);
+void enqueue_round_begin(Integrator kind, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,
                          LaunchHook* hook);
+// n: even, or the whole of a compact round whose paths all start at once
 void enqueue_iterations(bool batch, Integrator kind, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,
                         int n, bool count, LaunchHook* hook);
 void enqueue_round_end(bool batch, Integrator kind, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,

@@ -187,12 +187,24 @@ __global__ __launch_bounds__(256) void k_regen(Work<BATCH> W, PathBuf P, const C
 // continue from the previous iteration, up to n_slots, with the seeding and
 // primary rays of k_regen.  A path's radiance is accumulated in L_out[path
 // id] for the whole round, from zero here.
+// first: the round's first iteration; the counters need not be set up (its
+// first block sets them, in place of k_ctl_clear and k_prep).
 template <bool BATCH>
-__global__ __launch_bounds__(256) void k_regen_c(Work<BATCH> W, PathBuf X, const Ctl* ctl, int cur,
-                                                 uint32_t n_slots, float4* L_out) {
-    const uint32_t n_act = ctl->q_count[cur];
-    const uint32_t next_pid = ctl->next_pid;
+__global__ __launch_bounds__(256) void k_regen_c(Work<BATCH> W, PathBuf X, Ctl* ctl, int cur, uint32_t n_slots,
+                                                 float4* L_out, bool first, uint32_t* fetch_seg) {
+    const uint32_t n_act = first ? 0 : ctl->q_count[cur];
+    const uint32_t next_pid = first ? 0 : ctl->next_pid;
     const uint32_t n_new = new_paths(n_slots - n_act, next_pid, W.total_paths());
+    if (first && blockIdx.x == 0) {
+        uint32_t* w = reinterpret_cast<uint32_t*>(ctl);
+        for (int i = threadIdx.x; i < (int)(sizeof(Ctl) / 4); i += blockDim.x) w[i] = 0;
+        for (int i = threadIdx.x; i < 2 * kFetchSegs; i += blockDim.x) fetch_seg[(size_t)i * kSegStride] = 0;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            ctl->q_count[cur] = n_new;
+            ctl->next_pid = n_new;
+        }
+    }
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n_new; j += gridDim.x * blockDim.x) {
         const uint32_t pos = n_act + j;
         const uint32_t id = next_pid + j;
@@ -422,6 +434,11 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
                                                        uint32_t refill, unsigned long long* stats, uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = ctl->q_count[cur];
+    // what this iteration's shading counts up from
+    if (blockIdx.x == 0 && threadIdx.x <= kBins) {
+        if (threadIdx.x < kBins) ctl->bin_count[threadIdx.x] = 0;
+        else ctl->q_count[1 - cur] = 0;
+    }
     TraceCount tc{0, 0, 0};
     persistent_trace<false, COUNT, K>(
         SegFetch{seg, kFetchSegs}, count, stk, spill, spill_stride, refill, tc,
@@ -804,13 +821,23 @@ __device__ __forceinline__ void shade_tile(const Work<BATCH>& W, const PathBuf& 
 // nee_a.w.  Blocks stride over the tiles and append in completion order (one
 // atomic per block and output; an order-preserving scan was measured: the
 // traversal of the next bounce ran no faster).  The vertices shaded are
-// counted in bin_count[0].  skip_dark: no shadow ray is cast for an NEE term
+// counted in bin_count[0].  The first block clears the counters that the next
+// iteration's traversals and shadow rays count up from: the closest-hit
+// traversal of this iteration and the shadow rays of the last one are done.
+// skip_dark: no shadow ray is cast for an NEE term
 // that is exactly zero (dark_term), which leaves the film unchanged.
 template <bool BATCH, bool ORDER>
 __global__ __launch_bounds__(256, 3) void k_shade_c(Work<BATCH> W, PathBuf X, PathState Y, Ctl* ctl, int cur,
-                                                    int nxt, float4* L_out, int skip_dark) {
+                                                    int nxt, float4* L_out, int skip_dark, uint32_t* fetch_seg) {
     __shared__ ShadeStage sg;
     const uint32_t total = ctl->q_count[cur];
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < kFetchSegs) fetch_seg[(size_t)threadIdx.x * kSegStride] = 0;
+        else if (threadIdx.x < kFetchSegs + kShadowSegs)
+            fetch_seg[(size_t)(threadIdx.x + nxt * kShadowSegs) * kSegStride] = 0;
+        else if (threadIdx.x == kFetchSegs + kShadowSegs)
+            ctl->shc[nxt] = 0;
+    }
     uint32_t shaded = 0;
     uint32_t* const ctr[2] = {&ctl->q_count[nxt], &ctl->shc[cur]};
     for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += gridDim.x * blockDim.x)
@@ -1194,7 +1221,8 @@ __global__ void k_film(Work<BATCH> W, const float4* L_out, float* film) {
         const uint32_t q =
             ((uint32_t)((y >> 3) * c.tiles_x + (x >> 3)) << 6) | ((uint32_t)(y & 7) << 3) | (uint32_t)(x & 7);
         float* f = film + c.film_offset + 3 * ((size_t)(c.height - y - 1) * c.width + x);
-        float ax = f[0], ay = f[1], az = f[2];
+        float ax = 0.0f, ay = 0.0f, az = 0.0f;                // an item's first samples start its film
+        if (c.s0 > 0) { ax = f[0]; ay = f[1]; az = f[2]; }
         for (int s = 0; s < c.ns; ++s) {
             const float4 L = L_out[(size_t)c.path_base + (size_t)s * c.p_pad + q];
             ax = fmaf(c.inv_spp, L.x * rcp_e(1.0f), ax);
@@ -1378,16 +1406,8 @@ struct Bracket {
     ~Bracket() { if (h) h->end(s); }
 };
 
-template <bool BATCH>
-static void round_begin_t(const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B, LaunchHook* hook) {
-    hipStream_t st = L.stream;
-    { Bracket b(hook, "ctl_clear", st); hipLaunchKernelGGL(k_ctl_clear, dim3(1), dim3(64), 0, st, ctl); }
-    { Bracket b(hook, "init_slots", st);
-      hipLaunchKernelGGL(k_init_slots, dim3(L.grid_shade), dim3(256), 0, st, P, ctl, B.freel[0], L.n_slots); }
-}
-
 // Path-tracing rounds run compact unless material binning is forced.
-static bool compact_round(Integrator kind, const Buffers& B) {
+bool compact_round(Integrator kind, const Buffers& B) {
     return kind == Integrator::Path && B.alt.o != nullptr && B.sort != 1;
 }
 static PathBuf with_state(PathBuf P, const PathState& S) {
@@ -1418,6 +1438,10 @@ static void compact_iterations_t(const Work<BATCH>& W, const Launch& L, const Pa
     // regen, prep and trace_closest of iteration i + 1 run: shade_c(i + 1)
     // waits for trace_shadow(i) (it reuses the shadow arrays and adds to the
     // same radiance slots), and the block ends with both streams joined.
+    // A round whose paths all start in its first iteration (L.at_once) starts
+    // paths and sets its counters up there only: three launches an iteration
+    // (regen and prep of the others took 20 us each time, a tenth of a small
+    // frame).
     const bool overlap = L.stream2 != nullptr;
     hipStream_t st2 = overlap ? L.stream2 : st;
     uint32_t* spill_sh = overlap ? B.spill2 : B.spill;
@@ -1425,27 +1449,32 @@ static void compact_iterations_t(const Work<BATCH>& W, const Launch& L, const Pa
         const int cur = i & 1, nxt = 1 - cur;
         const PathBuf& X = copies[cur];
         const PathBuf& Y = copies[nxt];
-        { Bracket b(hook, "regen", st);
-          hipLaunchKernelGGL(k_regen_c<BATCH>, dim3(grid_c), dim3(256), 0, st, W, X, ctl, cur, L.n_slots,
-                             B.L_out); }
-        { Bracket b(hook, "prep", st);
-          hipLaunchKernelGGL(k_prep<BATCH>, dim3(1), dim3(2 * kFetchSegs), 0, st, W, ctl, cur, B.fetch_seg,
-                             L.n_slots); }
+        const bool first = L.at_once && i == 0;
+        if (first || !L.at_once) {
+            Bracket b(hook, "regen", st);
+            hipLaunchKernelGGL(k_regen_c<BATCH>, dim3(grid_c), dim3(256), 0, st, W, X, ctl, cur, L.n_slots, B.L_out,
+                               first, B.fetch_seg);
+        }
+        if (!L.at_once) {
+            Bracket b(hook, "prep", st);
+            hipLaunchKernelGGL(k_prep<BATCH>, dim3(1), dim3(2 * kFetchSegs), 0, st, W, ctl, cur, B.fetch_seg,
+                               L.n_slots);
+        }
         { Bracket b(hook, "trace_closest", st);
           if (one_scene)
               launch_closest_t<false>(count, B.stack_k, plain_work(L), X, ctl, cur, nullptr, B, L.refill,
                                       L.grid_uniform, st);
           else
               launch_closest_t<BATCH>(count, B.stack_k, W, X, ctl, cur, nullptr, B, L.refill, L.grid_trace, st); }
-        if (overlap) (void)hipStreamWaitEvent(st, L.ev_shadow, 0);
+        if (overlap && i > 0) (void)hipStreamWaitEvent(st, L.ev_shadow, 0);
         { Bracket b(hook, "shade", st);
           const int skip = L.skip_dark == 2 || (L.skip_dark == 1 && !count);
           if (L.octant_order)
               hipLaunchKernelGGL((k_shade_c<BATCH, true>), dim3(grid_c), dim3(256), 0, st, W, X, state_of(Y), ctl,
-                                 cur, nxt, B.L_out, skip);
+                                 cur, nxt, B.L_out, skip, B.fetch_seg);
           else
               hipLaunchKernelGGL((k_shade_c<BATCH, false>), dim3(grid_c), dim3(256), 0, st, W, X, state_of(Y), ctl,
-                                 cur, nxt, B.L_out, skip); }
+                                 cur, nxt, B.L_out, skip, B.fetch_seg); }
         if (overlap) {
             (void)hipEventRecord(L.ev_shade, st);
             (void)hipStreamWaitEvent(st2, L.ev_shade, 0);
@@ -1562,10 +1591,20 @@ static void round_end_t(const Work<BATCH>& W, Integrator kind, const Launch& L, 
                          B.L_out, B.film); }
 }
 
-void enqueue_round_begin(bool batch, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,
+// A compact round has no slots to set up, and sets its counters in its first
+// iteration when all its paths start there.
+void enqueue_round_begin(Integrator kind, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,
                          LaunchHook* hook) {
-    if (batch) round_begin_t<true>(L, P, ctl, B, hook);
-    else round_begin_t<false>(L, P, ctl, B, hook);
+    hipStream_t st = L.stream;
+    const bool compact = compact_round(kind, B);
+    if (!compact || !L.at_once) {
+        Bracket b(hook, "ctl_clear", st);
+        hipLaunchKernelGGL(k_ctl_clear, dim3(1), dim3(64), 0, st, ctl);
+    }
+    if (!compact) {
+        Bracket b(hook, "init_slots", st);
+        hipLaunchKernelGGL(k_init_slots, dim3(L.grid_shade), dim3(256), 0, st, P, ctl, B.freel[0], L.n_slots);
+    }
 }
 void enqueue_iterations(bool batch, Integrator kind, const Launch& L, const PathBuf& P, Ctl* ctl, const Buffers& B,
                         int n, bool count, LaunchHook* hook) {
