@@ -549,7 +549,7 @@ void render_frames(Ctx* c, SceneRec& sc, const bn_pt_params& p, bnd::Integrator 
         c->fwd.slots = slots;
     }
     hip_check(hipGetLastError(), "kernel launch");
-    if (film_host) hip_check(hipMemcpyAsync(film_host, c->film.p, film_n * 4, hipMemcpyDeviceToHost, s), "film D2H");
+    if (film_host) c->host_copy.download(c->film.p, {{film_host, film_n * 4}}, s);
     hip_check(hipStreamSynchronize(s), "render");
     c->timer.resolve();
     if (stats) {
@@ -873,11 +873,12 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
         ++rounds;
     }
     hip_check(hipGetLastError(), "kernel launch");
-    for (int k = 0; k < n; ++k)
-        if (films && films[k])
-            hip_check(hipMemcpyAsync(films[k], (float*)c->film.p + base[k].film_offset,
-                                     (size_t)items[k].params.width * items[k].params.height * 12,
-                                     hipMemcpyDeviceToHost, s), "film D2H");
+    if (films) {
+        std::vector<HostCopy::Part> parts(n);
+        for (int k = 0; k < n; ++k)
+            parts[k] = {films[k], (size_t)items[k].params.width * items[k].params.height * 12};
+        c->host_copy.download(c->film.p, parts, s);
+    }
     hip_check(hipStreamSynchronize(s), "batch");
     c->timer.resolve();
     if (stats) {
@@ -1113,7 +1114,7 @@ void render_pssmlt(Ctx* c, SceneRec& sc, const bn_mlt_params& p, float* film_hos
                                  hipMemcpyDeviceToHost, s), "accepts D2H");
     }
     hip_check(hipGetLastError(), "kernel launch");
-    if (film_host) hip_check(hipMemcpyAsync(film_host, c->film.p, film_n * 4, hipMemcpyDeviceToHost, s), "film D2H");
+    if (film_host) c->host_copy.download(c->film.p, {{film_host, film_n * 4}}, s);
     hip_check(hipStreamSynchronize(s), "pssmlt");
     c->timer.resolve();
     for (int32_t a : c->last_chain_accepts) accepted += a;
@@ -1472,19 +1473,16 @@ int bn_first_hit(bn_ctx* ctx, int32_t scene, const bn_pt_params* p, int32_t samp
         camera_constants(s, p->width, p->height);
         ensure_spill(c);
         const size_t n = (size_t)p->width * p->height;
-        c->out_a.ensure(n * 4);
-        c->out_b.ensure(n * 4);
-        c->out_c.ensure(n * 4);
+        c->out_hit.ensure(3 * n * 4);
+        int* out = (int*)c->out_hit.p;
         c->ctl.ensure(sizeof(bnd::Ctl));
         const bnd::Buffers B = buffers(c);
         bnd::launch_reset((bnd::Ctl*)c->ctl.p, 0, B.fetch_seg, c->stream);
-        bnd::launch_first_hit(s.dev, p->width, p->height, sample_id, p->spp, p->frame_id, (int*)c->out_a.p,
-                              (int*)c->out_b.p, (float*)c->out_c.p, (uint32_t*)c->spill.p, c->spill_stride,
+        bnd::launch_first_hit(s.dev, p->width, p->height, sample_id, p->spp, p->frame_id, out, out + n,
+                              (float*)(out + 2 * n), (uint32_t*)c->spill.p, c->spill_stride,
                               B.fetch_seg, bnd::kFetchSegs, c->stack_k, grid_trace(c), c->stream);
         hip_check(hipGetLastError(), "kernel launch");
-        hip_check(hipMemcpyAsync(inst, c->out_a.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
-        hip_check(hipMemcpyAsync(prim, c->out_b.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
-        hip_check(hipMemcpyAsync(t, c->out_c.p, n * 4, hipMemcpyDeviceToHost, c->stream), "D2H");
+        c->host_copy.download(out, {{inst, n * 4}, {prim, n * 4}, {t, n * 4}}, c->stream);
         hip_check(hipStreamSynchronize(c->stream), "first hit");
     });
 }

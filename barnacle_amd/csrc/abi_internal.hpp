@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/barnacle_hip.h"
+#include "host_copy.hpp"
 #include "host_scene.hpp"
 #include "kernels.hpp"
 #include "kernels_mlt.hpp"
@@ -103,7 +104,8 @@ struct Ctx {
     // (what bn_backward_pt replays against), when valid.
     struct { bool valid; const SceneRec* scene; uint64_t gen; bn_pt_params p; size_t slots; } fwd{};
     size_t spill_stride = 0;
-    DevBuf out_a, out_b, out_c;
+    DevBuf out_hit;                       // instance, primitive and t of bn_first_hit
+    HostCopy host_copy;                   // results into the caller's arrays
     KernelTimer timer;
     // batched rounds
     bool use_graph = true;
