@@ -30,6 +30,7 @@
 
 #include "abi_internal.hpp"
 #include "bvh_gpu.hpp"
+#include "wave.hpp"
 
 namespace bvhg {
 
@@ -113,16 +114,6 @@ __device__ __forceinline__ int wave_sum(int x) {
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) x += __shfl_xor(x, s);
     return x;
-}
-__device__ __forceinline__ int wave_excl_scan(int x) {
-    const int lane = threadIdx.x & 63;
-    int v = x;
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) {
-        const int y = __shfl_up(v, s);
-        if (lane >= s) v += y;
-    }
-    return v - x;
 }
 // Ordered union over a block (waves in order); every thread gets the result.
 __device__ DBox block_union(DBox v, DBox* sh) {
@@ -437,143 +428,216 @@ __device__ __forceinline__ bn_bvh_node make_node(const DBox& b, int32_t word, bo
 
 // One wave builds the whole subtree of a small task (Tree.Build, recursive,
 // left first) into the task's node region, numbered in pre-order from 0.
-// A task has at most 64 * kPer items, so each lane holds its run of at most
-// kPer consecutive items in registers while a node is processed.
-constexpr int kPer = 8;
+//
+// The task's items live in LDS; a lane holds its run of at most kPer
+// consecutive ones in registers while they are moved.  A box is kept as six
+// maxima (-lo, hi): the negation is exact and a min whose second operand wins
+// ties is the negated max whose second operand wins them.  Most nodes hold a
+// few items, so a node's cost has to follow its item count: the bins are
+// folded by 48 lanes, one per bin, side and half of the items, each walking
+// the items in order (24 x 7 values through six lane-reduction steps took the
+// same time for every node: the kernel ran 2.6 ms for 240,000 items, 0.50 ms
+// like this), and the SAH sweep runs in 22 lanes, one per prefix and suffix.
+constexpr int kPer = 4;
 constexpr int kSmallMax = 64 * kPer;
+constexpr int kRow = kSmallMax + 4;               // the two sides' rows start in different banks
+struct Box6 { float v[6]; };                      // -lo xyz, hi xyz
+struct SmallLds {
+    float f[6][kRow];
+    int id[kSmallMax];
+    uint8_t bin[kSmallMax];
+    float bin_box[kBins][6];
+    int bin_n[kBins];
+    int4 frames[kMaxDepth + 2];                   // first, last (in the task), depth, parent
+};
+__device__ __forceinline__ float later_max(float a, float b) { return a > b ? a : b; }
+__device__ __forceinline__ Box6 empty6() { return {{-kInf, -kInf, -kInf, -kInf, -kInf, -kInf}}; }
+__device__ __forceinline__ void join6(Box6& a, const Box6& b) {
+#pragma unroll
+    for (int c = 0; c < 6; ++c) a.v[c] = later_max(a.v[c], b.v[c]);
+}
+__device__ __forceinline__ DBox dbox(const Box6& b) { return {{-b.v[0], -b.v[1], -b.v[2]}, {b.v[3], b.v[4], b.v[5]}}; }
+// Ordered union over the first `lanes` lanes, in lane 0; broadcast.
+__device__ __forceinline__ void wave_union6(Box6& b, int lanes) {
+    for (int s = 1; s < lanes; s <<= 1) {
+        Box6 o;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) o.v[c] = __shfl_down(b.v[c], s);
+        join6(b, o);                              // meaningful in lanes that are multiples of 2s
+    }
+#pragma unroll
+    for (int c = 0; c < 6; ++c) b.v[c] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(b.v[c])));
+}
+__device__ __forceinline__ int sreg(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// The best split of the binned items [0, cnt) of a node (Util/BVH.fs:183-203)
+// and the number of items left of it.
+__device__ __forceinline__ void small_split(SmallLds& S, int first, int cnt, float cb_area, int& best, int& n_left) {
+    const int lane = threadIdx.x & 63;
+    const int half = lane >= 24 ? 1 : 0, j = lane - 24 * half;
+    const int k = j >> 1, side = j & 1;
+    const int mid = (cnt + 1) >> 1;
+    float x = -kInf, y = -kInf, z = -kInf;
+    int n = 0;
+    if (lane < 48) {
+        const float* fx = S.f[3 * side];
+        const int e = first + (half ? cnt : mid);
+        for (int i = first + (half ? mid : 0); i < e; ++i) {
+            const bool in = S.bin[i] == k;
+            const float a = fx[i], b = fx[kRow + i], c = fx[2 * kRow + i];
+            x = in ? later_max(x, a) : x;
+            y = in ? later_max(y, b) : y;
+            z = in ? later_max(z, c) : z;
+            n += in ? 1 : 0;
+        }
+    }
+    const float ox = __shfl(x, lane + 24), oy = __shfl(y, lane + 24), oz = __shfl(z, lane + 24);
+    const int on = __shfl(n, lane + 24);
+    if (lane < 24) {
+        float* o = &S.bin_box[k][3 * side];
+        o[0] = later_max(x, ox);
+        o[1] = later_max(y, oy);
+        o[2] = later_max(z, oz);
+        S.bin_n[k] = n + on;
+    }
+    bnd::wave_sync();
+    // lane s < 11: bins [0, s] in ascending order; lane 16 + s: bins [s + 1, 12) in descending order
+    const bool right = (lane & 16) != 0;
+    const int s = lane & 15;
+    Box6 acc = empty6();
+    int c = 0;
+    for (int t = 0; t < kBins - 1; ++t) {
+        const int q = right ? kBins - 1 - t : t;
+        if (right ? t <= kBins - 2 - s : t <= s) {
+#pragma unroll
+            for (int w = 0; w < 6; ++w) acc.v[w] = later_max(acc.v[w], S.bin_box[q][w]);
+            c += S.bin_n[q];
+        }
+    }
+    const float cost1 = (float)c * area(dbox(acc));
+    const float cost = (cost1 + __shfl(cost1, lane + 16)) + (float)cnt * cb_area;
+    const bool valid = lane < kBins - 1 && cost < kInf;
+    float m = valid ? cost : kInf;
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) m = fminf(m, __shfl_xor(m, o));
+    const uint64_t at = __ballot(valid && cost == m);
+    best = at ? __ffsll((unsigned long long)at) - 1 : 0;
+    n_left = __builtin_amdgcn_readlane(c, best);
+}
+
 __global__ void __launch_bounds__(kThreads) k_small(Bufs B, int n_small) {
-    struct Frame { int first, last, depth, parent, buf; };
-    __shared__ Frame stack[kWavesPerBlock][kMaxDepth + 2];
+    __shared__ SmallLds lds[kWavesPerBlock];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ti = blockIdx.x * kWavesPerBlock + w;
+    const int ti = sreg(blockIdx.x * kWavesPerBlock + w);
     if (ti >= n_small) return;
+    SmallLds& S = lds[w];
     const SmallTask task = B.small[ti];
     const int off = B.set_off[task.set];
     bn_bvh_node* region = B.region + 2 * (size_t)task.first;
-    Frame* st = stack[w];
-    int sp = 0, nodes = 0;
-    st[sp++] = {task.first, task.last, task.depth, -1, task.buf};
+    const int total = task.last - task.first;
+    for (int i = lane; i < total; i += 64) {
+        const Item it = load_item(B.items[task.buf] + task.first + i);
+        S.f[0][i] = -it.lx; S.f[1][i] = -it.ly; S.f[2][i] = -it.lz;
+        S.f[3][i] = it.hx; S.f[4][i] = it.hy; S.f[5][i] = it.hz;
+        S.id[i] = it.id;
+    }
+    if (lane == 0) S.frames[0] = make_int4(0, total, task.depth, -1);
+    bnd::wave_sync();
+    int sp = 1, nodes = 0;
     while (sp > 0) {
-        const Frame f = st[--sp];
+        const int4 f = S.frames[--sp];
+        const int first = sreg(f.x), last = sreg(f.y), depth = sreg(f.z), parent = sreg(f.w);
         const int me = nodes++;
-        if (f.parent >= 0 && lane == 0) region[f.parent].right_or_offset = me;
-        const int cnt = f.last - f.first;
-        const int per = (cnt + 63) / 64;                  // at most kPer
-        const int b = min(f.first + lane * per, f.last), n = min(b + per, f.last) - b;
-        const Item* in = B.items[f.buf];
-        Item its[kPer];
-        DBox bb = empty_box(), cb = empty_box();
+        if (parent >= 0 && lane == 0) region[parent].right_or_offset = me;
+        const int cnt = last - first;
+        const int per = (cnt + 63) >> 6;                  // at most kPer
+        const int lanes = (cnt + per - 1) / per;          // lanes with items
+        const int b = min(first + lane * per, last), n = min(b + per, last) - b;
+        Box6 its[kPer], bb = empty6(), cb = empty6();
+        int ids[kPer];
 #pragma unroll
-        for (int j = 0; j < kPer; ++j)
+        for (int j = 0; j < kPer; ++j) {
+            if (j >= per) break;
             if (j < n) {
-                its[j] = load_item(in + b + j);
-                bb = join(bb, item_box(its[j]));
-                cb = join(cb, centroid_box(its[j]));
+#pragma unroll
+                for (int c = 0; c < 6; ++c) its[j].v[c] = S.f[c][b + j];
+                ids[j] = S.id[b + j];
+                join6(bb, its[j]);
+                Box6 ce;                                  // the centroid 0.5 * (lo + hi), as a point
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const float m = 0.5f * (-its[j].v[c] + its[j].v[3 + c]);
+                    ce.v[c] = -m;
+                    ce.v[3 + c] = m;
+                }
+                join6(cb, ce);
             }
-        bb = wave_union(bb);
-        if (cnt <= kLeaf || f.depth >= kMaxDepth) {
+        }
+        wave_union6(bb, lanes);
+        if (cnt <= kLeaf || depth >= kMaxDepth) {
             if (cnt > 127) {
                 if (lane == 0) atomicOr(&B.ctl->err, 1);
             } else if (lane == 0) {
-                region[me] = make_node(bb, f.first - off, true, 0, cnt);
+                region[me] = make_node(dbox(bb), task.first + first - off, true, 0, cnt);
             }
 #pragma unroll
             for (int j = 0; j < kPer; ++j)
-                if (j < n) B.perm[b + j] = its[j].id;
+                if (j < n) B.perm[task.first + b + j] = ids[j];
             continue;
         }
-        cb = wave_union(cb);
-        const int axis = split_axis(cb);
-        const float extent = cb.h[axis] - cb.l[axis];
-        if (lane == 0) region[me] = make_node(bb, 0, false, axis, 0);
-        int mid;
-        int child_buf = f.buf;
+        wave_union6(cb, lanes);
+        const DBox cbox = dbox(cb);
+        const int axis = sreg(split_axis(cbox));
+        const float lo = axis == 0 ? cbox.l[0] : axis == 1 ? cbox.l[1] : cbox.l[2];
+        const float extent = (axis == 0 ? cbox.h[0] : axis == 1 ? cbox.h[1] : cbox.h[2]) - lo;
+        if (lane == 0) region[me] = make_node(dbox(bb), 0, false, axis, 0);
+        int n_left;
         if (extent == 0.0f) {
-            mid = f.first + cnt / 2;                       // items stay where they are
+            n_left = cnt / 2;                              // items stay where they are
         } else {
-            const float lo = cb.l[axis];
             int bin[kPer];
 #pragma unroll
-            for (int j = 0; j < kPer; ++j) bin[j] = j < n ? bin_of(its[j], axis, lo, extent) : -1;
-            DBox bbin[kBins];
-            int bn[kBins];
-#pragma unroll
-            for (int k = 0; k < kBins; ++k) {
-                bbin[k] = empty_box();
-                bn[k] = 0;
-#pragma unroll
-                for (int j = 0; j < kPer; ++j)
-                    if (bin[j] == k) { bbin[k] = join(bbin[k], item_box(its[j])); ++bn[k]; }
-            }
-            // the twelve ordered lane reductions, interleaved step by step
-#pragma unroll
-            for (int s = 1; s < 64; s <<= 1) {
-#pragma unroll
-                for (int k = 0; k < kBins; ++k) {
-                    DBox o;
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) {
-                        o.l[q] = __shfl_down(bbin[k].l[q], s);
-                        o.h[q] = __shfl_down(bbin[k].h[q], s);
-                    }
-                    bbin[k] = join(bbin[k], o);
-                    bn[k] += __shfl_down(bn[k], s);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < kBins; ++k) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    bbin[k].l[q] = __shfl(bbin[k].l[q], 0);
-                    bbin[k].h[q] = __shfl(bbin[k].h[q], 0);
-                }
-                bn[k] = __shfl(bn[k], 0);
-            }
-            float lcost[kBins - 1], rcost[kBins - 1];
-            DBox acc = empty_box();
-            int c = 0;
-#pragma unroll
-            for (int s = 0; s < kBins - 1; ++s) {
-                acc = join(acc, bbin[s]);
-                c += bn[s];
-                lcost[s] = (float)c * area(acc);
-            }
-            acc = empty_box();
-            c = 0;
-#pragma unroll
-            for (int s = kBins - 2; s >= 0; --s) {
-                acc = join(acc, bbin[s + 1]);
-                c += bn[s + 1];
-                rcost[s] = (float)c * area(acc);
-            }
-            const float base = (float)cnt * area(cb);
-            float best_cost = kInf;
-            int best = 0;
-#pragma unroll
-            for (int s = 0; s < kBins - 1; ++s) {
-                const float cost = (lcost[s] + rcost[s]) + base;
-                if (cost < best_cost) { best_cost = cost; best = s; }
-            }
-            // partition into the other buffer: lefts from first, rights from last - 1 down
-            int nl = 0;
-#pragma unroll
-            for (int j = 0; j < kPer; ++j) nl += (j < n && bin[j] <= best) ? 1 : 0;
-            const int nr = n - nl;
-            const int tl = wave_sum(nl);
-            int l = f.first + wave_excl_scan(nl), r = f.last - 1 - wave_excl_scan(nr);
-            Item* out = B.items[f.buf ^ 1];
-#pragma unroll
-            for (int j = 0; j < kPer; ++j)
+            for (int j = 0; j < kPer; ++j) {
+                bin[j] = -1;
+                if (j >= per) break;
                 if (j < n) {
-                    if (bin[j] <= best) store_item(out + l++, its[j]);
-                    else store_item(out + r--, its[j]);
+                    const Box6& q = its[j];
+                    const float l = axis == 0 ? q.v[0] : axis == 1 ? q.v[1] : q.v[2];
+                    const float h = axis == 0 ? q.v[3] : axis == 1 ? q.v[4] : q.v[5];
+                    const float v = (12.0f * (0.5f * (-l + h) - lo)) / extent;
+                    bin[j] = min(kBins - 1, (int)v);       // findBinIndex, as bin_of
+                    S.bin[b + j] = (uint8_t)bin[j];
                 }
-            __threadfence_block();                 // the children read what other lanes wrote
-            mid = f.first + tl;
-            child_buf = f.buf ^ 1;
+            }
+            bnd::wave_sync();
+            int best;
+            small_split(S, first, cnt, area(cbox), best, n_left);
+            // partition: lefts in order from first, rights in order from last - 1 down
+            int before = 0;                                // lefts before this lane's items
+#pragma unroll
+            for (int j = 0; j < kPer; ++j) {
+                if (j >= per) break;
+                before += (int)bnd::mbcnt(__ballot(j < n && bin[j] <= best));
+            }
+            int l = first + before, r = last - 1 - (b - first - before);
+#pragma unroll
+            for (int j = 0; j < kPer; ++j) {
+                if (j >= per) break;
+                if (j < n) {
+                    const int to = bin[j] <= best ? l++ : r--;
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) S.f[c][to] = its[j].v[c];
+                    S.id[to] = ids[j];
+                }
+            }
         }
-        st[sp++] = {mid, f.last, f.depth + 1, me, child_buf};
-        st[sp++] = {f.first, mid, f.depth + 1, -1, child_buf};
+        const int mid = first + n_left;
+        if (lane == 0) {
+            S.frames[sp] = make_int4(mid, last, depth + 1, me);
+            S.frames[sp + 1] = make_int4(first, mid, depth + 1, -1);
+        }
+        sp += 2;
+        bnd::wave_sync();
     }
     if (lane == 0) B.small_size[ti] = nodes;
 }
