@@ -1200,13 +1200,10 @@ int bn_bvh_build_gpu(bn_ctx* ctx, const float* b, int32_t n, bn_bvh_node* out_no
         Ctx* c = reinterpret_cast<Ctx*>(ctx);
         if (!c || n <= 0 || !b || !out_nodes || !out_n_nodes || !out_perm) throw Error(BN_E_INVALID, "bad arguments");
         hip_check(hipSetDevice(c->device), "hipSetDevice");
-        std::vector<std::vector<bn_bvh_node>> nodes;
-        std::vector<std::vector<int32_t>> perm;
-        bvh_build_gpu(c, {b}, {n}, nodes, perm);
-        if ((int)nodes[0].size() > *out_n_nodes) throw Error(BN_E_CAPACITY, "node buffer too small");
-        std::memcpy(out_nodes, nodes[0].data(), nodes[0].size() * sizeof(bn_bvh_node));
-        *out_n_nodes = (int)nodes[0].size();
-        std::memcpy(out_perm, perm[0].data(), perm[0].size() * 4);
+        const GpuBvh g = bvh_build_gpu(c, {b}, {n});
+        if (g.n_nodes[0] > *out_n_nodes) throw Error(BN_E_CAPACITY, "node buffer too small");
+        bvh_fetch(c, g, {out_nodes}, {out_perm});
+        *out_n_nodes = g.n_nodes[0];
     });
 }
 
@@ -1289,7 +1286,18 @@ int bn_scene_build(bn_ctx* ctx, const bn_scene_desc* desc, int32_t* out_scene) {
         const bnh::BatchBvhBuild gpu_build = [c](const std::vector<const float*>& sets, const std::vector<int>& counts,
                                                  std::vector<std::vector<bn_bvh_node>>& nodes,
                                                  std::vector<std::vector<int32_t>>& perms) {
-            bvh_build_gpu(c, sets, counts, nodes, perms);
+            const GpuBvh g = bvh_build_gpu(c, sets, counts);
+            nodes.resize(sets.size());
+            perms.resize(sets.size());
+            std::vector<bn_bvh_node*> dn;
+            std::vector<int32_t*> dp;
+            for (size_t k = 0; k < sets.size(); ++k) {
+                nodes[k].resize(g.n_nodes[k]);
+                perms[k].resize(counts[k]);
+                dn.push_back(nodes[k].data());
+                dp.push_back(perms[k].data());
+            }
+            bvh_fetch(c, g, dn, dp);
         };
         bnh::build_scene(*desc, *hs, c->bvh_gpu ? &gpu_build : nullptr);
         std::vector<int> blas_of(hs->meshes.size(), -1);

@@ -15,12 +15,16 @@
 //  * The SAH sweep of a node runs in one thread in the reference's order.
 //
 // Schedule: a task is a node's item range.  Tasks of more than `small` items
-// run level by level over chunks of kChunk items (one block per chunk):
-// bounds, bins and the scatter are chunk kernels, the per-node decisions one
-// thread per task.  A task of at most `small` items (or at depth 64) is built
-// whole by one wave, recursively with an LDS stack, into a node region of its
-// own.  The host numbers the upper nodes and regions in pre-order, and a
-// last pass writes the flattened nodes.
+// run level by level over chunks of kChunk items: bounds, bins and the scatter
+// by one block per chunk, the decisions (split axis; split and children) by one
+// wave or block per task.  Task and chunk counts stay on the device: the levels
+// are launched for the most they can have, several levels at a time.  A task of
+// at most `small` items (or at depth 64) is built whole by one wave into a node
+// region of its own.  One block numbers the upper nodes and regions in
+// pre-order, and a last pass writes the flattened nodes.  A level takes 55 us
+// for 240,000 items; with decisions by one thread per task, a copy of the
+// counters and a host synchronisation it took 120, and with the decisions in
+// the block that finishes a task's last chunk 90 (the fences).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,7 +39,7 @@
 namespace bvhg {
 
 constexpr int kBins = 12, kLeaf = 4, kMaxDepth = 64;        // BVHBuildConfig (Util/BVH.fs:99-107)
-constexpr int kThreads = 256, kIpt = 8;
+constexpr int kThreads = 256, kIpt = 4;
 constexpr int kChunk = kThreads * kIpt;                     // items per chunk block
 constexpr int kWavesPerBlock = kThreads / 64;
 constexpr float kInf = __builtin_huge_valf();
@@ -44,10 +48,16 @@ constexpr float kInf = __builtin_huge_valf();
 struct alignas(16) Item { float lx, ly, lz; int32_t id; float hx, hy, hz; int32_t pad; };
 struct DBox { float l[3], h[3]; };
 struct BigTask { int first, last, depth, unode, set, chunk0, nchunks, pad; };
-struct BigInfo { int mode, axis, best, nl; float lo_axis, extent, pad0, pad1; DBox cb; };   // mode 0 bin, 1 middle
+struct BigInfo { int mode, axis, best, pad; float lo_axis, extent, cb_area, pad1; };   // mode 0 bin, 1 middle
 struct SmallTask { int first, last, depth, buf, set, pad0, pad1, pad2; };
 struct UNode { DBox b; int axis, left, right, set; };      // child < 0: small task ~child
-struct Ctl { int n_next_big, n_small, n_unodes, n_chunks, err, pad[3]; };
+constexpr int kLevels = kMaxDepth + 1;
+struct Ctl {
+    int n_small, n_unodes, err, pad;
+    int n_big[kLevels], n_chunks[kLevels];                 // tasks and chunks of each level
+    int unode_end[kLevels];                                // end of the level's upper nodes (numbered level by level)
+};
+constexpr int kErrLeaf = 1, kErrCapacity = 2, kErrFinite = 4, kErrCount = 8;
 
 __device__ __forceinline__ float omin(float a, float b) { return a < b ? a : b; }
 __device__ __forceinline__ float omax(float a, float b) { return a > b ? a : b; }
@@ -110,11 +120,6 @@ __device__ DBox wave_union(DBox v) {
     for (int k = 0; k < 3; ++k) { v.l[k] = __shfl(v.l[k], 0); v.h[k] = __shfl(v.h[k], 0); }
     return v;
 }
-__device__ __forceinline__ int wave_sum(int x) {
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) x += __shfl_xor(x, s);
-    return x;
-}
 // Ordered union over a block (waves in order); every thread gets the result.
 __device__ DBox block_union(DBox v, DBox* sh) {
     v = wave_union(v);
@@ -123,16 +128,6 @@ __device__ DBox block_union(DBox v, DBox* sh) {
     __syncthreads();
     DBox r = sh[0];
     for (int k = 1; k < kWavesPerBlock; ++k) r = join(r, sh[k]);
-    __syncthreads();
-    return r;
-}
-__device__ int block_sum(int x, int* sh) {
-    x = wave_sum(x);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) sh[w] = x;
-    __syncthreads();
-    int r = 0;
-    for (int k = 0; k < kWavesPerBlock; ++k) r += sh[k];
     __syncthreads();
     return r;
 }
@@ -152,30 +147,64 @@ __device__ int block_excl_scan(int x, int* sh) {
     return off + v - x;
 }
 
+// A box as six maxima (-lo, hi): the negation is exact, and a min whose second
+// operand wins ties is the negated max whose second operand wins them.
+struct Box6 { float v[6]; };
+__device__ __forceinline__ float later_max(float a, float b) { return a > b ? a : b; }
+__device__ __forceinline__ Box6 empty6() { return {{-kInf, -kInf, -kInf, -kInf, -kInf, -kInf}}; }
+__device__ __forceinline__ void join6(Box6& a, const Box6& b) {
+#pragma unroll
+    for (int c = 0; c < 6; ++c) a.v[c] = later_max(a.v[c], b.v[c]);
+}
+__device__ __forceinline__ DBox dbox(const Box6& b) { return {{-b.v[0], -b.v[1], -b.v[2]}, {b.v[3], b.v[4], b.v[5]}}; }
+
 struct Bufs {
     Item* items[2];
-    const BigTask* big;
+    BigTask* big[2];         // by level parity
     BigInfo* info;
-    BigTask* next_big;
     SmallTask* small;
-    const int* chunk_task;
-    const int* chunk_start;
-    int* chunk_task_next;
-    int* chunk_start_next;
-    DBox* part_b;       // per chunk: item bounds
-    DBox* part_cb;      // per chunk: centroid bounds
-    DBox* bin_b;        // per chunk x bin
+    int* chunk_task[2];      // by level parity
+    int* chunk_start[2];
+    DBox* part_b;            // per chunk: item bounds
+    DBox* part_cb;           // per chunk: centroid bounds
+    Box6* bin_b;             // per chunk x bin
     int* bin_n;
     int* chunk_lbase;
     int* chunk_rbase;
     UNode* unodes;
-    bn_bvh_node* region; // 2 * first: the region of the small task starting at `first`
-    int* small_size;     // nodes of each small task's region
-    int32_t* perm;       // per position: item id
-    const int* set_off;
+    int *udfs, *uright, *usize;   // per upper node: index, right child, subtree nodes
+    bn_bvh_node* region;     // 2 * first: the region of the small task starting at `first`
+    int* small_size;         // nodes of each small task's region
+    int* small_base;         // the region's first node in its set
+    int32_t* perm;           // per position: item id
+    const int* set_off;      // first item of each set, and the end
+    const int* root;         // root code of each set: an upper node, or ~(small task)
+    int* set_nodes;          // nodes of each set
+    int* set_base;           // first node of each set in the output
     Ctl* ctl;
-    int big_cap, small_cap, unode_cap, chunk_cap;
+    int n_sets, n_items, small_max, big_cap, small_cap, unode_cap, chunk_cap;
 };
+
+// The items of all sets from their bounds; their ids count within the set.
+__global__ void __launch_bounds__(kThreads) k_items(Bufs B, const float* bounds) {
+    bool finite = true;
+    for (int i = blockIdx.x * kThreads + threadIdx.x; i < B.n_items; i += gridDim.x * kThreads) {
+        const float2* p = reinterpret_cast<const float2*>(bounds) + 3 * (size_t)i;
+        const float2 a = p[0], b = p[1], c = p[2];
+        int lo = 0, hi = B.n_sets - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (B.set_off[mid] <= i) lo = mid; else hi = mid - 1;
+        }
+        Item it;
+        it.lx = a.x; it.ly = a.y; it.lz = b.x; it.id = i - B.set_off[lo];
+        it.hx = b.y; it.hy = c.x; it.hz = c.y; it.pad = 0;
+        finite = finite && isfinite(a.x) && isfinite(a.y) && isfinite(b.x) && isfinite(b.y) && isfinite(c.x) &&
+                 isfinite(c.y);
+        store_item(B.items[0] + i, it);
+    }
+    if (__ballot(!finite) != 0 && (threadIdx.x & 63) == 0) atomicOr(&B.ctl->err, kErrFinite);
+}
 
 // The thread's items of a chunk: [s + t * kIpt, ...) within [s, e).
 __device__ __forceinline__ void thread_range(int s, int e, int& b, int& en) {
@@ -183,17 +212,53 @@ __device__ __forceinline__ void thread_range(int s, int e, int& b, int& en) {
     en = min(b + kIpt, e);
 }
 
-// K1: item bounds and centroid bounds of every chunk.
-__global__ void __launch_bounds__(kThreads) k_chunk_bounds(Bufs B, int src) {
+// Bounds and counts of a node's twelve bins, for the sweep.
+struct SplitLds {
+    float bin_box[kBins][6];
+    int bin_n[kBins];
+};
+// SAH sweep of a node of cnt items (Util/BVH.fs:183-203) by one wave, prefixes
+// and suffixes of the bins side by side, each folded in the reference's order:
+// the best split and the number of items left of it.
+__device__ __forceinline__ void sah_sweep(const SplitLds& S, int cnt, float cb_area, int& best, int& n_left) {
+    const int lane = threadIdx.x & 63;
+    // lane s < 11: bins [0, s] in ascending order; lane 16 + s: bins [s + 1, 12) in descending order
+    const bool right = (lane & 16) != 0;
+    const int s = lane & 15;
+    Box6 acc = empty6();
+    int c = 0;
+    for (int t = 0; t < kBins - 1; ++t) {
+        const int q = right ? kBins - 1 - t : t;
+        if (right ? t <= kBins - 2 - s : t <= s) {
+#pragma unroll
+            for (int w = 0; w < 6; ++w) acc.v[w] = later_max(acc.v[w], S.bin_box[q][w]);
+            c += S.bin_n[q];
+        }
+    }
+    const float cost1 = (float)c * area(dbox(acc));
+    const float cost = (cost1 + __shfl(cost1, lane + 16)) + (float)cnt * cb_area;
+    const bool valid = lane < kBins - 1 && cost < kInf;
+    float m = valid ? cost : kInf;
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) m = fminf(m, __shfl_xor(m, o));
+    const uint64_t at = __ballot(valid && cost == m);
+    best = at ? __ffsll((unsigned long long)at) - 1 : 0;
+    n_left = __builtin_amdgcn_readlane(c, best);
+}
+
+// Per chunk: item bounds and centroid bounds.
+__global__ void __launch_bounds__(kThreads) k_chunk_bounds(Bufs B, int level) {
     __shared__ DBox sh[kWavesPerBlock];
-    const int c = blockIdx.x;
-    const BigTask t = B.big[B.chunk_task[c]];
-    const int s = B.chunk_start[c], e = min(s + kChunk, t.last);
+    const int c = blockIdx.x, cur = level & 1;
+    if (c == 0 && threadIdx.x == 0) B.ctl->unode_end[level] = B.ctl->n_unodes;
+    if (c >= B.ctl->n_chunks[level] || (B.ctl->err & kErrFinite)) return;
+    const BigTask t = B.big[cur][B.chunk_task[cur][c]];
+    const int s = B.chunk_start[cur][c], e = min(s + kChunk, t.last);
     int b, en;
     thread_range(s, e, b, en);
     DBox bb = empty_box(), cb = empty_box();
     for (int i = b; i < en; ++i) {
-        const Item it = load_item(B.items[src] + i);
+        const Item it = load_item(B.items[cur] + i);
         bb = join(bb, item_box(it));
         cb = join(cb, centroid_box(it));
     }
@@ -202,13 +267,18 @@ __global__ void __launch_bounds__(kThreads) k_chunk_bounds(Bufs B, int src) {
     if (threadIdx.x == 0) { B.part_b[c] = bb; B.part_cb[c] = cb; }
 }
 
-// K2: per task: node bounds, centroid bounds, split axis and mode.
-__global__ void k_task_bounds(Bufs B, int n_big) {
-    const int ti = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ti >= n_big) return;
-    const BigTask t = B.big[ti];
+// Per task (one wave): node bounds, split axis and mode.
+__global__ void __launch_bounds__(64) k_task_bounds(Bufs B, int level) {
+    const int ti = blockIdx.x, cur = level & 1;
+    if (ti >= B.ctl->n_big[level] || (B.ctl->err & kErrFinite)) return;
+    const BigTask t = B.big[cur][ti];
+    const int run = (t.nchunks + 63) / 64;                          // chunks in order, a run per lane
+    const int q0 = min((int)threadIdx.x * run, t.nchunks), q1 = min(q0 + run, t.nchunks);
     DBox bb = empty_box(), cb = empty_box();
-    for (int c = t.chunk0; c < t.chunk0 + t.nchunks; ++c) { bb = join(bb, B.part_b[c]); cb = join(cb, B.part_cb[c]); }
+    for (int q = t.chunk0 + q0; q < t.chunk0 + q1; ++q) { bb = join(bb, B.part_b[q]); cb = join(cb, B.part_cb[q]); }
+    bb = wave_union(bb);
+    cb = wave_union(cb);
+    if (threadIdx.x != 0) return;
     const int axis = split_axis(cb);
     const float extent = cb.h[axis] - cb.l[axis];
     BigInfo inf{};
@@ -216,7 +286,7 @@ __global__ void k_task_bounds(Bufs B, int n_big) {
     inf.axis = axis;
     inf.lo_axis = cb.l[axis];
     inf.extent = extent;
-    inf.cb = cb;
+    inf.cb_area = area(cb);
     B.info[ti] = inf;
     UNode& u = B.unodes[t.unode];
     u.b = bb;
@@ -224,133 +294,193 @@ __global__ void k_task_bounds(Bufs B, int n_big) {
     u.set = t.set;
 }
 
-// K3: per chunk of a binned task: each bin's bounds (ordered) and count.
-__global__ void __launch_bounds__(kThreads) k_chunk_bins(Bufs B, int src) {
-    __shared__ DBox sh[kWavesPerBlock];
-    __shared__ int shn[kWavesPerBlock];
-    const int c = blockIdx.x;
-    const int ti = B.chunk_task[c];
+// Per chunk of a binned task: each bin's bounds (ordered) and count, by a
+// thread per bin, side and run of items, then the runs in order.
+constexpr int kRuns = kThreads / (2 * kBins);
+__global__ void __launch_bounds__(kThreads) k_chunk_bins(Bufs B, int level) {
+    __shared__ float f[6][kChunk + 4];
+    __shared__ uint8_t bin[kChunk];
+    __shared__ float run_box[kRuns][kBins][6];
+    __shared__ int run_n[kRuns][kBins];
+    const int c = blockIdx.x, cur = level & 1;
+    if (c >= B.ctl->n_chunks[level] || (B.ctl->err & kErrFinite)) return;
+    const int ti = B.chunk_task[cur][c];
     const BigInfo inf = B.info[ti];
     if (inf.mode != 0) return;                    // uniform per block
-    const BigTask t = B.big[ti];
-    const int s = B.chunk_start[c], e = min(s + kChunk, t.last);
-    int b, en;
-    thread_range(s, e, b, en);
-    Item its[kIpt];
-    int bins[kIpt];
-#pragma unroll
-    for (int j = 0; j < kIpt; ++j) {
-        if (b + j < en) {
-            its[j] = load_item(B.items[src] + b + j);
-            bins[j] = bin_of(its[j], inf.axis, inf.lo_axis, inf.extent);
-        } else {
-            bins[j] = -1;
-        }
+    const int s = B.chunk_start[cur][c], n = min(s + kChunk, B.big[cur][ti].last) - s;
+    for (int i = threadIdx.x; i < n; i += kThreads) {
+        const Item it = load_item(B.items[cur] + s + i);
+        f[0][i] = -it.lx; f[1][i] = -it.ly; f[2][i] = -it.lz;
+        f[3][i] = it.hx; f[4][i] = it.hy; f[5][i] = it.hz;
+        bin[i] = (uint8_t)bin_of(it, inf.axis, inf.lo_axis, inf.extent);
     }
-    for (int k = 0; k < kBins; ++k) {
-        DBox bb = empty_box();
-        int n = 0;
-#pragma unroll
-        for (int j = 0; j < kIpt; ++j)
-            if (bins[j] == k) { bb = join(bb, item_box(its[j])); ++n; }
-        bb = block_union(bb, sh);
-        n = block_sum(n, shn);
-        if (threadIdx.x == 0) { B.bin_b[(size_t)c * kBins + k] = bb; B.bin_n[(size_t)c * kBins + k] = n; }
+    __syncthreads();
+    const int r = (int)threadIdx.x / (2 * kBins), j = (int)threadIdx.x % (2 * kBins);
+    if (r < kRuns) {
+        const int k = j >> 1, side = j & 1, len = (n + kRuns - 1) / kRuns;
+        const int e = min((r + 1) * len, n);
+        float x = -kInf, y = -kInf, z = -kInf;
+        int m = 0;
+        for (int i = min(r * len, n); i < e; ++i) {
+            const bool in = bin[i] == k;
+            const float a = f[3 * side][i], b = f[3 * side + 1][i], d = f[3 * side + 2][i];
+            x = in ? later_max(x, a) : x;
+            y = in ? later_max(y, b) : y;
+            z = in ? later_max(z, d) : z;
+            m += in ? 1 : 0;
+        }
+        float* o = &run_box[r][k][3 * side];
+        o[0] = x; o[1] = y; o[2] = z;
+        if (side == 0) run_n[r][k] = m;
+    }
+    __syncthreads();
+    if (threadIdx.x < kBins * 6) {
+        const int k = (int)threadIdx.x / 6, w = (int)threadIdx.x % 6;
+        float v = -kInf;
+        for (int q = 0; q < kRuns; ++q) v = later_max(v, run_box[q][k][w]);
+        B.bin_b[(size_t)c * kBins + k].v[w] = v;
+    } else if (threadIdx.x >= 128 && threadIdx.x < 128 + kBins) {
+        int m = 0;
+        for (int q = 0; q < kRuns; ++q) m += run_n[q][threadIdx.x - 128];
+        B.bin_n[(size_t)c * kBins + (threadIdx.x - 128)] = m;
     }
 }
 
-// K4: per task: SAH sweep (Util/BVH.fs:183-203), chunk scatter bases and the
-// two children, each either a task of the next level or a small task.
-__global__ void k_task_split(Bufs B, int n_big, int level, int small) {
-    const int ti = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ti >= n_big) return;
-    const BigTask t = B.big[ti];
-    BigInfo inf = B.info[ti];
-    const int cnt = t.last - t.first;
-    int nl;
-    if (inf.mode == 0) {
-        DBox bb[kBins];
-        int bn[kBins];
-        for (int k = 0; k < kBins; ++k) { bb[k] = empty_box(); bn[k] = 0; }
-        for (int c = t.chunk0; c < t.chunk0 + t.nchunks; ++c)
-            for (int k = 0; k < kBins; ++k) {
-                bb[k] = join(bb[k], B.bin_b[(size_t)c * kBins + k]);
-                bn[k] += B.bin_n[(size_t)c * kBins + k];
-            }
-        float lcost[kBins - 1], rcost[kBins - 1];
-        DBox acc = empty_box();
-        int n = 0;
-        for (int s = 0; s < kBins - 1; ++s) {
-            acc = join(acc, bb[s]);
-            n += bn[s];
-            lcost[s] = (float)n * area(acc);
-        }
-        acc = empty_box();
-        n = 0;
-        for (int s = kBins - 2; s >= 0; --s) {
-            acc = join(acc, bb[s + 1]);
-            n += bn[s + 1];
-            rcost[s] = (float)n * area(acc);
-        }
-        const float base = (float)cnt * area(inf.cb);
-        float best_cost = kInf;
-        int best = 0;
-        for (int s = 0; s < kBins - 1; ++s) {
-            const float cost = (lcost[s] + rcost[s]) + base;
-            if (cost < best_cost) { best_cost = cost; best = s; }
-        }
-        nl = 0;
-        for (int k = 0; k <= best; ++k) nl += bn[k];
-        // scatter bases: lefts ascend from first, rights descend from last - 1
-        int lo = t.first, hi = t.last - 1;
-        for (int c = t.chunk0; c < t.chunk0 + t.nchunks; ++c) {
-            int l = 0, r = 0;
-            for (int k = 0; k < kBins; ++k) (k <= best ? l : r) += B.bin_n[(size_t)c * kBins + k];
-            B.chunk_lbase[c] = lo;
-            B.chunk_rbase[c] = hi;
-            lo += l;
-            hi -= r;
-        }
-        inf.best = best;
-    } else {
-        nl = cnt / 2;                                          // equal centroids: split in the middle
-    }
-    inf.nl = nl;
-    B.info[ti] = inf;
-    const int ranges[2][2] = {{t.first, t.first + nl}, {t.first + nl, t.last}};
-    int code[2];
-    for (int side = 0; side < 2; ++side) {
-        const int f = ranges[side][0], l = ranges[side][1];
-        if (l - f > small && t.depth + 1 < kMaxDepth) {
-            const int u = atomicAdd(&B.ctl->n_unodes, 1);
-            const int k = atomicAdd(&B.ctl->n_next_big, 1);
-            if (u >= B.unode_cap || k >= B.big_cap) { atomicOr(&B.ctl->err, 2); code[side] = -1; continue; }
-            B.next_big[k] = {f, l, t.depth + 1, u, t.set, 0, 0, 0};
-            code[side] = u;
-        } else {
-            const int k = atomicAdd(&B.ctl->n_small, 1);
-            if (k >= B.small_cap) { atomicOr(&B.ctl->err, 2); code[side] = -1; continue; }
-            B.small[k] = {f, l, t.depth + 1, (level + 1) & 1, t.set, 0, 0, 0};
-            code[side] = ~k;
-        }
-    }
-    B.unodes[t.unode].left = code[0];
-    B.unodes[t.unode].right = code[1];
-}
-
-// K5: per chunk: move the items to the next level's buffer, lefts and rights
-// in order (a middle split keeps every item's position).
-__global__ void __launch_bounds__(kThreads) k_chunk_scatter(Bufs B, int src) {
-    __shared__ int sh[kWavesPerBlock];
-    const int c = blockIdx.x;
-    const int ti = B.chunk_task[c];
+// Per task (one block): the split, the chunks' scatter bases and the two
+// children, each either a task of the next level or a small task.
+__global__ void __launch_bounds__(kThreads) k_task_split(Bufs B, int level) {
+    __shared__ int shn[kWavesPerBlock];
+    __shared__ SplitLds sp;
+    __shared__ float run_box[kRuns][kBins][6];
+    __shared__ int run_n[kRuns][kBins];
+    __shared__ int child_chunk0[2], child_task[2], pick[2];
+    const int ti = blockIdx.x, cur = level & 1;
+    if (ti >= B.ctl->n_big[level] || (B.ctl->err & kErrFinite)) return;
     const BigInfo inf = B.info[ti];
-    const BigTask t = B.big[ti];
-    const int s = B.chunk_start[c], e = min(s + kChunk, t.last);
+    const BigTask t = B.big[cur][ti];
+    const int cnt = t.last - t.first;
+    if (inf.mode == 0) {
+        // the bins over all chunks: a thread per bin, side and run of chunks, then the runs in order
+        const int j = (int)threadIdx.x % (2 * kBins), r = (int)threadIdx.x / (2 * kBins);
+        const int k = j >> 1, side = j & 1;
+        if (r < kRuns) {
+            const int len = (t.nchunks + kRuns - 1) / kRuns;
+            const int a = t.chunk0 + min(r * len, t.nchunks), z = t.chunk0 + min((r + 1) * len, t.nchunks);
+            float v[3] = {-kInf, -kInf, -kInf};
+            int n = 0;
+            for (int q = a; q < z; ++q) {
+                const Box6& x = B.bin_b[(size_t)q * kBins + k];
+#pragma unroll
+                for (int w = 0; w < 3; ++w) v[w] = later_max(v[w], x.v[3 * side + w]);
+                n += B.bin_n[(size_t)q * kBins + k];
+            }
+#pragma unroll
+            for (int w = 0; w < 3; ++w) run_box[r][k][3 * side + w] = v[w];
+            if (side == 0) run_n[r][k] = n;
+        }
+        __syncthreads();
+        if (threadIdx.x < kBins * 6) {
+            const int kk = (int)threadIdx.x / 6, w = (int)threadIdx.x % 6;
+            float v = -kInf;
+            for (int q = 0; q < kRuns; ++q) v = later_max(v, run_box[q][kk][w]);
+            sp.bin_box[kk][w] = v;
+        }
+        if (threadIdx.x < kBins) {
+            int n = 0;
+            for (int q = 0; q < kRuns; ++q) n += run_n[q][threadIdx.x];
+            sp.bin_n[threadIdx.x] = n;
+        }
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            int best, nl;
+            sah_sweep(sp, cnt, inf.cb_area, best, nl);
+            if (threadIdx.x == 0) { pick[0] = best; pick[1] = nl; }
+        }
+    } else if (threadIdx.x == 0) {
+        pick[0] = 0;
+        pick[1] = cnt / 2;                                          // equal centroids: split in the middle
+    }
+    __syncthreads();
+    const int best = pick[0], nl = pick[1];
+    const int run = (t.nchunks + kThreads - 1) / kThreads;
+    const int q0 = t.chunk0 + min((int)threadIdx.x * run, t.nchunks);
+    const int q1 = t.chunk0 + min(((int)threadIdx.x + 1) * run, t.nchunks);
+    if (inf.mode == 0) {
+        // scatter bases: lefts ascend from first, rights descend from last - 1
+        int l = 0, all = 0;
+        for (int q = q0; q < q1; ++q)
+            for (int k = 0; k < kBins; ++k) {
+                const int n = B.bin_n[(size_t)q * kBins + k];
+                l += k <= best ? n : 0;
+                all += n;
+            }
+        int lo = t.first + block_excl_scan(l, shn);
+        int hi = t.last - 1 - block_excl_scan(all - l, shn);
+        for (int q = q0; q < q1; ++q) {
+            B.chunk_lbase[q] = lo;
+            B.chunk_rbase[q] = hi;
+            for (int k = 0; k < kBins; ++k) {
+                const int n = B.bin_n[(size_t)q * kBins + k];
+                if (k <= best) lo += n; else hi -= n;
+            }
+        }
+    }
+    if (threadIdx.x == 0) {
+        B.info[ti].best = best;
+        int code[2];
+        for (int side = 0; side < 2; ++side) {
+            const int f = side ? t.first + nl : t.first, l = side ? t.last : t.first + nl;
+            child_task[side] = -1;
+            code[side] = -1;
+            if (l - f > B.small_max && t.depth + 1 < kMaxDepth) {
+                const int nc = (l - f + kChunk - 1) / kChunk;
+                const int u = atomicAdd(&B.ctl->n_unodes, 1);
+                const int k = atomicAdd(&B.ctl->n_big[level + 1], 1);
+                const int c0 = atomicAdd(&B.ctl->n_chunks[level + 1], nc);
+                if (u >= B.unode_cap || k >= B.big_cap || c0 + nc > B.chunk_cap) {
+                    atomicOr(&B.ctl->err, kErrCapacity);
+                    continue;
+                }
+                B.big[cur ^ 1][k] = {f, l, t.depth + 1, u, t.set, c0, nc, 0};
+                child_task[side] = k;
+                child_chunk0[side] = c0;
+                code[side] = u;
+            } else {
+                const int k = atomicAdd(&B.ctl->n_small, 1);
+                if (k >= B.small_cap) { atomicOr(&B.ctl->err, kErrCapacity); continue; }
+                B.small[k] = {f, l, t.depth + 1, cur ^ 1, t.set, 0, 0, 0};
+                code[side] = ~k;
+            }
+        }
+        B.unodes[t.unode].left = code[0];
+        B.unodes[t.unode].right = code[1];
+    }
+    __syncthreads();
+    for (int side = 0; side < 2; ++side) {
+        if (child_task[side] < 0) continue;
+        const int f = side ? t.first + nl : t.first, l = side ? t.last : t.first + nl;
+        const int nc = (l - f + kChunk - 1) / kChunk;
+        for (int k = threadIdx.x; k < nc; k += kThreads) {
+            B.chunk_task[cur ^ 1][child_chunk0[side] + k] = child_task[side];
+            B.chunk_start[cur ^ 1][child_chunk0[side] + k] = f + k * kChunk;
+        }
+    }
+}
+
+// Per chunk: move the items to the next level's buffer, lefts and rights
+// in order (a middle split keeps every item's position).
+__global__ void __launch_bounds__(kThreads) k_scatter(Bufs B, int level) {
+    __shared__ int sh[kWavesPerBlock];
+    const int c = blockIdx.x, cur = level & 1;
+    if (c >= B.ctl->n_chunks[level] || (B.ctl->err & kErrFinite)) return;
+    const int ti = B.chunk_task[cur][c];
+    const BigInfo inf = B.info[ti];
+    const BigTask t = B.big[cur][ti];
+    const int s = B.chunk_start[cur][c], e = min(s + kChunk, t.last);
     int b, en;
     thread_range(s, e, b, en);
-    const Item* in = B.items[src];
-    Item* out = B.items[src ^ 1];
+    const Item* in = B.items[cur];
+    Item* out = B.items[cur ^ 1];
     if (inf.mode != 0) {
         for (int i = b; i < en; ++i) store_item(out + i, load_item(in + i));
         return;
@@ -379,41 +509,6 @@ __global__ void __launch_bounds__(kThreads) k_chunk_scatter(Bufs B, int src) {
     }
 }
 
-// Next level: chunk lists of the tasks K4 appended (one block).
-__global__ void __launch_bounds__(kThreads) k_plan(Bufs B) {
-    __shared__ int sh[kWavesPerBlock];
-    __shared__ int carry;
-    const int n = B.ctl->n_next_big < B.big_cap ? B.ctl->n_next_big : B.big_cap;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < n; base += kThreads) {
-        const int i = base + threadIdx.x;
-        BigTask t{};
-        int nc = 0;
-        if (i < n) {
-            t = B.next_big[i];
-            nc = (t.last - t.first + kChunk - 1) / kChunk;
-        }
-        const int off = carry + block_excl_scan(nc, sh);
-        if (i < n) {
-            if (off + nc > B.chunk_cap) {
-                atomicOr(&B.ctl->err, 2);
-            } else {
-                B.next_big[i].chunk0 = off;
-                B.next_big[i].nchunks = nc;
-                for (int k = 0; k < nc; ++k) {
-                    B.chunk_task_next[off + k] = i;
-                    B.chunk_start_next[off + k] = t.first + k * kChunk;
-                }
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == kThreads - 1) carry = off + nc;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) B.ctl->n_chunks = carry;
-}
-
 __device__ __forceinline__ bn_bvh_node make_node(const DBox& b, int32_t word, bool leaf, int axis, int count) {
     bn_bvh_node n;
     n.pmin[0] = b.l[0]; n.pmin[1] = b.l[1]; n.pmin[2] = b.l[2];
@@ -430,33 +525,22 @@ __device__ __forceinline__ bn_bvh_node make_node(const DBox& b, int32_t word, bo
 // left first) into the task's node region, numbered in pre-order from 0.
 //
 // The task's items live in LDS; a lane holds its run of at most kPer
-// consecutive ones in registers while they are moved.  A box is kept as six
-// maxima (-lo, hi): the negation is exact and a min whose second operand wins
-// ties is the negated max whose second operand wins them.  Most nodes hold a
+// consecutive ones in registers while they are moved.  Most nodes hold a
 // few items, so a node's cost has to follow its item count: the bins are
 // folded by 48 lanes, one per bin, side and half of the items, each walking
 // the items in order (24 x 7 values through six lane-reduction steps took the
 // same time for every node: the kernel ran 2.6 ms for 240,000 items, 0.50 ms
-// like this), and the SAH sweep runs in 22 lanes, one per prefix and suffix.
+// like this, 0.26 ms for tasks of up to 128 items), and the SAH sweep runs in 22 lanes, one per prefix and suffix.
 constexpr int kPer = 4;
 constexpr int kSmallMax = 64 * kPer;
 constexpr int kRow = kSmallMax + 4;               // the two sides' rows start in different banks
-struct Box6 { float v[6]; };                      // -lo xyz, hi xyz
 struct SmallLds {
     float f[6][kRow];
     int id[kSmallMax];
     uint8_t bin[kSmallMax];
-    float bin_box[kBins][6];
-    int bin_n[kBins];
+    SplitLds split;
     int4 frames[kMaxDepth + 2];                   // first, last (in the task), depth, parent
 };
-__device__ __forceinline__ float later_max(float a, float b) { return a > b ? a : b; }
-__device__ __forceinline__ Box6 empty6() { return {{-kInf, -kInf, -kInf, -kInf, -kInf, -kInf}}; }
-__device__ __forceinline__ void join6(Box6& a, const Box6& b) {
-#pragma unroll
-    for (int c = 0; c < 6; ++c) a.v[c] = later_max(a.v[c], b.v[c]);
-}
-__device__ __forceinline__ DBox dbox(const Box6& b) { return {{-b.v[0], -b.v[1], -b.v[2]}, {b.v[3], b.v[4], b.v[5]}}; }
 // Ordered union over the first `lanes` lanes, in lane 0; broadcast.
 __device__ __forceinline__ void wave_union6(Box6& b, int lanes) {
     for (int s = 1; s < lanes; s <<= 1) {
@@ -494,35 +578,14 @@ __device__ __forceinline__ void small_split(SmallLds& S, int first, int cnt, flo
     const float ox = __shfl(x, lane + 24), oy = __shfl(y, lane + 24), oz = __shfl(z, lane + 24);
     const int on = __shfl(n, lane + 24);
     if (lane < 24) {
-        float* o = &S.bin_box[k][3 * side];
+        float* o = &S.split.bin_box[k][3 * side];
         o[0] = later_max(x, ox);
         o[1] = later_max(y, oy);
         o[2] = later_max(z, oz);
-        S.bin_n[k] = n + on;
+        S.split.bin_n[k] = n + on;
     }
     bnd::wave_sync();
-    // lane s < 11: bins [0, s] in ascending order; lane 16 + s: bins [s + 1, 12) in descending order
-    const bool right = (lane & 16) != 0;
-    const int s = lane & 15;
-    Box6 acc = empty6();
-    int c = 0;
-    for (int t = 0; t < kBins - 1; ++t) {
-        const int q = right ? kBins - 1 - t : t;
-        if (right ? t <= kBins - 2 - s : t <= s) {
-#pragma unroll
-            for (int w = 0; w < 6; ++w) acc.v[w] = later_max(acc.v[w], S.bin_box[q][w]);
-            c += S.bin_n[q];
-        }
-    }
-    const float cost1 = (float)c * area(dbox(acc));
-    const float cost = (cost1 + __shfl(cost1, lane + 16)) + (float)cnt * cb_area;
-    const bool valid = lane < kBins - 1 && cost < kInf;
-    float m = valid ? cost : kInf;
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) m = fminf(m, __shfl_xor(m, o));
-    const uint64_t at = __ballot(valid && cost == m);
-    best = at ? __ffsll((unsigned long long)at) - 1 : 0;
-    n_left = __builtin_amdgcn_readlane(c, best);
+    sah_sweep(S.split, cnt, cb_area, best, n_left);
 }
 
 __global__ void __launch_bounds__(kThreads) k_small(Bufs B, int n_small) {
@@ -642,23 +705,78 @@ __global__ void __launch_bounds__(kThreads) k_small(Bufs B, int n_small) {
     if (lane == 0) B.small_size[ti] = nodes;
 }
 
-__global__ void k_write_upper(Bufs B, int n_unodes, const int* udfs, const int* uright, bn_bvh_node* out) {
+// Pre-order numbering (one block): subtree sizes from the deepest level up,
+// the sets' places in the output, then indices from the roots down.
+constexpr int kNumThreads = 1024;
+__global__ void __launch_bounds__(kNumThreads) k_number(Bufs B, int levels) {
+    __shared__ int sh[kNumThreads / 64], carry;
+    auto size_of = [&](int code) { return code < 0 ? B.small_size[~code] : B.usize[code]; };
+    auto place = [&](int code, int idx) { if (code < 0) B.small_base[~code] = idx; else B.udfs[code] = idx; };
+    for (int d = levels - 1; d >= 0; --d) {
+        const int u0 = d > 0 ? B.ctl->unode_end[d - 1] : 0, u1 = B.ctl->unode_end[d];
+        for (int u = u0 + threadIdx.x; u < u1; u += kNumThreads)
+            B.usize[u] = 1 + size_of(B.unodes[u].left) + size_of(B.unodes[u].right);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) carry = 0;
+    __syncthreads();
+    for (int base = 0; base < B.n_sets; base += kNumThreads) {
+        const int s = base + threadIdx.x;
+        int n = 0;
+        if (s < B.n_sets) {
+            n = size_of(B.root[s]);
+            if (n <= 0 || n > 2 * (B.set_off[s + 1] - B.set_off[s])) {
+                atomicOr(&B.ctl->err, kErrCount);
+                n = 0;
+            }
+            place(B.root[s], 0);
+            B.set_nodes[s] = n;
+        }
+        int v = n;                                        // inclusive scan over the block
+        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(v, o);
+            if (lane >= o) v += y;
+        }
+        if (lane == 63) sh[w] = v;
+        __syncthreads();
+        int before = carry;
+        for (int k = 0; k < w; ++k) before += sh[k];
+        if (s < B.n_sets) B.set_base[s] = before + v - n;
+        __syncthreads();
+        if (threadIdx.x == kNumThreads - 1) carry = before + v;
+        __syncthreads();
+    }
+    for (int d = 0; d < levels; ++d) {
+        const int u0 = d > 0 ? B.ctl->unode_end[d - 1] : 0, u1 = B.ctl->unode_end[d];
+        for (int u = u0 + threadIdx.x; u < u1; u += kNumThreads) {
+            const UNode n = B.unodes[u];
+            const int idx = B.udfs[u], r = idx + 1 + size_of(n.left);
+            place(n.left, idx + 1);
+            place(n.right, r);
+            B.uright[u] = r;
+        }
+        __syncthreads();
+    }
+}
+
+__global__ void k_write_upper(Bufs B, int n_unodes, bn_bvh_node* out) {
     const int u = blockIdx.x * blockDim.x + threadIdx.x;
     if (u >= n_unodes) return;
     const UNode n = B.unodes[u];
-    out[2 * (size_t)B.set_off[n.set] + udfs[u]] = make_node(n.b, uright[u], false, n.axis, 0);
+    out[(size_t)B.set_base[n.set] + B.udfs[u]] = make_node(n.b, B.uright[u], false, n.axis, 0);
 }
 
 // Copy each region to its place in its set's node array; right-child indices
 // move with the region's base.
-__global__ void __launch_bounds__(kThreads) k_write_regions(Bufs B, int n_small, const int* rbase, bn_bvh_node* out) {
+__global__ void __launch_bounds__(kThreads) k_write_regions(Bufs B, int n_small, bn_bvh_node* out) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int ti = blockIdx.x * kWavesPerBlock + w;
     if (ti >= n_small) return;
     const SmallTask t = B.small[ti];
-    const int base = rbase[ti], n = B.small_size[ti];
+    const int base = B.small_base[ti], n = B.small_size[ti];
     const bn_bvh_node* src = B.region + 2 * (size_t)t.first;
-    bn_bvh_node* dst = out + 2 * (size_t)B.set_off[t.set] + base;
+    bn_bvh_node* dst = out + (size_t)B.set_base[t.set] + base;
     for (int k = lane; k < n; k += 64) {
         bn_bvh_node x = src[k];
         if (!x.is_leaf) x.right_or_offset += base;
@@ -685,14 +803,14 @@ void* pinned(Ctx* c, size_t bytes) {
     }
     return c->g_pinned;
 }
+size_t up16(size_t n) { return (n + 15) / 16 * 16; }
 }  // namespace
 
-void bvh_build_gpu(Ctx* c, const std::vector<const float*>& sets, const std::vector<int>& counts,
-                   std::vector<std::vector<bn_bvh_node>>& nodes_out, std::vector<std::vector<int32_t>>& perm_out) {
+GpuBvh bvh_build_gpu(Ctx* c, const std::vector<const float*>& sets, const std::vector<int>& counts) {
     const int S = (int)sets.size();
-    nodes_out.assign(S, {});
-    perm_out.assign(S, {});
-    if (S == 0) return;
+    GpuBvh g;
+    g.counts = counts;
+    if (S == 0) return g;
     std::vector<int> off(S + 1, 0);
     for (int s = 0; s < S; ++s) {
         if (counts[s] <= 0) throw Error(BN_E_INVALID, "BVH build of an empty item set");
@@ -702,28 +820,17 @@ void bvh_build_gpu(Ctx* c, const std::vector<const float*>& sets, const std::vec
     const int N = off[S];
     const int small = std::min(c->bvh_small, kSmallMax);
     const size_t item_bytes = (size_t)N * sizeof(Item);
-    // host: items into page-locked staging, finiteness, the level-0 tasks
-    Item* items = (Item*)pinned(c, std::max(item_bytes, (size_t)N * (sizeof(bn_bvh_node) * 2 + 4)));
-    for (int s = 0; s < S; ++s) {
-        const float* src = sets[s];
-        Item* dst = items + off[s];
-        bool finite = true;
-        for (int i = 0; i < counts[s]; ++i) {
-            const float* b = src + 6 * (size_t)i;
-            finite = finite && std::isfinite(b[0]) && std::isfinite(b[1]) && std::isfinite(b[2]) &&
-                     std::isfinite(b[3]) && std::isfinite(b[4]) && std::isfinite(b[5]);
-            dst[i] = {b[0], b[1], b[2], i, b[3], b[4], b[5], 0};
-        }
-        if (!finite) throw Error(BN_E_INVALID, "GPU BVH build needs finite bounds (bn_bvh_build takes any)");
-    }
     const int big_cap = N / small + S + 1;
     const int unode_cap = kMaxDepth * big_cap;
     const int small_cap = (int)std::min((int64_t)N + S, 2 * (int64_t)unode_cap + S) + 1;
     const int chunk_cap = 2 * (N / kChunk + big_cap) + 1;
+    // the level-0 tasks
     std::vector<BigTask> big0;
     std::vector<SmallTask> small0;
     std::vector<int> root(S), ctask, cstart;
+    int largest = 0;
     for (int s = 0; s < S; ++s) {
+        largest = std::max(largest, counts[s]);
         if (counts[s] > small) {
             const int u = (int)big0.size();
             const int nc = (counts[s] + kChunk - 1) / kChunk;
@@ -737,155 +844,147 @@ void bvh_build_gpu(Ctx* c, const std::vector<const float*>& sets, const std::vec
     }
     // device memory (grow-only buffers of the context)
     c->g_items.ensure(2 * std::max(item_bytes, (size_t)N * sizeof(bn_bvh_node)));   // A | B, then the nodes
-    c->g_region.ensure(2 * (size_t)N * sizeof(bn_bvh_node));
+    c->g_region.ensure(2 * (size_t)N * sizeof(bn_bvh_node));                        // the bounds, then the regions
     c->g_perm.ensure((size_t)N * 4);
     c->g_rsize.ensure((size_t)small_cap * 4 * 2);         // region sizes, region bases (by small task)
     c->g_big.ensure(2 * (size_t)big_cap * sizeof(BigTask));
     c->g_info.ensure((size_t)big_cap * sizeof(BigInfo));
     c->g_small.ensure((size_t)small_cap * sizeof(SmallTask));
     c->g_chunks.ensure(4 * (size_t)chunk_cap * 4);
-    c->g_part.ensure((size_t)chunk_cap * (2 + kBins) * sizeof(DBox) + (size_t)chunk_cap * (kBins + 2) * 4);
-    c->g_unodes.ensure((size_t)unode_cap * (sizeof(UNode) + 2 * 4));
-    c->g_misc.ensure(sizeof(Ctl) + (size_t)S * 4);
+    c->g_part.ensure((size_t)chunk_cap * (2 * sizeof(DBox) + kBins * sizeof(Box6)) + (size_t)chunk_cap * (kBins + 2) * 4);
+    c->g_unodes.ensure((size_t)unode_cap * (sizeof(UNode) + 3 * 4));
+    // what the host sets up, in one block: counters, set offsets, roots, the
+    // level-0 tasks; then what it reads back: the sets' nodes and places
+    const size_t o_off = up16(sizeof(Ctl)), o_root = o_off + up16(((size_t)S + 1) * 4);
+    const size_t o_nodes = o_root + up16((size_t)S * 4), o_base = o_nodes + up16((size_t)S * 4);
+    c->g_misc.ensure(o_base + (size_t)S * 4);
     hipStream_t st = c->stream;
     char* items_base = (char*)c->g_items.p;
+    char* misc = (char*)c->g_misc.p;
     Bufs B{};
     B.items[0] = (Item*)items_base;
     B.items[1] = (Item*)(items_base + item_bytes);
-    BigTask* bigs[2] = {(BigTask*)c->g_big.p, (BigTask*)c->g_big.p + big_cap};
     B.info = (BigInfo*)c->g_info.p;
     B.small = (SmallTask*)c->g_small.p;
-    int* chunks[4];
-    for (int k = 0; k < 4; ++k) chunks[k] = (int*)c->g_chunks.p + (size_t)k * chunk_cap;
+    for (int k = 0; k < 2; ++k) {
+        B.big[k] = (BigTask*)c->g_big.p + (size_t)k * big_cap;
+        B.chunk_task[k] = (int*)c->g_chunks.p + (size_t)(2 * k) * chunk_cap;
+        B.chunk_start[k] = (int*)c->g_chunks.p + (size_t)(2 * k + 1) * chunk_cap;
+    }
     B.part_b = (DBox*)c->g_part.p;
     B.part_cb = B.part_b + chunk_cap;
-    B.bin_b = B.part_cb + chunk_cap;
+    B.bin_b = (Box6*)(B.part_cb + chunk_cap);
     B.bin_n = (int*)(B.bin_b + (size_t)chunk_cap * kBins);
     B.chunk_lbase = B.bin_n + (size_t)chunk_cap * kBins;
     B.chunk_rbase = B.chunk_lbase + chunk_cap;
     B.unodes = (UNode*)c->g_unodes.p;
-    int* udfs = (int*)(B.unodes + unode_cap);
-    int* uright = udfs + unode_cap;
+    B.udfs = (int*)(B.unodes + unode_cap);
+    B.uright = B.udfs + unode_cap;
+    B.usize = B.uright + unode_cap;
     B.region = (bn_bvh_node*)c->g_region.p;
     B.small_size = (int*)c->g_rsize.p;
-    int* rbase = B.small_size + small_cap;
+    B.small_base = B.small_size + small_cap;
     B.perm = (int32_t*)c->g_perm.p;
-    B.ctl = (Ctl*)c->g_misc.p;
-    int* d_off = (int*)((char*)c->g_misc.p + sizeof(Ctl));
-    B.set_off = d_off;
+    B.ctl = (Ctl*)misc;
+    B.set_off = (const int*)(misc + o_off);
+    B.root = (const int*)(misc + o_root);
+    B.set_nodes = (int*)(misc + o_nodes);
+    B.set_base = (int*)(misc + o_base);
+    B.n_sets = S; B.n_items = N; B.small_max = small;
     B.big_cap = big_cap; B.small_cap = small_cap; B.unode_cap = unode_cap; B.chunk_cap = chunk_cap;
 
-    hip_check(hipMemcpyAsync(B.items[0], items, item_bytes, hipMemcpyHostToDevice, st), "bvh items");
+    // The bounds go up a piece at a time through page-locked memory, each
+    // piece copied in while the one before is on its way.
+    const size_t bounds_bytes = (size_t)N * 24;
+    char* host = (char*)pinned(c, std::max(bounds_bytes, o_base + (size_t)S * 4) + o_nodes);
+    char* head = host;                                     // the block above, then the bounds
+    char* stage = host + o_nodes;
+    Ctl ctl{};
+    ctl.n_small = (int)small0.size();
+    ctl.n_unodes = (int)big0.size();
+    ctl.n_big[0] = (int)big0.size();
+    ctl.n_chunks[0] = (int)ctask.size();
+    std::memcpy(head, &ctl, sizeof(ctl));
+    std::memcpy(head + o_off, off.data(), ((size_t)S + 1) * 4);
+    std::memcpy(head + o_root, root.data(), (size_t)S * 4);
+    hip_check(hipMemcpyAsync(misc, head, o_nodes, hipMemcpyHostToDevice, st), "bvh ctl");
     if (!big0.empty()) {
-        hip_check(hipMemcpyAsync(bigs[0], big0.data(), big0.size() * sizeof(BigTask), hipMemcpyHostToDevice, st), "bvh tasks");
-        hip_check(hipMemcpyAsync(chunks[0], ctask.data(), ctask.size() * 4, hipMemcpyHostToDevice, st), "bvh chunks");
-        hip_check(hipMemcpyAsync(chunks[1], cstart.data(), cstart.size() * 4, hipMemcpyHostToDevice, st), "bvh chunks");
+        hip_check(hipMemcpyAsync(B.big[0], big0.data(), big0.size() * sizeof(BigTask), hipMemcpyHostToDevice, st), "bvh tasks");
+        hip_check(hipMemcpyAsync(B.chunk_task[0], ctask.data(), ctask.size() * 4, hipMemcpyHostToDevice, st), "bvh chunks");
+        hip_check(hipMemcpyAsync(B.chunk_start[0], cstart.data(), cstart.size() * 4, hipMemcpyHostToDevice, st), "bvh chunks");
     }
     if (!small0.empty())
         hip_check(hipMemcpyAsync(B.small, small0.data(), small0.size() * sizeof(SmallTask), hipMemcpyHostToDevice, st),
                   "bvh small tasks");
-    hip_check(hipMemcpyAsync(d_off, off.data(), S * 4, hipMemcpyHostToDevice, st), "bvh sets");
-    Ctl ctl{};
-    ctl.n_small = (int)small0.size();
-    ctl.n_unodes = (int)big0.size();
-    hip_check(hipMemcpyAsync(B.ctl, &ctl, sizeof(Ctl), hipMemcpyHostToDevice, st), "bvh ctl");
-
-    int n_big = (int)big0.size(), n_chunks = (int)ctask.size(), cur = 0;
-    for (int level = 0; n_big > 0; ++level) {
-        if (level >= kMaxDepth) throw Error(BN_E_INVALID, "GPU BVH build: deeper than the depth limit");
-        B.big = bigs[cur];
-        B.next_big = bigs[cur ^ 1];
-        B.chunk_task = chunks[2 * cur];
-        B.chunk_start = chunks[2 * cur + 1];
-        B.chunk_task_next = chunks[2 * (cur ^ 1)];
-        B.chunk_start_next = chunks[2 * (cur ^ 1) + 1];
-        const int src = level & 1;
-        const int tb = (n_big + 63) / 64;
-        hip_check(hipMemsetAsync(&B.ctl->n_next_big, 0, 4, st), "bvh ctl");
-        k_chunk_bounds<<<n_chunks, kThreads, 0, st>>>(B, src);
-        k_task_bounds<<<tb, 64, 0, st>>>(B, n_big);
-        k_chunk_bins<<<n_chunks, kThreads, 0, st>>>(B, src);
-        k_task_split<<<tb, 64, 0, st>>>(B, n_big, level, small);
-        k_chunk_scatter<<<n_chunks, kThreads, 0, st>>>(B, src);
-        k_plan<<<1, kThreads, 0, st>>>(B);
-        hip_check(hipGetLastError(), "bvh level launch");
-        hip_check(hipMemcpyAsync(&ctl, B.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st), "bvh ctl");
-        hip_check(hipStreamSynchronize(st), "bvh level");
-        if (ctl.err) throw Error(BN_E_CAPACITY, "GPU BVH build: task capacity exceeded");
-        n_big = ctl.n_next_big;
-        n_chunks = ctl.n_chunks;
-        cur ^= 1;
-    }
-    const int n_small = ctl.n_small;
-    const int n_unodes = ctl.n_unodes;
-    if (n_small > 0) k_small<<<(n_small + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, 0, st>>>(B, n_small);
-    hip_check(hipGetLastError(), "bvh small launch");
-    // Pre-order numbering of the upper trees on the host (a few nodes per
-    // 512 items): subtree sizes, then each upper node's index and right
-    // child and each region's base.
-    std::vector<UNode> un(n_unodes);
-    std::vector<SmallTask> sm(n_small);
-    std::vector<int> rsize(n_small);
-    if (n_unodes) hip_check(hipMemcpyAsync(un.data(), B.unodes, n_unodes * sizeof(UNode), hipMemcpyDeviceToHost, st), "bvh upper");
-    hip_check(hipMemcpyAsync(sm.data(), B.small, n_small * sizeof(SmallTask), hipMemcpyDeviceToHost, st), "bvh small");
-    hip_check(hipMemcpyAsync(rsize.data(), B.small_size, n_small * 4, hipMemcpyDeviceToHost, st), "bvh sizes");
-    hip_check(hipMemcpyAsync(&ctl, B.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st), "bvh ctl");
-    hip_check(hipStreamSynchronize(st), "bvh subtrees");
-    if (ctl.err & 1) throw Error(BN_E_CAPACITY, "BVH leaf larger than the int8 count field");
-    if (ctl.err) throw Error(BN_E_CAPACITY, "GPU BVH build: task capacity exceeded");
-    std::vector<int> usize(n_unodes), h_udfs(n_unodes), h_uright(n_unodes), h_rbase(n_small), nn(S);
-    auto size_of = [&](int code) { return code < 0 ? rsize[~code] : usize[code]; };
-    std::vector<std::pair<int, int>> stk;
-    for (int s = 0; s < S; ++s) {
-        stk.assign(1, {root[s], 0});
-        while (!stk.empty()) {                               // post-order: sizes
-            auto& [code, vis] = stk.back();
-            if (code < 0) { stk.pop_back(); continue; }
-            const int u = code;
-            if (!vis) {
-                vis = 1;
-                stk.push_back({un[u].right, 0});
-                stk.push_back({un[u].left, 0});
-            } else {
-                stk.pop_back();
-                usize[u] = 1 + size_of(un[u].left) + size_of(un[u].right);
+    constexpr size_t kUp = (size_t)1 << 20;
+    size_t sent = 0, filled = 0;
+    for (int s = 0; s < S; ++s)
+        for (size_t a = 0, n = (size_t)counts[s] * 24; a < n;) {
+            const size_t m = std::min(n - a, kUp - (filled - sent));
+            std::memcpy(stage + filled, (const char*)sets[s] + a, m);
+            a += m;
+            filled += m;
+            if (filled - sent == kUp || filled == bounds_bytes) {
+                hip_check(hipMemcpyAsync((char*)c->g_region.p + sent, stage + sent, filled - sent, hipMemcpyHostToDevice, st),
+                          "bvh bounds");
+                sent = filled;
             }
         }
-        nn[s] = size_of(root[s]);
-        if (nn[s] <= 0 || nn[s] > 2 * counts[s]) throw Error(BN_E_DEVICE, "GPU BVH build: inconsistent node count");
-        stk.assign(1, {root[s], 0});
-        while (!stk.empty()) {                               // pre-order: indices
-            const auto [code, idx] = stk.back();
-            stk.pop_back();
-            if (code < 0) { h_rbase[~code] = idx; continue; }
-            const int sl = size_of(un[code].left);
-            h_udfs[code] = idx;
-            h_uright[code] = idx + 1 + sl;
-            stk.push_back({un[code].right, idx + 1 + sl});
-            stk.push_back({un[code].left, idx + 1});
+    k_items<<<std::min((N + kThreads - 1) / kThreads, 8 * c->n_cu), kThreads, 0, st>>>(B, (const float*)c->g_region.p);
+    hip_check(hipGetLastError(), "bvh items launch");
+    auto read_ctl = [&] {
+        hip_check(hipMemcpyAsync(&ctl, B.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st), "bvh ctl");
+        hip_check(hipStreamSynchronize(st), "bvh level");
+        if (ctl.err & kErrFinite) throw Error(BN_E_INVALID, "GPU BVH build needs finite bounds (bn_bvh_build takes any)");
+        if (ctl.err & kErrCapacity) throw Error(BN_E_CAPACITY, "GPU BVH build: task capacity exceeded");
+    };
+    // Levels: as many as an even tree has and three more, then four at a time
+    // while there are tasks left.  A level holds at most twice the tasks of
+    // the one before, and a chunk more than its items fill per task.
+    int level = 0;
+    if (big0.empty()) read_ctl();
+    for (int todo = 3 + (int)std::ceil(std::log2(std::max(2.0, (double)largest / small)));
+         !big0.empty() && (level == 0 || ctl.n_big[level] > 0); todo = 4) {
+        for (int k = 0; k < todo && level < kMaxDepth; ++k, ++level) {
+            const int64_t tasks = std::min<int64_t>((int64_t)big0.size() << std::min(level, 30), big_cap);
+            const int grid = (int)std::min<int64_t>(N / kChunk + tasks + 1, chunk_cap);
+            k_chunk_bounds<<<grid, kThreads, 0, st>>>(B, level);
+            k_task_bounds<<<(int)tasks, 64, 0, st>>>(B, level);
+            k_chunk_bins<<<grid, kThreads, 0, st>>>(B, level);
+            k_task_split<<<(int)tasks, kThreads, 0, st>>>(B, level);
+            k_scatter<<<grid, kThreads, 0, st>>>(B, level);
         }
+        hip_check(hipGetLastError(), "bvh level launch");
+        read_ctl();
+        if (level >= kMaxDepth && ctl.n_big[kMaxDepth] > 0)
+            throw Error(BN_E_INVALID, "GPU BVH build: deeper than the depth limit");
     }
-    bn_bvh_node* out = (bn_bvh_node*)items_base;                // the item buffers are done with
-    if (n_unodes) {
-        hip_check(hipMemcpyAsync(udfs, h_udfs.data(), n_unodes * 4, hipMemcpyHostToDevice, st), "bvh numbering");
-        hip_check(hipMemcpyAsync(uright, h_uright.data(), n_unodes * 4, hipMemcpyHostToDevice, st), "bvh numbering");
-        k_write_upper<<<(n_unodes + 255) / 256, 256, 0, st>>>(B, n_unodes, udfs, uright, out);
-    }
-    hip_check(hipMemcpyAsync(rbase, h_rbase.data(), n_small * 4, hipMemcpyHostToDevice, st), "bvh numbering");
-    k_write_regions<<<(n_small + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, 0, st>>>(B, n_small, rbase, out);
+    const int n_small = ctl.n_small, n_unodes = ctl.n_unodes;
+    bn_bvh_node* out = (bn_bvh_node*)items_base;                // the item buffers are done with after k_small
+    if (n_small > 0) k_small<<<(n_small + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, 0, st>>>(B, n_small);
+    k_number<<<1, kNumThreads, 0, st>>>(B, level);
+    if (n_unodes) k_write_upper<<<(n_unodes + 255) / 256, 256, 0, st>>>(B, n_unodes, out);
+    if (n_small > 0) k_write_regions<<<(n_small + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, 0, st>>>(B, n_small, out);
     hip_check(hipGetLastError(), "bvh flatten launch");
-    // results through the staging memory: the nodes of every set, then the permutation
-    bn_bvh_node* h_nodes = (bn_bvh_node*)items;
-    int32_t* h_perm = (int32_t*)(h_nodes + 2 * (size_t)N);
-    for (int s = 0; s < S; ++s)
-        hip_check(hipMemcpyAsync(h_nodes + 2 * (size_t)off[s], out + 2 * (size_t)off[s], nn[s] * sizeof(bn_bvh_node),
-                                 hipMemcpyDeviceToHost, st), "bvh nodes");
-    hip_check(hipMemcpyAsync(h_perm, B.perm, (size_t)N * 4, hipMemcpyDeviceToHost, st), "bvh perm");
-    hip_check(hipStreamSynchronize(st), "bvh copy");
-    for (int s = 0; s < S; ++s) {
-        nodes_out[s].assign(h_nodes + 2 * (size_t)off[s], h_nodes + 2 * (size_t)off[s] + nn[s]);
-        perm_out[s].assign(h_perm + off[s], h_perm + off[s + 1]);
+    hip_check(hipMemcpyAsync(host, misc, o_base, hipMemcpyDeviceToHost, st), "bvh sizes");
+    hip_check(hipStreamSynchronize(st), "bvh subtrees");
+    std::memcpy(&ctl, host, sizeof(ctl));
+    if (ctl.err & kErrLeaf) throw Error(BN_E_CAPACITY, "BVH leaf larger than the int8 count field");
+    if (ctl.err & kErrCount) throw Error(BN_E_DEVICE, "GPU BVH build: inconsistent node count");
+    g.n_nodes.assign((const int*)(host + o_nodes), (const int*)(host + o_nodes) + S);
+    g.nodes = out;
+    g.perm = B.perm;
+    return g;
+}
+
+void bvh_fetch(Ctx* c, const GpuBvh& g, const std::vector<bn_bvh_node*>& nodes, const std::vector<int32_t*>& perms) {
+    std::vector<HostCopy::Part> pn, pp;
+    for (size_t s = 0; s < g.counts.size(); ++s) {
+        pn.push_back({nodes[s], (size_t)g.n_nodes[s] * sizeof(bn_bvh_node)});
+        pp.push_back({perms[s], (size_t)g.counts[s] * 4});
     }
+    c->host_copy.download(g.nodes, pn, c->stream);
+    c->host_copy.download(g.perm, pp, c->stream);
 }
 
 }  // namespace bnx

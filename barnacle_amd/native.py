@@ -13,12 +13,14 @@ import os
 import numpy as np
 
 from . import abi
+from .bvh_util import NODE_DTYPE
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libbarnacle_hip.so")
 
 f32p = C.POINTER(C.c_float)
 i32p = C.POINTER(C.c_int32)
+nodep = C.POINTER(abi.BVHNode)
 
 
 class BarnacleError(RuntimeError):
@@ -102,12 +104,9 @@ def bvh_build(bounds):
     lib = load()
     b = np.ascontiguousarray(bounds, np.float32).reshape(-1, 6)
     n = len(b)
-    nodes = (abi.BVHNode * (2 * n + 1))()
-    nn = C.c_int32(2 * n + 1)
-    perm = np.zeros(n, np.int32)
-    check(lib.bn_bvh_build(_p(b, f32p), n, nodes, C.byref(nn), _p(perm, i32p)))
-    from .bvh_util import nodes_to_numpy
-    return nodes_to_numpy(nodes, nn.value), perm
+    nodes, nn, perm = np.empty(2 * n + 1, NODE_DTYPE), C.c_int32(2 * n + 1), np.empty(n, np.int32)
+    check(lib.bn_bvh_build(_p(b, f32p), n, _p(nodes, nodep), C.byref(nn), _p(perm, i32p)))
+    return nodes[:nn.value], perm
 
 
 class Context:
@@ -137,12 +136,10 @@ class Context:
         """BVHNode.Build (Util/BVH.fs:128-247) on this context's GPU: (nodes, perm)."""
         b = np.ascontiguousarray(bounds, np.float32).reshape(-1, 6)
         n = len(b)
-        nodes = (abi.BVHNode * (2 * n + 1))()
-        nn = C.c_int32(2 * n + 1)
-        perm = np.zeros(n, np.int32)
-        check(self.lib.bn_bvh_build_gpu(self.h, _p(b, f32p), n, nodes, C.byref(nn), _p(perm, i32p)))
-        from .bvh_util import nodes_to_numpy
-        return nodes_to_numpy(nodes, nn.value), perm
+        # memory that the build does not write stays untouched
+        nodes, nn, perm = np.empty(2 * n + 1, NODE_DTYPE), C.c_int32(2 * n + 1), np.empty(n, np.int32)
+        check(self.lib.bn_bvh_build_gpu(self.h, _p(b, f32p), n, _p(nodes, nodep), C.byref(nn), _p(perm, i32p)))
+        return nodes[:nn.value], perm
 
     def kernel_times(self):
         """{kernel name: (launches, total ms)} accumulated since the last reset."""

@@ -375,8 +375,12 @@ int bn_render_batch(bn_ctx* ctx, const bn_batch_item* items, int32_t n, float* c
  *                          atomics gain from material-coherent waves
  *   "bvh_gpu"              1 (default): bn_scene_build builds mesh BLAS on the
  *                          GPU (bn_bvh_build_gpu); 0: on the host
- *   "bvh_small"            largest subtree (triangles, 128..512, default 512)
- *                          that one workgroup of the GPU build finishes alone
+ *   "bvh_small"            largest subtree (triangles, 128..512, default 128)
+ *                          that one wave of the GPU build finishes alone; more
+ *                          than 256 mean 256
+ *   "mlt_wave_chains"      up to so many PSSMLT chains (default 20480) one wave
+ *                          runs each chain's mutations; more advance together
+ *                          as a wavefront.  The chains are the same either way.
  *   "overlap_shadow"       1 (default): path-tracing frames trace each bounce's
  *                          shadow rays on a second stream beside the next
  *                          bounce's closest-hit traversal; 0: one stream
