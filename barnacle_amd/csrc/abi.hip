@@ -254,7 +254,28 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     sc.lights_host = lights;
     const std::vector<float4> dmats = pack_materials(mats);
     const std::vector<float4> dl = pack_lights(lights);
+    std::vector<bnh::Box> boxes(insts.size());
+    for (size_t i = 0; i < insts.size(); ++i) {
+        const float* b = insts[i].bounds;
+        boxes[i] = {{b[0], b[1], b[2]}, {b[3], b[4], b[5]}};
+    }
+    bnh::VisitOrder vo;
+    bool flat = bnh::visit_order(tlas, boxes, bnd::kFlatMax, vo);
+    bnd::FlatScene fs{};
+    if (flat) {
+        for (size_t i = 0; i < insts.size(); ++i) {
+            std::memcpy(fs.inst[i].lo, insts[i].bounds, 12);
+            std::memcpy(fs.inst[i].hi, insts[i].bounds + 3, 12);
+        }
+        for (int o = 0; o < 8; ++o)
+            for (size_t p = 0; p < insts.size(); ++p) {
+                fs.order[o][p] = vo.order[o][p];
+                fs.inst[vo.order[o][p]].place[o / 4] |= (uint32_t)p << (8 * (o % 4));
+            }
+        std::copy(vo.after.begin(), vo.after.end(), fs.after);
+    }
     hipStream_t s = c->stream;
+    sc.flat.upload(&fs, sizeof fs, s);
     sc.tlas.upload(tlas.data(), tlas.size() * sizeof(bn_bvh_node), s);
     sc.blas.upload(nodes.data(), nodes.size() * sizeof(bn_bvh_node), s);
     sc.tris.upload(tris.data(), tris.size() * sizeof(float), s);
@@ -295,6 +316,10 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     for (const auto& in : insts)
         for (int k = 0; k < 6; ++k) finite = finite && std::isfinite(in.bounds[k]);
     sc.dev.exact_only = finite ? 0 : 1;
+    flat = flat && finite;
+    sc.dev.flat = flat ? (const bnd::FlatScene*)sc.flat.p : nullptr;
+    sc.dev.n_insts = sc.n_insts;
+    sc.dev.n_tlas = (int)tlas.size();
     sc.live = true;
 }
 
@@ -764,10 +789,11 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
                           ":" + std::to_string(whole ? n : 0) + ":" + std::to_string(Lr.stream2 != nullptr);
         if (Lr.uniform) {
             const bnd::DevScene& d = Lr.scene;
-            for (const void* q : {(const void*)d.tlas, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
+            for (const void* q : {(const void*)d.tlas, (const void*)d.flat, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
                                   (const void*)d.mats})
                 key += ":" + std::to_string((uintptr_t)q);
-            key += ":" + std::to_string(d.exact_only) + ":" + std::to_string(Lr.grid_uniform);
+            key += ":" + std::to_string(d.exact_only) + ":" + std::to_string(d.n_insts) + ":" +
+                   std::to_string(d.n_tlas) + ":" + std::to_string(Lr.grid_uniform);
         }
         auto f = c->graphs.find(key);
         if (f == c->graphs.end()) {

@@ -120,6 +120,18 @@ struct DevInst {
     int4 info;      // x = BLAS root node (-1: sphere), y = first triangle, z = material, w = light
     int4 aux;       // x = 1: w2o is exactly the identity (entries +0.0f and 1.0f), yzw unused
 };
+// A scene of few instances as a list (bnh::flat_instances): what a ray needs
+// to find the instances whose bounds it meets without the TLAS.
+// 32: the bits of one register hold a ray's instances; testing all of them
+// costs a refill about two wave steps then, and a walk takes more.
+constexpr int kFlatMax = 32;
+struct FlatScene {
+    // bounds of each instance, and its place in the visit order of each octant
+    // of ray directions (a byte per octant)
+    struct Inst { float lo[3], hi[3]; uint32_t place[2]; } inst[kFlatMax];
+    uint8_t order[8][kFlatMax];      // the instance at each place, per octant (bit k: component k > 0)
+    int after[2 * kFlatMax];         // per TLAS node: the first node behind its subtree
+};
 struct DevScene {
     const float4* tlas;
     const float4* blas;
@@ -139,6 +151,8 @@ struct DevScene {
     float4 dv;                  // pixel delta V, w = focus distance
     int cam_kind;
     int exact_only;             // scene has non-finite geometry: exact slab tests only
+    const FlatScene* flat;      // null: the scene is traversed through its TLAS
+    int n_insts, n_tlas;
 };
 
 struct Ray { V3 o, d; };

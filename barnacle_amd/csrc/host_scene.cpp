@@ -358,6 +358,59 @@ void build_bvh(const std::vector<Box>& in, std::vector<bn_bvh_node>& nodes, std:
     for (int i = 0; i < n; ++i) perm[i] = items[i].id;
 }
 
+bool visit_order(const std::vector<bn_bvh_node>& nodes, const std::vector<Box>& items, int most, VisitOrder& out) {
+    const int n = (int)items.size(), n_nodes = (int)nodes.size();
+    if (n < 1 || n > most || n_nodes > 2 * most) return false;
+    for (const Box& b : items)
+        for (const float* f : {&b.lo.x, &b.hi.x})
+            for (int k = 0; k < 3; ++k)
+                if (!std::isfinite(f[k])) return false;
+    out.after.assign(n_nodes, 0);
+    // inside(i): the items below node i lie in its bounds and in those above
+    std::function<bool(int, Box)> inside = [&](int i, Box above) {
+        const bn_bvh_node& b = nodes[i];
+        above.lo = vmax(above.lo, {b.pmin[0], b.pmin[1], b.pmin[2]});
+        above.hi = vmin(above.hi, {b.pmax[0], b.pmax[1], b.pmax[2]});
+        if (!b.is_leaf) {
+            if (!inside(i + 1, above) || !inside(b.right_or_offset, above)) return false;
+            out.after[i] = out.after[b.right_or_offset];
+            return b.right_or_offset == out.after[i + 1];
+        }
+        out.after[i] = i + 1;
+        for (int k = b.right_or_offset; k < b.right_or_offset + b.count; ++k) {
+            const Box& t = items[k];
+            if (!(t.lo.x >= above.lo.x && t.lo.y >= above.lo.y && t.lo.z >= above.lo.z && t.hi.x <= above.hi.x &&
+                  t.hi.y <= above.hi.y && t.hi.z <= above.hi.z))
+                return false;
+        }
+        return true;
+    };
+    if (!inside(0, {{-kInf, -kInf, -kInf}, {kInf, kInf, kInf}})) return false;
+    for (int o = 0; o < 8; ++o) {
+        std::vector<uint8_t>& seq = out.order[o];
+        seq.clear();
+        std::vector<int> stack{0};
+        while (!stack.empty()) {
+            const int i = stack.back();
+            stack.pop_back();
+            const bn_bvh_node& b = nodes[i];
+            if (b.is_leaf) {
+                for (int k = 0; k < b.count; ++k) seq.push_back((uint8_t)(b.right_or_offset + k));
+                if ((int)seq.size() > n) return false;
+                continue;
+            }
+            const bool left_near = (o >> b.split_axis) & 1;
+            stack.push_back(left_near ? b.right_or_offset : i + 1);
+            stack.push_back(left_near ? i + 1 : b.right_or_offset);
+        }
+        std::vector<uint8_t> sorted = seq;
+        std::sort(sorted.begin(), sorted.end());
+        for (int k = 0; k < n; ++k)
+            if ((int)sorted.size() != n || sorted[k] != k) return false;
+    }
+    return true;
+}
+
 AliasTable build_alias(const float* w, int n) {
     AliasTable t;
     t.alias.resize(n);

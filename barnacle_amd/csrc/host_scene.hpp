@@ -89,6 +89,18 @@ Box transform_box(const Box& b, const M4& m);    // AxisAlignedBoundingBox.Trans
 // pre-order; perm[i] is the input index of the item placed at position i.
 void build_bvh(const std::vector<Box>& items, std::vector<bn_bvh_node>& nodes, std::vector<int32_t>& perm);
 
+// The order in which a TLAS walk reaches the instances, for a scene of few.
+// order[o][p]: the instance that a ray of octant o (bit k: direction component
+// k > 0) meets as the p-th, if it meets them all; after[i]: the first node
+// behind the subtree of node i.  False where a list cannot stand for the tree:
+// more than `most` instances, non-finite bounds, an instance outside the nodes
+// above it, or one that is not in exactly one leaf.
+struct VisitOrder {
+    std::vector<uint8_t> order[8];
+    std::vector<int32_t> after;
+};
+bool visit_order(const std::vector<bn_bvh_node>& nodes, const std::vector<Box>& items, int most, VisitOrder& out);
+
 // AliasTable construction (Util/AliasTable.fs:14-51).
 struct AliasTable {
     std::vector<int32_t> alias;

@@ -63,6 +63,7 @@ template <>
 struct Work<false> {
     DevScene S;
     RoundItem it;
+    bool flat() const { return S.flat != nullptr; }
     __device__ __forceinline__ int n() const { return 1; }
     __device__ __forceinline__ int item_of_path(uint32_t) const { return 0; }
     __device__ __forceinline__ int item_of(const PathBuf&, uint32_t) const { return 0; }
@@ -80,6 +81,7 @@ struct Work<true> {
     const RoundHeader* hdr;
     const RoundItem* items;
     const DevScene* scenes;
+    bool flat() const { return false; }
     __device__ __forceinline__ int n() const { return hdr->n_items; }
     // item owning a path id (the round table is ordered by path_base)
     __device__ __forceinline__ int item_of_path(uint32_t id) const {
@@ -349,12 +351,12 @@ __device__ __forceinline__ int next_segment(const SegFetch& F, uint32_t pick, ui
     return -1;
 }
 
-template <bool ANY, bool COUNT, int K, typename Setup, typename Init, typename Done>
+template <bool ANY, bool COUNT, int K, bool FLAT, typename Setup, typename Init, typename Done>
 __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uint32_t* stk, uint32_t* spill,
                                                  size_t spill_stride, uint32_t refill, TraceCount& tc, Setup setup,
                                                  Init init, Done done) {
     const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    Traversal<K> tr;
+    Traversal<K, FLAT> tr;
     tr.st = LaneStack<K>{stk + threadIdx.x, (int)blockDim.x, spill + gid, spill_stride, 0};
     tr.clear();
     setup(tr);
@@ -428,7 +430,7 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
 // With a 16-entry LDS stack window seven blocks fit a CU's LDS; the register
 // budget is then set for seven waves per SIMD (72 VGPRs; eight would spill),
 // six in batches.
-template <bool COUNT, bool BATCH, int K>
+template <bool COUNT, bool BATCH, int K, bool FLAT>
 __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_closest(Work<BATCH> W, PathBuf P, Ctl* ctl, int cur,
                                                        const uint32_t* queue, uint32_t* spill, size_t spill_stride,
                                                        uint32_t refill, unsigned long long* stats, uint32_t* seg) {
@@ -440,20 +442,21 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
         else ctl->q_count[1 - cur] = 0;
     }
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, COUNT, K>(
+    persistent_trace<false, COUNT, K, FLAT>(
         SegFetch{seg, kFetchSegs}, count, stk, spill, spill_stride, refill, tc,
-        [&](Traversal<K>& tr) { W.bind(tr.G); },
-        [&](Traversal<K>& tr, uint32_t i) {
+        [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
+        [&](Traversal<K, FLAT>& tr, uint32_t i) {
             const uint32_t slot = queue ? queue[i] : i;
             const float4 o4 = P.o[slot];
             const int k = W.item_of(P, slot);
             W.bind_lane(tr.G, k);
             tr.start({xyz(o4), xyz(P.d[slot])}, kInf, W.scene(k).exact_only != 0);
-            if (!COUNT) tr.take_tlas_root();
+            if (FLAT) tr.take_instances(false);
+            else if (!COUNT) tr.take_tlas_root();
             // a placeholder path (padding pixel, max-depth 0) misses at once
             if (__float_as_int(o4.w) < 0) tr.empty();
         },
-        [&](Traversal<K>& tr, uint32_t i, bool fin, bool) {
+        [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool) {
             if (fin) {
                 const uint32_t slot = queue ? queue[i] : i;
                 int bin = -1;
@@ -851,7 +854,7 @@ __global__ __launch_bounds__(256, 3) void k_shade_c(Work<BATCH> W, PathBuf X, Pa
 // an unoccluded ray adds beta*f * Le/(pdf_b + pdf_l) to L.  Slot rounds: the
 // rays of the slots in shq, added to the slot's L.  Compact rounds (shq
 // null): ray i, added to L_out[path id] (nee_a.w).
-template <bool COUNT, bool BATCH, int K>
+template <bool COUNT, bool BATCH, int K, bool FLAT>
 __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_shadow(Work<BATCH> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                       float4* L_out, int par,
                                                       uint32_t* spill, size_t spill_stride, uint32_t refill,
@@ -859,20 +862,21 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = shq && par < 0 ? ctl->sh_count : ctl->shc[par];
     TraceCount tc{0, 0, 0};
-    persistent_trace<true, COUNT, K>(
+    persistent_trace<true, COUNT, K, FLAT>(
         SegFetch{seg, kShadowSegs}, count, stk, spill, spill_stride, refill, tc,
-        [&](Traversal<K>& tr) { W.bind(tr.G); },
-        [&](Traversal<K>& tr, uint32_t i) {
+        [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
+        [&](Traversal<K, FLAT>& tr, uint32_t i) {
             const uint32_t slot = shq ? shq[i] : i;
             const float4 o4 = P.sh_o[slot], d4 = P.sh_d[slot];
             const int k = shq ? W.item_of(P, slot) : (BATCH ? __float_as_int(d4.w) : 0);
             W.bind_lane(tr.G, k);
             tr.start({xyz(o4), xyz(d4)}, o4.w, W.scene(k).exact_only != 0);
-            if (!COUNT) tr.take_tlas_root();
+            if (FLAT) tr.take_instances(true);
+            else if (!COUNT) tr.take_tlas_root();
             // a NaN t max fails every slab test of the reference: empty traversal
             if (!(o4.w == o4.w)) tr.empty();
         },
-        [&](Traversal<K>& tr, uint32_t i, bool fin, bool found) {
+        [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool found) {
             if (fin && !found) {
                 const uint32_t slot = shq ? shq[i] : i;
                 const float4 a = P.nee_a[slot];
@@ -1108,24 +1112,25 @@ __global__ __launch_bounds__(LDS ? kGradLdsThreads : 256) void k_shade_adj(
 // The shadow rays of a replayed bounce only record their visibility (in
 // nee_a.w): gradient sums belong in a kernel whose lanes are all busy, not in
 // the traversal loop.
-template <int K>
+template <int K, bool FLAT>
 __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_trace_shadow_vis(Work<false> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                           uint32_t* spill, size_t spill_stride, uint32_t refill,
                                                           uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = ctl->sh_count;
     TraceCount tc{0, 0, 0};
-    persistent_trace<true, false, K>(
+    persistent_trace<true, false, K, FLAT>(
         SegFetch{seg, kShadowSegs}, count, stk, spill, spill_stride, refill, tc,
-        [&](Traversal<K>& tr) { W.bind(tr.G); },
-        [&](Traversal<K>& tr, uint32_t i) {
+        [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
+        [&](Traversal<K, FLAT>& tr, uint32_t i) {
             const uint32_t slot = shq[i];
             const float4 o4 = P.sh_o[slot];
             tr.start({xyz(o4), xyz(P.sh_d[slot])}, o4.w, W.S.exact_only != 0);
-            tr.take_tlas_root();
+            if (FLAT) tr.take_instances(true);
+            else tr.take_tlas_root();
             if (!(o4.w == o4.w)) tr.empty();
         },
-        [&](Traversal<K>& tr, uint32_t i, bool fin, bool found) {
+        [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool found) {
             if (fin) P.nee_a[shq[i]].w = found ? 0.0f : 1.0f;
         });
 }
@@ -1329,26 +1334,27 @@ __global__ void k_shade_direct(Work<false> W, PathBuf P, Ctl* ctl, const uint32_
 }
 
 // First hit of one sample per pixel: (instance, primitive, t) in pixel order.
-template <int K>
+template <int K, bool FLAT>
 __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
                                                    int frame_id, int* out_inst, int* out_prim, float* out_t,
                                                    uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs) {
     __shared__ uint32_t stk[K * 256];
     const uint32_t n = (uint32_t)width * (uint32_t)height;
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, false, K>(
+    persistent_trace<false, false, K, FLAT>(
         SegFetch{fetch, segs}, n, stk, spill, spill_stride, 16u, tc,
-        [&](Traversal<K>& tr) { tr.G.set(S); },
-        [&](Traversal<K>& tr, uint32_t p) {
+        [&](Traversal<K, FLAT>& tr) { tr.G.set(S); },
+        [&](Traversal<K, FLAT>& tr, uint32_t p) {
             const int x = (int)(p % (uint32_t)width), y = (int)(p / (uint32_t)width);
             uint32_t rng = xxhash3((uint32_t)x, (uint32_t)y, (uint32_t)(frame_id * spp + sample_id));
             V2 uPix, uLens;
             uPix.x = lcg(rng); uPix.y = lcg(rng);
             uLens.x = lcg(rng); uLens.y = lcg(rng);
             tr.start(camera_ray(S, x, y, uPix, uLens), kInf, S.exact_only != 0);
-            tr.take_tlas_root();
+            if (FLAT) tr.take_instances(false);
+            else tr.take_tlas_root();
         },
-        [&](Traversal<K>& tr, uint32_t p, bool fin, bool) {
+        [&](Traversal<K, FLAT>& tr, uint32_t p, bool fin, bool) {
             if (fin) {
                 out_inst[p] = tr.hit_inst;
                 out_prim[p] = tr.hit_prim;
@@ -1376,11 +1382,12 @@ static Work<true> batch_work(const Launch& L) {
 template <bool BATCH>
 static void launch_closest_t(bool count, int k, const Work<BATCH>& W, const PathBuf& P, Ctl* ctl, int cur,
                              const uint32_t* queue, const Buffers& B, uint32_t refill, int grid, hipStream_t st) {
-#define BN_TC(C, KK)                                                                                            \
-    hipLaunchKernelGGL((k_trace_closest<C, BATCH, KK>), dim3(grid), dim3(256), 0, st, W, P, ctl, cur, queue, \
+#define BN_TC(C, KK, F)                                                                                            \
+    hipLaunchKernelGGL((k_trace_closest<C, BATCH, KK, F>), dim3(grid), dim3(256), 0, st, W, P, ctl, cur, queue, \
                        B.spill, B.spill_stride, refill, B.stats, B.fetch_seg)
-    if (k == 16) { if (count) BN_TC(true, 16); else BN_TC(false, 16); }
-    else { if (count) BN_TC(true, 32); else BN_TC(false, 32); }
+    if (count) { if (k == 16) BN_TC(true, 16, false); else BN_TC(true, 32, false); }
+    else if (W.flat()) { if (k == 16) BN_TC(false, 16, !BATCH); else BN_TC(false, 32, !BATCH); }
+    else { if (k == 16) BN_TC(false, 16, false); else BN_TC(false, 32, false); }
 #undef BN_TC
 }
 // par: the parity of a compact round's iteration (its shadow count and fetch
@@ -1391,11 +1398,12 @@ static void launch_shadow_t(bool count, int k, const Work<BATCH>& W, const PathB
                             uint32_t* spill = nullptr) {
     uint32_t* seg = B.fetch_seg + (size_t)(kFetchSegs + (par < 0 ? 0 : par) * kShadowSegs) * kSegStride;
     if (!spill) spill = B.spill;
-#define BN_TS(C, KK)                                                                                            \
-    hipLaunchKernelGGL((k_trace_shadow<C, BATCH, KK>), dim3(grid), dim3(256), 0, st, W, P, ctl, shq, L_out, par, \
+#define BN_TS(C, KK, F)                                                                                            \
+    hipLaunchKernelGGL((k_trace_shadow<C, BATCH, KK, F>), dim3(grid), dim3(256), 0, st, W, P, ctl, shq, L_out, par, \
                        spill, B.spill_stride, refill, B.stats, seg)
-    if (k == 16) { if (count) BN_TS(true, 16); else BN_TS(false, 16); }
-    else { if (count) BN_TS(true, 32); else BN_TS(false, 32); }
+    if (count) { if (k == 16) BN_TS(true, 16, false); else BN_TS(true, 32, false); }
+    else if (W.flat()) { if (k == 16) BN_TS(false, 16, !BATCH); else BN_TS(false, 32, !BATCH); }
+    else { if (k == 16) BN_TS(false, 16, false); else BN_TS(false, 32, false); }
 #undef BN_TS
 }
 
@@ -1546,12 +1554,10 @@ static void iterations_t(const Work<BATCH>& W, Integrator kind, const Launch& L,
                   } }
                 { Bracket b(hook, "trace_shadow", st);
                   uint32_t* seg = B.fetch_seg + kFetchSegs * kSegStride;
-                  if (B.stack_k == 16)
-                      hipLaunchKernelGGL(k_trace_shadow_vis<16>, dim3(L.grid_trace), dim3(256), 0, st, W, P, ctl,
-                                         B.shq, B.spill, B.spill_stride, L.refill, seg);
-                  else
-                      hipLaunchKernelGGL(k_trace_shadow_vis<32>, dim3(L.grid_trace), dim3(256), 0, st, W, P, ctl,
-                                         B.shq, B.spill, B.spill_stride, L.refill, seg); }
+                  auto* vis = W.flat() ? (B.stack_k == 16 ? k_trace_shadow_vis<16, true> : k_trace_shadow_vis<32, true>)
+                                       : (B.stack_k == 16 ? k_trace_shadow_vis<16, false> : k_trace_shadow_vis<32, false>);
+                  hipLaunchKernelGGL(vis, dim3(L.grid_trace), dim3(256), 0, st, W, P, ctl, B.shq, B.spill,
+                                     B.spill_stride, L.refill, seg); }
                 { Bracket b(hook, "nee_adj", st);
                   if (B.adj.lds_bytes > 0) {
                       hipFuncSetAttribute((const void*)k_nee_adj_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1645,12 +1651,10 @@ void launch_trace_shadow(bool count, const DevScene& S, const PathBuf& P, Ctl* c
 void launch_first_hit(const DevScene& S, int w, int h, int sample_id, int spp, int frame_id, int* inst, int* prim,
                       float* t, uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs, int stack_k, int grid,
                       hipStream_t st) {
-    if (stack_k == 16)
-        hipLaunchKernelGGL(k_first_hit<16>, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst,
-                           prim, t, spill, spill_stride, fetch, segs);
-    else
-        hipLaunchKernelGGL(k_first_hit<32>, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst,
-                           prim, t, spill, spill_stride, fetch, segs);
+    auto* hit = S.flat ? (stack_k == 16 ? k_first_hit<16, true> : k_first_hit<32, true>)
+                       : (stack_k == 16 ? k_first_hit<16, false> : k_first_hit<32, false>);
+    hipLaunchKernelGGL(hit, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst, prim, t, spill,
+                       spill_stride, fetch, segs);
 }
 
 }  // namespace bnd

@@ -59,10 +59,34 @@ struct TraceScene {
     const float4* blas;
     const float* tris;
     const DevInst* insts;
-    __device__ __forceinline__ void set(const DevScene& S) { tlas = S.tlas; blas = S.blas; tris = S.tris; insts = S.insts; }
+    const FlatScene* flat;
+    int n_insts, n_tlas;
+    __device__ __forceinline__ void set(const DevScene& S) {
+        tlas = S.tlas; blas = S.blas; tris = S.tris; insts = S.insts;
+        flat = S.flat; n_insts = S.n_insts; n_tlas = S.n_tlas;
+    }
 };
 
-template <int K>
+// Read through the scalar cache: the same address in all lanes, memory that no
+// kernel writes.
+template <typename T>
+using Scalar = const T __attribute__((address_space(4)));
+template <typename T>
+__device__ __forceinline__ Scalar<T>* scalar(const T* p) { return (Scalar<T>*)(uintptr_t)p; }
+
+// FLAT: for scenes of at most kFlatMax instances (DevScene::flat).  A ray meets
+// all instance bounds when it starts, and the ones it hits become the bits of
+// `left`, in the order in which the reference's TLAS walk reaches them (each
+// octant of ray directions has one order, known on the host; an any-hit query
+// takes them as they are).  An instance is tested again when it is taken, with
+// the t of that moment, as the reference does; a TLAS node contains the bounds
+// below it, so a ray that meets an instance has met the nodes above it.
+// The start costs about 27 instructions an instance, which all lanes of a
+// refill share; the walk was the larger part of the steps: with 9 instances 18
+// of 38 busy lanes of a wave step stood at a TLAS node or at an instance they
+// then missed, and the traversal is bound by instruction issue.  Config-1 frame
+// 109 -> 89 ms, 1024x768 frame of analytic spheres 11.7 -> 8.8 ms.
+template <int K, bool FLAT = false>
 struct Traversal {
     TraceScene G;
     // world ray and the ray of the current space (world, or object inside a BLAS)
@@ -76,6 +100,7 @@ struct Traversal {
     uint32_t nxt;        // node to take before the stack (kNoNode: none); kNeedTest: box not tested yet
     int blas_base;       // stack depth at BLAS entry, -1 in the TLAS
     int tl_cur, tl_end;  // instances left in the current TLAS leaf
+    uint32_t left;       // FLAT: places of the instances still to be taken
     int bl_cur, bl_end;  // triangles left in the current BLAS leaf (global indices)
     int blas_root, tri_base, cur_inst;
 
@@ -94,6 +119,7 @@ struct Traversal {
         tl_cur = tl_end = 0;
         bl_cur = bl_end = 0;
         blas_root = tri_base = cur_inst = 0;
+        if (FLAT) { left = 0; nxt = kNoNode; }
     }
 
     // No traversal at all (placeholder rays, NaN t max).
@@ -101,6 +127,42 @@ struct Traversal {
         st.sp = 0;
         nxt = kNoNode;
         tl_cur = tl_end = 0;
+        if (FLAT) left = 0;
+    }
+    // FLAT: the instances the ray of start() meets.
+    __device__ __forceinline__ uint32_t octant_shift() const {
+        return (wd.x > 0.0f ? 8u : 0u) + (wd.y > 0.0f ? 16u : 0u) + (wd.z > 0.0f ? 32u : 0u);
+    }
+    __device__ __forceinline__ void take_instances(bool any) {
+        Scalar<FlatScene>* F = scalar(G.flat);
+        const uint32_t oct = octant_shift();
+        for (int i = 0; i < G.n_insts; ++i) {
+            Scalar<FlatScene::Inst>& f = F->inst[i];
+            const uint64_t place = (uint64_t)f.place[1] << 32 | f.place[0];
+            const bool h = slab_fast(mk(f.lo[0], f.lo[1], f.lo[2]), mk(f.hi[0], f.hi[1], f.hi[2]), wo, winv, t);
+            const uint32_t bit = 1u << (any ? (uint32_t)i : (uint32_t)(place >> oct) & 31u);
+            left |= h ? bit : 0u;
+        }
+        if (exact) take_instances_exact(any);
+    }
+    // A ray whose slab test can see a NaN meets what the walk lets through:
+    // the node tests have NaNs of their own.
+    __device__ __forceinline__ void take_instances_exact(bool any) {
+        const uint32_t oct = octant_shift() >> 3;
+        left = 0;
+        for (int i = 0; i < G.n_tlas;) {
+            const NodeView n = load_node(G.tlas, i);
+            if (!slab(n.lo, n.hi, wo, winv, t)) {
+                i = G.flat->after[i];
+                continue;
+            }
+            if (n.leaf)
+                for (int k = 0; k < G.n_insts; ++k) {
+                    const int inst = any ? k : (int)G.flat->order[oct][k];
+                    if (inst >= n.word && inst < n.word + n.count) left |= 1u << k;
+                }
+            ++i;
+        }
     }
     // The fast traversal tests a root when it is reached: the TLAS root when
     // the ray starts, a BLAS root when its instance is entered.  A failing
@@ -131,6 +193,7 @@ struct Traversal {
         blas_base = -1;
         tl_cur = tl_end = 0;
         bl_cur = bl_end = 0;
+        if (FLAT) left = 0;
     }
 
     // The fast test is evaluated first, in the block that computes its
@@ -254,6 +317,12 @@ struct Traversal {
     // What this lane does next (leaving a finished BLAS first): kItemTri,
     // kItemInst, kItemTNode (any node), or kItemNone when it has finished.
     __device__ __forceinline__ int next_kind() {
+        if (FLAT) {
+            // the ray of a finished BLAS is simply not used any more
+            if (bl_cur < bl_end) return kItemTri;
+            if (nxt != kNoNode || st.sp > 0) return kItemTNode;
+            return left ? kItemInst : kItemNone;
+        }
         // Selects rather than a branch: the ray registers are then updated in
         // place instead of through copies at the join.
         const bool leave = blas_base >= 0 && bl_cur >= bl_end && nxt == kNoNode && st.sp == blas_base;
@@ -285,9 +354,22 @@ struct Traversal {
     // One instance of the current TLAS leaf: a sphere is intersected, a mesh
     // BLAS is entered.  Returns false on an any-hit.
     __device__ __forceinline__ bool do_inst(bool any, bool& found) {
-        const int idx = tl_cur++;
+        int idx;
+        if (FLAT) {
+            idx = __ffs((int)left) - 1;
+            left &= left - 1;
+            if (!any) idx = (int)G.flat->order[octant_shift() >> 3][idx];
+        } else {
+            idx = tl_cur++;
+        }
         const DevInst& I = G.insts[idx];
-        if (!box(xyz(I.lo), xyz(I.hi))) return true;
+        if (FLAT) {
+            bool r = slab_fast(xyz(I.lo), xyz(I.hi), wo, winv, t);
+            if (exact) r = slab(xyz(I.lo), xyz(I.hi), wo, winv, t);
+            if (!r) return true;
+        } else if (!box(xyz(I.lo), xyz(I.hi))) {
+            return true;
+        }
         const int4 info = I.info;
         if (info.x >= 0 && I.aux.x != 0 && !exact) {
             // Identity world-to-object map on a finite ray: Transform gives
@@ -327,7 +409,7 @@ struct Traversal {
         cur_inst = idx;
         blas_root = info.x;
         tri_base = info.y;
-        blas_base = st.sp;
+        if (!FLAT) blas_base = st.sp;
         take_root(G.blas + 2 * (size_t)info.x, true);
     }
 
@@ -351,14 +433,15 @@ struct Traversal {
         uint32_t e;
         if (nxt != kNoNode) { e = nxt; nxt = kNoNode; }
         else e = st.pop();
-        const float4* base = blas_base >= 0 ? G.blas + 2 * (size_t)blas_root : G.tlas;
+        const bool in_blas = FLAT || blas_base >= 0;
+        const float4* base = in_blas ? G.blas + 2 * (size_t)blas_root : G.tlas;
         const int node = (int)e;
         const float4 b = base[2 * node + 1];
         const int word = __float_as_int(b.z);
         const uint32_t f = __float_as_uint(b.w);
         if (f & 0xff) {
             const int count = (int)(int8_t)((f >> 16) & 0xff);
-            if (blas_base < 0) { tl_cur = word; tl_end = word + count; }
+            if (!in_blas) { tl_cur = word; tl_end = word + count; }
             else { bl_cur = tri_base + word; bl_end = bl_cur + count; }
             return;
         }
@@ -380,7 +463,7 @@ struct Traversal {
             if (tf & 0xff) {
                 const int cnt = (int)(int8_t)((tf >> 16) & 0xff);
                 const int w = __float_as_int(tb.z);
-                if (blas_base < 0) { tl_cur = w; tl_end = w + cnt; }
+                if (!in_blas) { tl_cur = w; tl_end = w + cnt; }
                 else { bl_cur = tri_base + w; bl_end = bl_cur + cnt; }
             } else {
                 nxt = (uint32_t)(take_left ? l : r);

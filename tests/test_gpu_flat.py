@@ -1,0 +1,78 @@
+"""Scenes of at most 32 instances are traversed through a list of their bounds
+in place of the TLAS: the same films and hits as the walk of the reference's
+tree (the counting kernels), on both sides of the limit, for rays with zero
+direction components (whose slab tests see NaNs: bounds in the plane of the
+origin) and for a tree whose nodes do not contain their instances."""
+import numpy as np
+import pytest
+
+from barnacle_amd import configs, scene
+from test_gpu_upload import reupload
+
+pytestmark = pytest.mark.gpu
+
+
+def cubes(n, fov):
+    info = configs.cornell_box(27, 21, 3, 5, boxes=False)
+    info["camera"]["fov"] = fov
+    eye = info["transforms"][-1]["keyframes"][0]["translation"]
+    info["primitives"].append({"type": "cube"})
+    rng = np.random.default_rng(n)
+    for k in range(n - len(info["instances"])):
+        key = {"time": 0.0, "scale": [float(x) for x in rng.uniform(10, 60, 3)],
+               "translation": [float(rng.uniform(50, 500)), float(rng.uniform(50, 500)), float(-rng.uniform(50, 500))]}
+        if k % 3 == 0:                      # a face in the plane of the camera
+            key["translation"][k % 2] = eye[k % 2] + key["scale"][k % 2]
+        elif k % 3 == 1:
+            key["rotation"] = [float(x) for x in rng.uniform(-1, 1, 3)]
+        info["instances"].append({"primitive": len(info["primitives"]) - 1, "material": k % 3})
+        info["transforms"].append({"keyframes": [key]})
+        info["nodes"].append({"instances": [len(info["instances"]) - 1], "transform": len(info["transforms"]) - 1})
+        info["nodes"][0]["children"].append(len(info["nodes"]) - 1)
+    return scene.load_scene(info)
+
+
+def same(a, b):
+    return np.array_equal(np.asarray(a).view(np.int32), np.asarray(b).view(np.int32))
+
+
+@pytest.mark.parametrize("fov", [39.3, 0.0])
+@pytest.mark.parametrize("n", [6, 7, 20, 31, 32, 33, 40])
+def test_few_instances_equal_the_tree_walk(ctx, orc, n, fov):
+    print(f"{n} instances, fov {fov}", flush=True)
+    sc = cubes(n, fov)
+    ds = ctx.scene(sc)
+    p = sc.pt_params()
+    walked, _ = ds.render_pt(p, stats=True)
+    assert same(ds.render_pt(p), walked)
+    for film in ctx.render_batch([(ds, p), (ds, p)])[0]:
+        assert same(film, walked)
+    for got, want in zip(ds.first_hit(p, 0), orc.scene(sc).first_hit(p, 0)):
+        assert same(got, want)
+    for got, want in zip(ds.first_hit_noalloc(p, 1), orc.scene(sc).first_hit(p, 1)):
+        assert same(got, want)
+    ds.release()
+
+
+@pytest.mark.parametrize("shrink", [0, 1, 2])
+def test_tree_that_does_not_contain_its_instances(ctx, shrink):
+    """An uploaded TLAS culls what its nodes leave out, whatever the bounds of
+    the instances say."""
+    sc = cubes(14, 39.3)
+    built = ctx.scene(sc)
+    export = built.export
+
+    def cut():
+        ex = export()
+        node = ex["tlas"][min(shrink, len(ex["tlas"]) - 1)]
+        node["pmin"][0] += np.float32(0.4) * (node["pmax"][0] - node["pmin"][0])
+        return ex
+
+    built.export = cut
+    up, _ = reupload(ctx, sc, built)
+    p = sc.pt_params()
+    walked, _ = up.render_pt(p, stats=True)
+    assert same(up.render_pt(p), walked)
+    assert not same(walked, built.render_pt(p))
+    up.release()
+    built.release()
