@@ -103,16 +103,14 @@ struct Timed {
     ~Timed() { t.end(s); }
 };
 
-// True when the row-major 4x4 map has 1.0f on the diagonal and +0.0f (the bit
-// pattern 0) everywhere else.  Vector3.Transform by such a map returns
-// x*1 + y*0 + z*0 + 0 = x + 0.0f per coordinate: the input with -0 made +0.
-static bool is_identity_bits(const float* m) {
+// True when the row-major 4x4 map has 1.0f on the diagonal and a zero of either
+// sign everywhere else (the inverse of an identity holds negative ones).
+// Vector3.Transform by such a map returns finite coordinates as they are, but
+// for the sign of a zero.
+static bool is_identity(const float* m) {
     for (int r = 0; r < 4; ++r)
-        for (int k = 0; k < 4; ++k) {
-            uint32_t u;
-            std::memcpy(&u, &m[4 * r + k], 4);
-            if (u != (r == k ? 0x3f800000u : 0u)) return false;
-        }
+        for (int k = 0; k < 4; ++k)
+            if (m[4 * r + k] != (r == k ? 1.0f : 0.0f)) return false;
     return true;
 }
 
@@ -245,7 +243,17 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
         d.hi = make_float4(in.bounds[3], in.bounds[4], in.bounds[5], pdf_const);
         d.info = make_int4(in.blas >= 0 ? base[in.blas].first : -1, in.blas >= 0 ? base[in.blas].second : 0,
                            in.material, in.light);
-        d.aux = make_int4(is_identity_bits(in.w2o) ? 1 : 0, 0, 0, 0);
+        d.aux = make_int4(0, -1, 0, 0);
+        if (in.blas >= 0) {
+            const bn_bvh_node& root = c->blas[in.blas].nodes[0];
+            bool own = is_identity(in.w2o);
+            for (int k = 0; k < 3; ++k) own = own && in.bounds[k] == root.pmin[k] && in.bounds[3 + k] == root.pmax[k];
+            d.aux.x = own ? 1 : 0;
+            if (root.is_leaf) {
+                d.aux.y = d.info.y + root.right_or_offset;
+                d.aux.z = d.aux.y + root.count;
+            }
+        }
         if (in.light >= 0) lrec.push_back(make_int4((int)i, d.info.y, ntri, in.light));
     }
     for (const auto& m : mats)

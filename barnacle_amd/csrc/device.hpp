@@ -118,7 +118,8 @@ struct DevInst {
     float4 lo;      // world bounds min, w = sphere radius
     float4 hi;      // world bounds max, w = EvalPDF constant of a mesh light
     int4 info;      // x = BLAS root node (-1: sphere), y = first triangle, z = material, w = light
-    int4 aux;       // x = 1: w2o is exactly the identity (entries +0.0f and 1.0f), yzw unused
+    int4 aux;       // x = 1: w2o is the identity (entries 1 and zeros of either sign) and the world bounds are
+                    // the BLAS root's; y, z: first triangle and end of a BLAS that is one leaf, else y = -1
 };
 // A scene of few instances as a list (bnh::flat_instances): what a ray needs
 // to find the instances whose bounds it meets without the TLAS.

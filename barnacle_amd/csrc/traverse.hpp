@@ -371,14 +371,26 @@ struct Traversal {
             return true;
         }
         const int4 info = I.info;
-        if (info.x >= 0 && I.aux.x != 0 && !exact) {
-            // Identity world-to-object map on a finite ray: Transform gives
-            // o + 0 per coordinate and d unchanged (no component of d is 0
-            // when 1/d is finite), so the object ray's 1/d is the world one.
-            co = mk(wo.x + 0.0f, wo.y + 0.0f, wo.z + 0.0f);
+        const int4 aux = I.aux;
+        if (info.x >= 0 && aux.x != 0 && !exact) {
+            // Identity world-to-object map on a finite ray: Transform gives o
+            // but for the signs of zeros and d unchanged (no component of d
+            // is 0 when 1/d is finite), so the object ray's 1/d is the world
+            // one.  The sign of a zero coordinate changes no test: it is
+            // subtracted from box and triangle coordinates, and no comparison
+            // sees the sign of a zero difference.  The instance's bounds are
+            // its root's, so the root is not tested again, and one that is a
+            // leaf is not even read (frame of instances 17.1 -> 16.8 ms,
+            // 2^20 Metropolis chains 123 -> 120).
+            co = wo;
             cd = wd;
             cinv = winv;
-            enter_blas(idx, info);
+            cur_inst = idx;
+            blas_root = info.x;
+            tri_base = info.y;
+            if (!FLAT) blas_base = st.sp;
+            if (aux.y >= 0) { bl_cur = aux.y; bl_end = aux.z; }
+            else nxt = 0u;
             return true;
         }
         const Xf w2o = I.w2o;

@@ -76,3 +76,33 @@ def test_tree_that_does_not_contain_its_instances(ctx, shrink):
     assert not same(walked, built.render_pt(p))
     up.release()
     built.release()
+
+
+@pytest.mark.parametrize("change", ["instance", "root"])
+def test_identity_instance_with_bounds_of_its_own(ctx, change):
+    """An instance with an identity transform enters its BLAS without a test of
+    the root only where the bounds of the two are the same."""
+    sc = cubes(8, 39.3)
+    built = ctx.scene(sc)
+    if change == "instance":
+        insts = built.export_instances()
+        for rec in insts[:4]:
+            rec.bounds[0] += np.float32(0.3) * np.float32(rec.bounds[3] - rec.bounds[0])
+        built.export_instances = lambda: insts
+    else:
+        export_blas = built.export_blas
+
+        def cut(prim):
+            b = export_blas(prim)
+            root = b["nodes"][0]
+            root["pmin"][0] += np.float32(0.3) * (root["pmax"][0] - root["pmin"][0])
+            return b
+
+        built.export_blas = cut
+    up, _ = reupload(ctx, sc, built)
+    p = sc.pt_params()
+    walked, _ = up.render_pt(p, stats=True)
+    assert same(up.render_pt(p), walked)
+    assert not same(walked, built.render_pt(p))
+    up.release()
+    built.release()
