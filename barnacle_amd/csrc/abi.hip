@@ -200,8 +200,8 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     }
     if (tlas.empty()) throw Error(BN_E_INVALID, "empty TLAS");
     validate_bvh(tlas, (int)insts.size(), "TLAS");
-    // BLAS pool: nodes keep their BLAS-local child indices; each instance
-    // records where its BLAS starts in the node and triangle pools.
+    // BLAS pool: child and triangle indices of the nodes become those of the
+    // node and triangle pools; each instance records where its BLAS starts.
     std::map<int, std::pair<int, int>> base;      // BLAS id -> (first node, first triangle)
     std::vector<bn_bvh_node> nodes;
     std::vector<float> tris, aprob, apdf;
@@ -210,7 +210,10 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
         if (in.blas < 0 || base.count(in.blas)) continue;
         const BlasRec& b = c->blas[in.blas];
         base[in.blas] = {(int)nodes.size(), (int)(tris.size() / 9)};
-        nodes.insert(nodes.end(), b.nodes.begin(), b.nodes.end());
+        for (bn_bvh_node n : b.nodes) {
+            n.right_or_offset += n.is_leaf ? base[in.blas].second : base[in.blas].first;
+            nodes.push_back(n);
+        }
         tris.insert(tris.end(), b.tris.begin(), b.tris.end());
         aprob.insert(aprob.end(), b.alias.prob.begin(), b.alias.prob.end());
         apdf.insert(apdf.end(), b.alias.pdf.begin(), b.alias.pdf.end());
@@ -324,7 +327,8 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     for (const auto& in : insts)
         for (int k = 0; k < 6; ++k) finite = finite && std::isfinite(in.bounds[k]);
     sc.dev.exact_only = finite ? 0 : 1;
-    flat = flat && finite;
+    // the list traversal addresses the pools with 32-bit byte offsets
+    flat = flat && finite && sc.blas.bytes < ((size_t)1 << 32) && sc.tris.bytes < ((size_t)1 << 32);
     sc.dev.flat = flat ? (const bnd::FlatScene*)sc.flat.p : nullptr;
     sc.dev.n_insts = sc.n_insts;
     sc.dev.n_tlas = (int)tlas.size();

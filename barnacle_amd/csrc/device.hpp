@@ -117,7 +117,8 @@ struct DevInst {
     Xf w2o, o2w;
     float4 lo;      // world bounds min, w = sphere radius
     float4 hi;      // world bounds max, w = EvalPDF constant of a mesh light
-    int4 info;      // x = BLAS root node (-1: sphere), y = first triangle, z = material, w = light
+    int4 info;      // x = BLAS root node (-1: sphere), y = first triangle, z = material, w = light (indices
+                    // into the scene's pools, as are those inside the BLAS nodes)
     int4 aux;       // x = 1: w2o is the identity (entries 1 and zeros of either sign) and the world bounds are
                     // the BLAS root's; y, z: first triangle and end of a BLAS that is one leaf, else y = -1
 };
@@ -226,26 +227,29 @@ __device__ __forceinline__ NodeView load_node(const float4* nodes, int i) {
     return n;
 }
 
-// Per-lane traversal stack: a window of K entries in LDS over a per-lane
-// overflow area in global memory (entry e of lane g at spill[e * stride + g]).
-template <int K>
+// Per-lane traversal stack: a window of K entries in LDS (rows of PITCH lanes)
+// over a per-lane overflow area in global memory (entry e of lane g at
+// spill[e * spill_stride + g]; the areas hold fewer than 2^32 words).
+template <int K, int PITCH>
 struct LaneStack {
-    uint32_t* lds;        // &shared[0][threadIdx.x], row pitch = blockDim.x
-    int pitch;
-    uint32_t* spill;      // &spill[gid]
-    size_t spill_stride;
+    uint32_t* lds;        // &shared[0][lane of the block]
+    uint32_t* spill;
+    uint32_t spill_stride, lane;
     int sp;
+    __device__ __forceinline__ uint32_t& over() const {
+        return spill[(uint32_t)(sp - K) * spill_stride + lane];
+    }
     __device__ __forceinline__ void push(uint32_t v) {
-        int slot = sp & (K - 1);
-        if (sp >= K) spill[(size_t)(sp - K) * spill_stride] = lds[slot * pitch];
-        lds[slot * pitch] = v;
+        const int slot = sp & (K - 1);
+        if (sp >= K) over() = lds[slot * PITCH];
+        lds[slot * PITCH] = v;
         ++sp;
     }
     __device__ __forceinline__ uint32_t pop() {
         --sp;
-        int slot = sp & (K - 1);
-        uint32_t v = lds[slot * pitch];
-        if (sp >= K) lds[slot * pitch] = spill[(size_t)(sp - K) * spill_stride];
+        const int slot = sp & (K - 1);
+        const uint32_t v = lds[slot * PITCH];
+        if (sp >= K) lds[slot * PITCH] = over();
         return v;
     }
 };

@@ -515,8 +515,8 @@ __global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBu
     extern __shared__ float4 xs[];
     __shared__ uint32_t stk[kMltWaveK * 64];
     const int lane = (int)lane_id();
-    Traversal<kMltWaveK> tr;
-    tr.st = LaneStack<kMltWaveK>{stk + lane, 64, spill + (size_t)blockIdx.x * 64 + lane, spill_stride, 0};
+    Traversal<kMltWaveK, false, 64> tr;
+    tr.st = LaneStack<kMltWaveK, 64>{stk + lane, spill, (uint32_t)spill_stride, blockIdx.x * 64u + (uint32_t)lane, 0};
     tr.clear();
     tr.G.set(S);
     // a whole traversal of one ray, the same in every lane
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBu
             for (int depth = 0; depth < max_depth; ++depth) {
                 trace(r, kInf, false);
                 if (tr.hit_inst < 0) break;
-                const Geom g = hit_geometry(S, r, tr.hit_inst, tr.hit_prim, tr.t);
+                const Geom g = hit_geometry(S, r, tr.hit_inst, tr.prim_of(S.insts[tr.hit_inst].info), tr.t);
                 const int4 info = S.insts[tr.hit_inst].info;
                 if (info.w >= 0) {
                     V3 Le;

@@ -355,11 +355,18 @@ template <bool ANY, bool COUNT, int K, bool FLAT, typename Setup, typename Init,
 __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uint32_t* stk, uint32_t* spill,
                                                  size_t spill_stride, uint32_t refill, TraceCount& tc, Setup setup,
                                                  Init init, Done done) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
     Traversal<K, FLAT> tr;
-    tr.st = LaneStack<K>{stk + threadIdx.x, (int)blockDim.x, spill + gid, spill_stride, 0};
+    tr.st = LaneStack<K, 256>{stk + threadIdx.x, spill, (uint32_t)spill_stride, gid, 0};
     tr.clear();
     setup(tr);
+    __shared__ uint8_t order[FLAT ? sizeof(FlatScene::order) : 1];
+    if (FLAT) {
+        static_assert(sizeof(FlatScene::order) == 256, "a byte for each thread");
+        order[threadIdx.x] = tr.G.flat->order[threadIdx.x / kFlatMax][threadIdx.x % kFlatMax];
+        tr.order = order;
+        __syncthreads();
+    }
     // wave-uniform values are kept in scalar registers
     const uint32_t wave = uniform(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     const uint32_t n_waves = gridDim.x * (blockDim.x >> 6);
@@ -431,7 +438,7 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
 // budget is then set for seven waves per SIMD (72 VGPRs; eight would spill),
 // six in batches.
 template <bool COUNT, bool BATCH, int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_closest(Work<BATCH> W, PathBuf P, Ctl* ctl, int cur,
+__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_trace_closest(Work<BATCH> W, PathBuf P, Ctl* ctl, int cur,
                                                        const uint32_t* queue, uint32_t* spill, size_t spill_stride,
                                                        uint32_t refill, unsigned long long* stats, uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
@@ -459,13 +466,14 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
         [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool) {
             if (fin) {
                 const uint32_t slot = queue ? queue[i] : i;
-                int bin = -1;
+                int bin = -1, prim = -1;
                 if (tr.hit_inst >= 0) {
                     const DevScene& S = W.scene(W.item_of(P, slot));
                     const int4 info = S.insts[tr.hit_inst].info;
+                    prim = tr.prim_of(info);
                     bin = info.z >= 0 ? __float_as_int(S.mats[2 * info.z].x) : kBins - 1;
                 }
-                P.hit[slot] = make_int4(tr.hit_inst, tr.hit_prim, __float_as_int(tr.t), bin);
+                P.hit[slot] = make_int4(tr.hit_inst, prim, __float_as_int(tr.t), bin);
             }
         });
     if (COUNT) {
@@ -855,7 +863,7 @@ __global__ __launch_bounds__(256, 3) void k_shade_c(Work<BATCH> W, PathBuf X, Pa
 // rays of the slots in shq, added to the slot's L.  Compact rounds (shq
 // null): ray i, added to L_out[path id] (nee_a.w).
 template <bool COUNT, bool BATCH, int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_shadow(Work<BATCH> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
+__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_trace_shadow(Work<BATCH> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                       float4* L_out, int par,
                                                       uint32_t* spill, size_t spill_stride, uint32_t refill,
                                                       unsigned long long* stats, uint32_t* seg) {
@@ -1113,7 +1121,7 @@ __global__ __launch_bounds__(LDS ? kGradLdsThreads : 256) void k_shade_adj(
 // nee_a.w): gradient sums belong in a kernel whose lanes are all busy, not in
 // the traversal loop.
 template <int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_trace_shadow_vis(Work<false> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
+__global__ __launch_bounds__(256, K == 16 ? (FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_trace_shadow_vis(Work<false> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                           uint32_t* spill, size_t spill_stride, uint32_t refill,
                                                           uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
@@ -1335,7 +1343,7 @@ __global__ void k_shade_direct(Work<false> W, PathBuf P, Ctl* ctl, const uint32_
 
 // First hit of one sample per pixel: (instance, primitive, t) in pixel order.
 template <int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
+__global__ __launch_bounds__(256, K == 16 ? (FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
                                                    int frame_id, int* out_inst, int* out_prim, float* out_t,
                                                    uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs) {
     __shared__ uint32_t stk[K * 256];
@@ -1357,7 +1365,7 @@ __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(De
         [&](Traversal<K, FLAT>& tr, uint32_t p, bool fin, bool) {
             if (fin) {
                 out_inst[p] = tr.hit_inst;
-                out_prim[p] = tr.hit_prim;
+                out_prim[p] = tr.hit_inst >= 0 ? tr.prim_of(S.insts[tr.hit_inst].info) : -1;
                 out_t[p] = tr.hit_inst >= 0 ? tr.t : kInf;
             }
         });

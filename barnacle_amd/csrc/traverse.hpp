@@ -86,23 +86,40 @@ __device__ __forceinline__ Scalar<T>* scalar(const T* p) { return (Scalar<T>*)(u
 // of 38 busy lanes of a wave step stood at a TLAS node or at an instance they
 // then missed, and the traversal is bound by instruction issue.  Config-1 frame
 // 109 -> 89 ms, 1024x768 frame of analytic spheres 11.7 -> 8.8 ms.
-template <int K, bool FLAT = false>
+template <int K, bool FLAT, int PITCH = 256>
 struct Traversal {
     TraceScene G;
     // world ray and the ray of the current space (world, or object inside a BLAS)
     V3 wo, wd, winv;
     V3 co, cd, cinv;
     float t;
-    int hit_inst, hit_prim;
+    int hit_inst, hit_prim;   // hit_prim: triangle of the pool, or the branch of a sphere
     bool exact;          // take the NaN-exact slab path
     // traversal position
-    LaneStack<K> st;
+    LaneStack<K, PITCH> st;
     uint32_t nxt;        // node to take before the stack (kNoNode: none); kNeedTest: box not tested yet
     int blas_base;       // stack depth at BLAS entry, -1 in the TLAS
     int tl_cur, tl_end;  // instances left in the current TLAS leaf
     uint32_t left;       // FLAT: places of the instances still to be taken
-    int bl_cur, bl_end;  // triangles left in the current BLAS leaf (global indices)
-    int blas_root, tri_base, cur_inst;
+    int bl_cur, bl_end;  // triangles left in the current BLAS leaf
+    int cur_inst;
+    const uint8_t* order;   // FLAT: a copy of FlatScene::order in LDS
+
+    // The primitive of the hit as the reference numbers it: a mesh's triangle.
+    __device__ __forceinline__ int prim_of(int4 info) const { return hit_prim - (info.x >= 0 ? info.y : 0); }
+
+    // Half of a node.  FLAT scenes have pools of less than 4 GiB: an offset of
+    // 32 bits to a base in scalar registers takes no 64-bit address arithmetic.
+    // (With indices into the pools in the nodes, so that a lane holds no BLAS
+    // root or first triangle, and the order in LDS: config-1 frame 89 -> 84 ms.)
+    __device__ __forceinline__ static float4 node_half(const float4* nodes, int i, int half) {
+        if (FLAT) return *(const float4*)((const char*)nodes + ((uint32_t)i * 32u + 16u * half));
+        return nodes[2 * i + half];
+    }
+    __device__ __forceinline__ static Tri load_tri32(const float* tris, int i) {
+        const float* p = (const float*)((const char*)tris + ((uint32_t)i * 32u + (uint32_t)i * 4u));
+        return {{p[0], p[1], p[2]}, {p[3], p[4], p[5]}, {p[6], p[7], p[8]}};
+    }
 
     // A new ray over the geometry already in G (set once per launch for a
     // single scene, per ray in a batch).
@@ -118,7 +135,7 @@ struct Traversal {
         blas_base = -1;
         tl_cur = tl_end = 0;
         bl_cur = bl_end = 0;
-        blas_root = tri_base = cur_inst = 0;
+        cur_inst = 0;
         if (FLAT) { left = 0; nxt = kNoNode; }
     }
 
@@ -158,7 +175,7 @@ struct Traversal {
             }
             if (n.leaf)
                 for (int k = 0; k < G.n_insts; ++k) {
-                    const int inst = any ? k : (int)G.flat->order[oct][k];
+                    const int inst = any ? k : (int)order[oct * kFlatMax + k];
                     if (inst >= n.word && inst < n.word + n.count) left |= 1u << k;
                 }
             ++i;
@@ -170,19 +187,19 @@ struct Traversal {
     // and an interior root is expanded next without a second test.  (The
     // counting traversal leaves the TLAS root to step(), which tests and
     // counts it.)
-    __device__ __forceinline__ void take_tlas_root() { take_root(G.tlas, false); }
-    __device__ __forceinline__ void take_root(const float4* base, bool in_blas) {
-        const float4 a = base[0], b = base[1];
+    __device__ __forceinline__ void take_tlas_root() { take_root(G.tlas, 0, false); }
+    __device__ __forceinline__ void take_root(const float4* nodes, int root, bool in_blas) {
+        const float4 a = node_half(nodes, root, 0), b = node_half(nodes, root, 1);
         nxt = kNoNode;
         if (!box(mk(a.x, a.y, a.z), mk(a.w, b.x, b.y))) return;
         const uint32_t f = __float_as_uint(b.w);
         if (f & 0xff) {
             const int cnt = (int)(int8_t)((f >> 16) & 0xff);
             const int w = __float_as_int(b.z);
-            if (in_blas) { bl_cur = tri_base + w; bl_end = bl_cur + cnt; }
+            if (in_blas) { bl_cur = w; bl_end = w + cnt; }
             else { tl_cur = w; tl_end = w + cnt; }
         } else {
-            nxt = 0u;
+            nxt = (uint32_t)root;
         }
     }
     // An idle lane: no item left anywhere, so next_kind() reports kItemNone
@@ -254,7 +271,7 @@ struct Traversal {
             const float4 a = G.insts[idx].lo, b = G.insts[idx].hi;
             lo = xyz(a); hi = xyz(b);
         } else {
-            n = load_node(kind == kItemTNode ? G.tlas : G.blas + 2 * (size_t)blas_root, idx);
+            n = load_node(kind == kItemTNode ? G.tlas : G.blas, idx);
             lo = n.lo; hi = n.hi;
             if (COUNT) cnt.nodes++;
         }
@@ -265,7 +282,7 @@ struct Traversal {
                 if (ANY) { found = true; return false; }
                 t = tt;
                 hit_inst = cur_inst;
-                hit_prim = idx - tri_base;
+                hit_prim = idx;
             }
         } else if (kind == kItemInst) {
             if (COUNT) cnt.insts++;
@@ -287,14 +304,12 @@ struct Traversal {
                 cinv = {1.0f / od.x, 1.0f / od.y, 1.0f / od.z};
                 exact = exact || !finite3(co) || !finite3(cinv);
                 cur_inst = idx;
-                blas_root = info.x;
-                tri_base = info.y;
                 blas_base = st.sp;
-                nxt = kNeedTest;         // the BLAS root
+                nxt = (uint32_t)info.x | kNeedTest;   // the BLAS root
             }
         } else if (n.leaf) {
             if (kind == kItemTNode) { tl_cur = n.word; tl_end = n.word + n.count; }
-            else { bl_cur = tri_base + n.word; bl_end = bl_cur + n.count; }
+            else { bl_cur = n.word; bl_end = bl_cur + n.count; }
         } else if (comp(cd, n.axis) > 0.0f) {
             st.push((uint32_t)n.word); st.push((uint32_t)(idx + 1));
         } else {
@@ -339,14 +354,14 @@ struct Traversal {
     // One triangle of the current BLAS leaf.  Returns false on an any-hit.
     __device__ __forceinline__ bool do_tri(bool any, bool& found) {
         const int idx = bl_cur++;
-        const Tri tr = load_tri(G.tris, idx);
+        const Tri tr = FLAT ? load_tri32(G.tris, idx) : load_tri(G.tris, idx);
         if (!box_tri(tr)) return true;
         float tt;
         if (tri_hit(tr, co, cd, t, tt)) {
             if (any) { found = true; return false; }
             t = tt;
             hit_inst = cur_inst;
-            hit_prim = idx - tri_base;
+            hit_prim = idx;
         }
         return true;
     }
@@ -358,7 +373,7 @@ struct Traversal {
         if (FLAT) {
             idx = __ffs((int)left) - 1;
             left &= left - 1;
-            if (!any) idx = (int)G.flat->order[octant_shift() >> 3][idx];
+            if (!any) idx = order[(octant_shift() << 2) + idx];
         } else {
             idx = tl_cur++;
         }
@@ -386,11 +401,9 @@ struct Traversal {
             cd = wd;
             cinv = winv;
             cur_inst = idx;
-            blas_root = info.x;
-            tri_base = info.y;
             if (!FLAT) blas_base = st.sp;
             if (aux.y >= 0) { bl_cur = aux.y; bl_end = aux.z; }
-            else nxt = 0u;
+            else nxt = (uint32_t)info.x;
             return true;
         }
         const Xf w2o = I.w2o;
@@ -419,10 +432,8 @@ struct Traversal {
     // step.
     __device__ __forceinline__ void enter_blas(int idx, int4 info) {
         cur_inst = idx;
-        blas_root = info.x;
-        tri_base = info.y;
         if (!FLAT) blas_base = st.sp;
-        take_root(G.blas + 2 * (size_t)info.x, true);
+        take_root(G.blas, info.x, true);
     }
 
     // One item of the fast traversal (all lanes of a wave advance together,
@@ -446,20 +457,21 @@ struct Traversal {
         if (nxt != kNoNode) { e = nxt; nxt = kNoNode; }
         else e = st.pop();
         const bool in_blas = FLAT || blas_base >= 0;
-        const float4* base = in_blas ? G.blas + 2 * (size_t)blas_root : G.tlas;
+        const float4* base = in_blas ? G.blas : G.tlas;
         const int node = (int)e;
-        const float4 b = base[2 * node + 1];
+        const float4 b = node_half(base, node, 1);
         const int word = __float_as_int(b.z);
         const uint32_t f = __float_as_uint(b.w);
         if (f & 0xff) {
             const int count = (int)(int8_t)((f >> 16) & 0xff);
             if (!in_blas) { tl_cur = word; tl_end = word + count; }
-            else { bl_cur = tri_base + word; bl_end = bl_cur + count; }
+            else { bl_cur = word; bl_end = word + count; }
             return;
         }
         const int axis = (int)(int8_t)((f >> 8) & 0xff);
         const int l = node + 1, r = word;
-        const float4 la = base[2 * l], lb = base[2 * l + 1], ra = base[2 * r], rb = base[2 * r + 1];
+        const float4 la = node_half(base, l, 0), lb = node_half(base, l, 1);
+        const float4 ra = node_half(base, r, 0), rb = node_half(base, r, 1);
         const bool hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
         const bool hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));
         const bool left_near = comp(cd, axis) > 0.0f;
@@ -476,7 +488,7 @@ struct Traversal {
                 const int cnt = (int)(int8_t)((tf >> 16) & 0xff);
                 const int w = __float_as_int(tb.z);
                 if (!in_blas) { tl_cur = w; tl_end = w + cnt; }
-                else { bl_cur = tri_base + w; bl_end = bl_cur + cnt; }
+                else { bl_cur = w; bl_end = w + cnt; }
             } else {
                 nxt = (uint32_t)(take_left ? l : r);
             }
