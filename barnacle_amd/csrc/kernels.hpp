@@ -18,16 +18,12 @@ constexpr int kSegStride = 64;    // words between two fetch counters (own cache
 
 constexpr uint32_t kNoPath = 0xffffffffu;
 
-// Waves per SIMD the 16-entry-window trace kernels are built for: seven for
-// one scene (72 VGPRs), six in batches, whose per-lane scene pointers need
-// the 80 VGPRs of six waves to avoid spilling, and eight for scenes of few
-// instances (64 VGPRs, two spilled outside the step; with the 66 of seven waves
-// a config-1 frame takes 84.0 ms, not 81.9, and the frame of spheres 8.55, not
-// 8.23: the traversals of two streams share the SIMDs, so the blocks of one
-// kernel, seven per CU, do not say how many waves there are).
-constexpr int kTraceWaves = 7;
-constexpr int kTraceWavesFlat = 8;
-constexpr int kTraceWavesBatch = 6;
+// Waves per SIMD the 16-entry-window trace kernels are built for (64 VGPRs, 72
+// in batches, whose lanes hold their scene's pointers; no spills).  The blocks
+// of one kernel, seven per CU by default, do not say how many waves there are:
+// the traversals of two streams share the SIMDs.
+constexpr int kTraceWaves = 8;
+constexpr int kTraceWavesBatch = 7;
 
 // Path state, struct of arrays indexed by slot.
 struct PathBuf {

@@ -411,10 +411,10 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
                 }
             }
         }
-        if (__ballot(active) == 0) {
-            if (!more) break;
-            continue;
-        }
+        // (no `continue` for a wave that waits for more rays: a second way
+        // round the loop costs a second set of state registers, 23 of them
+        // spilled)
+        if (!more && __ballot(active) == 0) break;
         // Every lane steps: an idle lane's cleared state has no item, so its
         // step does nothing (and keeps the loop free of a per-lane branch).
         bool found = false;
@@ -434,11 +434,10 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
 // material bin of the hit (kind of the instance's material; light-only
 // instances in the last bin, -1 for a miss) travels in the hit record.  The
 // rays are queue[i], or position i of a compact round (queue null).
-// With a 16-entry LDS stack window seven blocks fit a CU's LDS; the register
-// budget is then set for seven waves per SIMD (72 VGPRs; eight would spill),
-// six in batches.
+// Eight blocks' 16-entry LDS stack windows fit a CU; the register budget is set
+// for eight waves per SIMD, seven in batches.
 template <bool COUNT, bool BATCH, int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_trace_closest(Work<BATCH> W, PathBuf P, Ctl* ctl, int cur,
+__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_closest(Work<BATCH> W, PathBuf P, Ctl* ctl, int cur,
                                                        const uint32_t* queue, uint32_t* spill, size_t spill_stride,
                                                        uint32_t refill, unsigned long long* stats, uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
@@ -863,7 +862,7 @@ __global__ __launch_bounds__(256, 3) void k_shade_c(Work<BATCH> W, PathBuf X, Pa
 // rays of the slots in shq, added to the slot's L.  Compact rounds (shq
 // null): ray i, added to L_out[path id] (nee_a.w).
 template <bool COUNT, bool BATCH, int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_trace_shadow(Work<BATCH> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
+__global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_shadow(Work<BATCH> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                       float4* L_out, int par,
                                                       uint32_t* spill, size_t spill_stride, uint32_t refill,
                                                       unsigned long long* stats, uint32_t* seg) {
@@ -1121,7 +1120,7 @@ __global__ __launch_bounds__(LDS ? kGradLdsThreads : 256) void k_shade_adj(
 // nee_a.w): gradient sums belong in a kernel whose lanes are all busy, not in
 // the traversal loop.
 template <int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? (FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_trace_shadow_vis(Work<false> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
+__global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_trace_shadow_vis(Work<false> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                           uint32_t* spill, size_t spill_stride, uint32_t refill,
                                                           uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
@@ -1343,7 +1342,7 @@ __global__ void k_shade_direct(Work<false> W, PathBuf P, Ctl* ctl, const uint32_
 
 // First hit of one sample per pixel: (instance, primitive, t) in pixel order.
 template <int K, bool FLAT>
-__global__ __launch_bounds__(256, K == 16 ? (FLAT ? kTraceWavesFlat : kTraceWaves) : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
+__global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
                                                    int frame_id, int* out_inst, int* out_prim, float* out_t,
                                                    uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs) {
     __shared__ uint32_t stk[K * 256];

@@ -5,17 +5,16 @@
 // MeshPrimitive.Intersect (Extensions/Primitive/Mesh.fs:188-242): the same
 // items are visited in the same order with the same current t, so hit
 // (instance, triangle, t) and the traversal counters are identical to the
-// reference's.  The schedule differs: every loop iteration processes exactly
-// one item per lane, and an item is one of
+// reference's.  The schedule differs: in every loop iteration a lane processes
+// at most one item of each sort that it comes to,
 //
-//    TLAS node | BLAS node | triangle of a BLAS leaf | instance of a TLAS leaf
+//    instance of a TLAS leaf, then TLAS or BLAS node, then triangle of a leaf
 //
-// all of which start with the same slab test (node bounds, triangle bounds,
-// instance world bounds), so a wave executes one shared slab test per
-// iteration instead of serialising whole leaves.  Lanes whose ray finished are
-// refilled from the work queue in batches (one atomic per wave).
+// (the counting traversal: one item), and lanes whose ray finished are refilled
+// from the work queue in batches (one atomic per wave).
 #pragma once
 #include "device.hpp"
+#include "wave.hpp"
 
 namespace bnd {
 
@@ -202,8 +201,7 @@ struct Traversal {
             nxt = (uint32_t)root;
         }
     }
-    // An idle lane: no item left anywhere, so next_kind() reports kItemNone
-    // and a step does nothing.
+    // An idle lane: no item left anywhere, so a step does nothing.
     __device__ __forceinline__ void clear() {
         st.sp = 0;
         nxt = kNoNode;
@@ -329,46 +327,22 @@ struct Traversal {
     // world bounds); a box that passes with the current t passed with the
     // larger one too.  Every triangle the reference tests is tested, in the
     // same order, so ties resolve alike.
-    // What this lane does next (leaving a finished BLAS first): kItemTri,
-    // kItemInst, kItemTNode (any node), or kItemNone when it has finished.
-    __device__ __forceinline__ int next_kind() {
-        if (FLAT) {
-            // the ray of a finished BLAS is simply not used any more
-            if (bl_cur < bl_end) return kItemTri;
-            if (nxt != kNoNode || st.sp > 0) return kItemTNode;
-            return left ? kItemInst : kItemNone;
-        }
-        // Selects rather than a branch: the ray registers are then updated in
-        // place instead of through copies at the join.
-        const bool leave = blas_base >= 0 && bl_cur >= bl_end && nxt == kNoNode && st.sp == blas_base;
-        blas_base = leave ? -1 : blas_base;
-        co = sel(leave, wo, co);
-        cd = sel(leave, wd, cd);
-        cinv = sel(leave, winv, cinv);
-        if (blas_base >= 0 && bl_cur < bl_end) return kItemTri;
-        if (blas_base < 0 && tl_cur < tl_end) return kItemInst;
-        if (nxt != kNoNode || st.sp > (blas_base >= 0 ? blas_base : 0)) return kItemTNode;
-        return kItemNone;
-    }
-
-    // One triangle of the current BLAS leaf.  Returns false on an any-hit.
-    __device__ __forceinline__ bool do_tri(bool any, bool& found) {
+    // One triangle of the current BLAS leaf.
+    __device__ __forceinline__ void do_tri(bool any, bool& found) {
         const int idx = bl_cur++;
         const Tri tr = FLAT ? load_tri32(G.tris, idx) : load_tri(G.tris, idx);
-        if (!box_tri(tr)) return true;
-        float tt;
-        if (tri_hit(tr, co, cd, t, tt)) {
-            if (any) { found = true; return false; }
-            t = tt;
-            hit_inst = cur_inst;
-            hit_prim = idx;
+        if (box_tri(tr)) {
+            float tt;
+            if (tri_hit(tr, co, cd, t, tt)) {
+                if (any) found = true;
+                else { t = tt; hit_inst = cur_inst; hit_prim = idx; }
+            }
         }
-        return true;
     }
 
-    // One instance of the current TLAS leaf: a sphere is intersected, a mesh
-    // BLAS is entered.  Returns false on an any-hit.
-    __device__ __forceinline__ bool do_inst(bool any, bool& found) {
+    // One instance of the current TLAS leaf (FLAT: the next of the ray's): a
+    // sphere is intersected, a mesh BLAS is entered.
+    __device__ __forceinline__ void do_inst(bool any, bool& found) {
         int idx;
         if (FLAT) {
             idx = __ffs((int)left) - 1;
@@ -378,121 +352,132 @@ struct Traversal {
             idx = tl_cur++;
         }
         const DevInst& I = G.insts[idx];
+        bool in;
         if (FLAT) {
-            bool r = slab_fast(xyz(I.lo), xyz(I.hi), wo, winv, t);
-            if (exact) r = slab(xyz(I.lo), xyz(I.hi), wo, winv, t);
-            if (!r) return true;
-        } else if (!box(xyz(I.lo), xyz(I.hi))) {
-            return true;
+            in = slab_fast(xyz(I.lo), xyz(I.hi), wo, winv, t);
+            if (exact) in = slab(xyz(I.lo), xyz(I.hi), wo, winv, t);
+        } else {
+            in = box(xyz(I.lo), xyz(I.hi));
         }
+        if (!in) return;
         const int4 info = I.info;
         const int4 aux = I.aux;
-        if (info.x >= 0 && aux.x != 0 && !exact) {
-            // Identity world-to-object map on a finite ray: Transform gives o
-            // but for the signs of zeros and d unchanged (no component of d
-            // is 0 when 1/d is finite), so the object ray's 1/d is the world
-            // one.  The sign of a zero coordinate changes no test: it is
-            // subtracted from box and triangle coordinates, and no comparison
-            // sees the sign of a zero difference.  The instance's bounds are
-            // its root's, so the root is not tested again, and one that is a
-            // leaf is not even read (frame of instances 17.1 -> 16.8 ms,
-            // 2^20 Metropolis chains 123 -> 120).
+        if (!FLAT && info.x >= 0) blas_base = st.sp;
+        if (info.x >= 0) cur_inst = idx;
+        // Identity world-to-object map on a finite ray: Transform gives o but
+        // for the signs of zeros and d unchanged (no component of d is 0 when
+        // 1/d is finite), so the object ray's 1/d is the world one.  The sign
+        // of a zero coordinate changes no test: it is subtracted from box and
+        // triangle coordinates, and no comparison sees the sign of a zero
+        // difference.  The instance's bounds are its root's, so the root is
+        // not tested again, and one that is a leaf is not even read (frame of
+        // instances 17.1 -> 16.8 ms, 2^20 Metropolis chains 123 -> 120).
+        const bool same = info.x >= 0 && aux.x != 0 && !exact;
+        if (same) {
             co = wo;
             cd = wd;
             cinv = winv;
-            cur_inst = idx;
-            if (!FLAT) blas_base = st.sp;
             if (aux.y >= 0) { bl_cur = aux.y; bl_end = aux.z; }
-            else nxt = (uint32_t)info.x;
-            return true;
+            nxt = aux.y >= 0 ? kNoNode : (uint32_t)info.x;
         }
+        if (opaque(same)) return;
         const Xf w2o = I.w2o;
         const V3 oo = xf_point(w2o, wo), od = xf_dir(w2o, wd);
         if (info.x < 0) {
             float tt;
             int br;
             if (sphere_hit(I.lo.w, oo, od, t, tt, br)) {
-                if (any) { found = true; return false; }
-                t = tt;
-                hit_inst = idx;
-                hit_prim = br;
+                if (any) found = true;
+                else { t = tt; hit_inst = idx; hit_prim = br; }
             }
-        } else {
+        }
+        if (opaque(info.x) >= 0) {
+            // its root is tested at once, as the reference pops and tests it
+            // first (Mesh.fs:217-242); a lane whose root fails leaves the
+            // BLAS in its next step
             co = oo; cd = od;
             cinv = {1.0f / od.x, 1.0f / od.y, 1.0f / od.z};
             exact = exact || !finite3(co) || !finite3(cinv);
-            enter_blas(idx, info);
+            take_root(G.blas, info.x, true);
         }
-        return true;
-    }
-
-    // Entry into the BLAS of instance idx with the object ray set; its root
-    // is tested at once, as the reference pops and tests it first
-    // (Mesh.fs:217-242).  A lane whose root fails leaves the BLAS in its next
-    // step.
-    __device__ __forceinline__ void enter_blas(int idx, int4 info) {
-        cur_inst = idx;
-        if (!FLAT) blas_base = st.sp;
-        take_root(G.blas, info.x, true);
-    }
-
-    // One item of the fast traversal (all lanes of a wave advance together,
-    // whatever kind of item each has: measured faster than advancing only the
-    // lanes of the most common kind).  Returns false when the traversal has
-    // finished or an any-hit query (`any`, per lane) found its hit.
-    __device__ __forceinline__ bool step_fast(bool any, bool& found) {
-        const int kind = next_kind();
-        if (kind == kItemTri) return do_tri(any, found);
-        if (kind == kItemInst) return do_inst(any, found);
-        if (kind == kItemTNode) { do_node(); return true; }
-        return false;
     }
 
     // Expand the next node: a leaf sets its item range; an interior node
     // tests both children with the current t and keeps those that pass (the
     // near one in `nxt`, the far one on the stack, near first as in
-    // Extensions/Aggregate/BVH.fs:47-56 and Mesh.fs:233-240).
+    // Extensions/Aggregate/BVH.fs:47-56 and Mesh.fs:233-240).  A child taken
+    // next that is a leaf hands over its items at once (same items, same
+    // order), without being popped first.
     __device__ __forceinline__ void do_node() {
-        uint32_t e;
-        if (nxt != kNoNode) { e = nxt; nxt = kNoNode; }
-        else e = st.pop();
+        uint32_t e = nxt;
+        if (e == kNoNode) e = st.pop();
+        nxt = kNoNode;
         const bool in_blas = FLAT || blas_base >= 0;
         const float4* base = in_blas ? G.blas : G.tlas;
         const int node = (int)e;
         const float4 b = node_half(base, node, 1);
-        const int word = __float_as_int(b.z);
-        const uint32_t f = __float_as_uint(b.w);
-        if (f & 0xff) {
-            const int count = (int)(int8_t)((f >> 16) & 0xff);
-            if (!in_blas) { tl_cur = word; tl_end = word + count; }
-            else { bl_cur = word; bl_end = word + count; }
-            return;
+        int word = __float_as_int(b.z);
+        uint32_t f = __float_as_uint(b.w);
+        bool leaf = (f & 0xff) != 0;
+        if (!leaf) {
+            const int axis = (int)(int8_t)((f >> 8) & 0xff);
+            const int l = node + 1, r = word;
+            const float4 la = node_half(base, l, 0), lb = node_half(base, l, 1);
+            const float4 ra = node_half(base, r, 0), rb = node_half(base, r, 1);
+            const bool hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
+            const bool hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));
+            const bool left_near = comp(cd, axis) > 0.0f;
+            if (hl && hr) st.push((uint32_t)(left_near ? r : l));
+            const bool take_left = hl && (left_near || !hr);
+            f = __float_as_uint(take_left ? lb.w : rb.w);
+            word = __float_as_int(take_left ? lb.z : rb.z);
+            const bool any_child = hl || hr;
+            leaf = any_child && (f & 0xff) != 0;
+            if (any_child && !leaf) nxt = (uint32_t)(take_left ? l : r);
         }
-        const int axis = (int)(int8_t)((f >> 8) & 0xff);
-        const int l = node + 1, r = word;
-        const float4 la = node_half(base, l, 0), lb = node_half(base, l, 1);
-        const float4 ra = node_half(base, r, 0), rb = node_half(base, r, 1);
-        const bool hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
-        const bool hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));
-        const bool left_near = comp(cd, axis) > 0.0f;
-        const int near = left_near ? l : r, far = left_near ? r : l;
-        const bool hn = left_near ? hl : hr, hf = left_near ? hr : hl;
-        if (hn && hf) st.push((uint32_t)far);
-        if (hn || hf) {
-            // The child taken next: a leaf hands over its items at once, which
-            // saves the step that would only pop it (same items, same order).
-            const bool take_left = hn ? left_near : !left_near;
-            const float4 tb = take_left ? lb : rb;
-            const uint32_t tf = __float_as_uint(tb.w);
-            if (tf & 0xff) {
-                const int cnt = (int)(int8_t)((tf >> 16) & 0xff);
-                const int w = __float_as_int(tb.z);
-                if (!in_blas) { tl_cur = w; tl_end = w + cnt; }
-                else { bl_cur = w; bl_end = w + cnt; }
-            } else {
-                nxt = (uint32_t)(take_left ? l : r);
-            }
+        if (leaf) {
+            const int end = word + (int)(int8_t)((f >> 16) & 0xff);
+            if (in_blas) { bl_cur = word; bl_end = end; }
+            if (!in_blas) { tl_cur = word; tl_end = end; }
         }
+    }
+
+    // One step of the fast traversal: an instance, then a node, then a
+    // triangle, each if it is what the lane has next at that moment, so one
+    // step can take a lane from an instance through its root to the first
+    // triangle of a leaf (each lane's items in its own order).  Returns false
+    // when the traversal has finished or an any-hit query (`any`, per lane)
+    // found its hit.
+    //
+    // The three run one behind the other, each updating the lane's state in
+    // place under the mask of its lanes.  As branches of one choice they cost
+    // two copies of the state: the compiler lets the branches write a second
+    // set of registers, which lanes of the other branches fill by moves (14
+    // for each branch and 18 at the end of a step, of about 330 instructions).
+    // Config-1 frame 82.0 -> 77.1 ms, preview 1.18 -> 1.03, adjoint step
+    // 51.6 -> 45.6 ms; 64 VGPRs hold both kinds of scene.
+    __device__ __forceinline__ bool step_fast(bool any, bool& found) {
+        if (!FLAT) {
+            // leave a finished BLAS; selects, so that the ray's registers are
+            // updated in place
+            const bool leave = blas_base >= 0 && bl_cur >= bl_end && nxt == kNoNode && st.sp == blas_base;
+            blas_base = leave ? -1 : blas_base;
+            co = sel(leave, wo, co);
+            cd = sel(leave, wd, cd);
+            cinv = sel(leave, winv, cinv);
+        }
+        if (FLAT ? left != 0 && nothing_in_blas() : blas_base < 0 && tl_cur < tl_end) do_inst(any, found);
+        if (bl_cur >= bl_end && (FLAT ? nxt != kNoNode || st.sp > 0
+                                      : (blas_base >= 0 || tl_cur >= tl_end) &&
+                                            (nxt != kNoNode || st.sp > (blas_base >= 0 ? blas_base : 0))))
+            do_node();
+        if (bl_cur < bl_end) do_tri(any, found);
+        if (FLAT) return !found && (left != 0 || !nothing_in_blas());
+        return !found && (tl_cur < tl_end || !nothing_in_blas());
+    }
+    // FLAT: also no BLAS is being traversed; otherwise the TLAS stack is empty as well.
+    __device__ __forceinline__ bool nothing_in_blas() const {
+        return bl_cur >= bl_end && nxt == kNoNode && st.sp == 0;
     }
 };
 
