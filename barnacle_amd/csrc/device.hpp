@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "trig.hpp"
+
 namespace bnd {
 
 constexpr float kPi = 3.14159265358979323846f;
@@ -19,8 +21,6 @@ constexpr float kInf = __builtin_inff();
 constexpr float kEps = 1.40129846e-45f;   // Single.Epsilon
 
 // ---------------------------------------------------------------- scalars
-__device__ __forceinline__ float sin_f(float x) { return (float)::sin((double)x); }
-__device__ __forceinline__ float cos_f(float x) { return (float)::cos((double)x); }
 __device__ __forceinline__ float atan_f(float x) { return (float)::atan((double)x); }
 __device__ __forceinline__ float log_f(float x) { return (float)::log((double)x); }
 __device__ __forceinline__ float exp_f(float x) { return (float)::exp((double)x); }

@@ -98,10 +98,12 @@ __device__ __forceinline__ BSDF mat_eval(const Mat& m, V3 wo, V3 wi) {
     return {{0, 0, 0}, 0.0f};                                             // Mirror.fs:11, Dielectric.fs:13
 }
 __device__ __forceinline__ BSDF mat_sample(const Mat& m, V3 wo, float ul, V2 u, V3& wi) {
+    // the azimuth of a Lambertian and of either PBR sample, for all lanes of a
+    // wave that hold one of the three
+    float sp = 0.0f, cp = 0.0f;
+    if (m.kind == 0 || m.kind == 3) sincos_f(2.0f * kPi * u.y, sp, cp);
     if (m.kind == 0) {                                                    // Lambertian.fs:18-26
         float ct = sqrtf(u.x), st = sqrtf(1.0f - u.x);
-        float ph = 2.0f * kPi * u.y;
-        float sp = sin_f(ph), cp = cos_f(ph);
         V3 w = {st * cp, st * sp, ct};
         float pdf = w.z / kPi;
         wi = wo.z > 0.0f ? w : -w;
@@ -128,14 +130,12 @@ __device__ __forceinline__ BSDF mat_sample(const Mat& m, V3 wo, float ul, V2 u, 
     // PBR.fs:50-64
     if (ul < 1.0f - 0.5f * (1.0f - m.metallic)) {
         float th = atan_f(m.alpha * sqrtf(u.x / (1.0f - u.x)));
-        float ph = 2.0f * kPi * u.y;
-        float st = sin_f(th), ct = cos_f(th), sp = sin_f(ph), cp = cos_f(ph);
+        float st, ct;
+        sincos_f(th, st, ct);
         V3 wh = {st * cp, st * sp, ct};
         wi = 2.0f * dot(wo, wh) * wh - wo;
     } else {
         float ct = sqrtf(u.x), st = sqrtf(1.0f - u.x);
-        float ph = 2.0f * kPi * u.y;
-        float sp = sin_f(ph), cp = cos_f(ph);
         wi = {st * cp, st * sp, ct};
     }
     return pbr_eval(m, wo, wi);
@@ -241,7 +241,8 @@ __device__ __forceinline__ LightSample light_sample(const DevScene& S, V3 p, flo
     if (I.info.x < 0) {
         const float radius = I.lo.w;
         float a = 2.0f * kPi * u.x;
-        float st = sin_f(a), ct = cos_f(a);
+        float st, ct;
+        sincos_f(a, st, ct);
         float cp = fmaf(-2.0f, u.y, 1.0f);
         float sp = sqrtf(fmaf(-cp, cp, 1.0f));
         V3 nn = {ct * sp, st * sp, cp};
@@ -319,14 +320,13 @@ __device__ __forceinline__ Ray camera_ray(const DevScene& S, int x, int y, V2 uP
     if (S.cam_kind == 1 && aperture > 0.0f) {
         V2 u = {uLens.x * 2.0f - 1.0f, uLens.y * 2.0f - 1.0f};
         V2 d = {0.0f, 0.0f};
-        if (u.x == 0.0f || u.y == 0.0f) {
-            d = {0.0f, 0.0f};
-        } else if (fabsf(u.x) > fabsf(u.y)) {
-            float rr = u.x, th = kPi / 4.0f * (u.y / u.x);
-            d = {rr * cos_f(th), rr * sin_f(th)};
-        } else {
-            float rr = u.y, th = kPi / 2.0f - kPi / 4.0f * (u.x / u.y);
-            d = {rr * cos_f(th), rr * sin_f(th)};
+        if (u.x != 0.0f && u.y != 0.0f) {
+            const bool wide = fabsf(u.x) > fabsf(u.y);
+            const float rr = wide ? u.x : u.y;
+            const float th = wide ? kPi / 4.0f * (u.y / u.x) : kPi / 2.0f - kPi / 4.0f * (u.x / u.y);
+            float st, ct;
+            sincos_f(th, st, ct);
+            d = {rr * ct, rr * st};
         }
         V3 o = r.o + mk(aperture * d.x, aperture * d.y, 0.0f);
         V3 dir = normalize(point_at(r, S.dv.w) - o);
