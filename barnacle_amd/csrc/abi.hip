@@ -798,7 +798,8 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
                           std::to_string(B.stack_k) + ":" + std::to_string(L.n_slots) + ":" +
                           std::to_string((uintptr_t)c->b_items.p) + ":" + std::to_string((uintptr_t)c->b_scenes.p) +
                           ":" + std::to_string((uintptr_t)c->L_out.p) + ":" + std::to_string((int)L.octant_order) + ":" + std::to_string(L.skip_dark) +
-                          ":" + std::to_string(whole ? n : 0) + ":" + std::to_string(Lr.stream2 != nullptr);
+                          ":" + std::to_string(whole ? n : 0) + ":" + std::to_string(Lr.stream2 != nullptr) + ":" +
+                          std::to_string(Lr.list);
         if (Lr.uniform) {
             const bnd::DevScene& d = Lr.scene;
             for (const void* q : {(const void*)d.tlas, (const void*)d.flat, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
@@ -872,11 +873,13 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
         }
         int path = 0, pix = 0, round_depth = 0;
         L.uniform = true;
+        L.list = true;
         int k0 = -1;
         for (int k = 0; k < n; ++k) {
             if (take[k] == 0) continue;
             if (k0 < 0) k0 = k;
             L.uniform = L.uniform && items[k].scene == items[k0].scene;
+            L.list = L.list && scenes[k].flat != nullptr;
             bnd::RoundItem it = base[k];
             it.s0 = next[k];
             it.ns = take[k];

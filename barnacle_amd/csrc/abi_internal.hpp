@@ -118,9 +118,10 @@ struct Ctx {
     size_t mlt_cap = 0;
     int mlt_nx = 0;
     size_t mlt_chunk = (size_t)1 << 20;   // chains (or bootstrap paths) in flight
-    // Up to so many chains, one wave per chain runs its mutations (16384
-    // chains: 37 ms against 51 ms of wavefronts; 32768: 66 against 58).
-    int mlt_wave_chains = 20480;
+    // Up to so many chains, one wave per chain runs its mutations (60 mutations
+    // of 24576 chains: 52 to 56 ms against 62 to 66 of wavefronts; 32768: 71 to
+    // 74 against 67 to 71; 65536: 150 against 84).
+    int mlt_wave_chains = 28672;
     DevBuf m_inner, m_outer, m_state, m_bid, m_pix_new, m_pix_cur, m_Lcur, m_rad, m_acc, m_xs;
     DevBuf m_weights, m_aprob, m_aidx, m_accepted_out;
     // GPU BVH builder (bvh_gpu.hip): items (two buffers, then the output

@@ -19,7 +19,8 @@ constexpr int kSegStride = 64;    // words between two fetch counters (own cache
 constexpr uint32_t kNoPath = 0xffffffffu;
 
 // Waves per SIMD the 16-entry-window trace kernels are built for (64 VGPRs, 72
-// in batches, whose lanes hold their scene's pointers; no spills).  The blocks
+// in batches, whose lanes hold their scene's pointers; no spills: with eight
+// spilled for eight waves, 48 thumbnails take 5.64 ms, not 5.42).  The blocks
 // of one kernel, seven per CU by default, do not say how many waves there are:
 // the traversals of two streams share the SIMDs.
 constexpr int kTraceWaves = 8;
@@ -100,6 +101,7 @@ struct Launch {
     // its compact rounds launch the single-scene trace kernels (the scene
     // bound once per launch) on grid_uniform blocks.
     bool uniform;
+    bool list;                // batch mode: every scene of the round has a DevScene::flat
     int grid_uniform;
     uint32_t refill;
     hipStream_t stream;

@@ -508,21 +508,28 @@ constexpr int kMltWaveK = 16;
 // WAVES per SIMD: alone on its SIMD a wave may use every register; where there
 // are more chains than SIMDs four waves share one, at 128 VGPRs, with spills
 // (1024 chains: 63.5 ms alone, 67.9 ms with four; 16384: 47.1 and 36.6 ms).
-template <int WAVES>
+template <int WAVES, bool FLAT>
 __global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBuf M, MltParamsDev p, float* film,
                                                            uint32_t* spill, size_t spill_stride, int n,
                                                            int mutations, int nx, int max_depth, int rr_depth) {
     extern __shared__ float4 xs[];
     __shared__ uint32_t stk[kMltWaveK * 64];
     const int lane = (int)lane_id();
-    Traversal<kMltWaveK, false, 64> tr;
+    Traversal<kMltWaveK, FLAT, 64> tr;
     tr.st = LaneStack<kMltWaveK, 64>{stk + lane, spill, (uint32_t)spill_stride, blockIdx.x * 64u + (uint32_t)lane, 0};
     tr.clear();
     tr.G.set(S);
+    __shared__ uint8_t order[FLAT ? sizeof(FlatScene::order) : 1];
+    if (FLAT) {
+        for (int k = lane; k < (int)sizeof order; k += 64) order[k] = S.flat->order[k / kFlatMax][k % kFlatMax];
+        tr.order = order;
+        wave_sync();
+    }
     // a whole traversal of one ray, the same in every lane
     auto trace = [&](const Ray& r, float tmax, bool any) {
         tr.start(r, tmax, S.exact_only != 0);
-        tr.take_tlas_root();
+        if (FLAT) tr.take_instances_wave(any);
+        else tr.take_tlas_root();
         if (!(tmax == tmax)) tr.empty();
         bool found = false;
         while (tr.step_fast(any, found)) {}
@@ -661,12 +668,10 @@ void launch_mlt_wave_chains(const DevScene& S, const MltBuf& M, const MltParamsD
                             hipStream_t st) {
     const int nx = 4 + 7 * max_depth;
     const size_t lds = (size_t)nx * sizeof(float4);
-    if (n <= n_simd)
-        hipLaunchKernelGGL(k_mlt_wave_chains<1>, dim3(min(n, grid)), dim3(64), lds, st, S, M, p, film, B.spill,
-                           B.spill_stride, n, mutations, nx, max_depth, rr_depth);
-    else
-        hipLaunchKernelGGL(k_mlt_wave_chains<4>, dim3(min(n, grid)), dim3(64), lds, st, S, M, p, film, B.spill,
-                           B.spill_stride, n, mutations, nx, max_depth, rr_depth);
+    auto* run = n <= n_simd ? (S.flat ? k_mlt_wave_chains<1, true> : k_mlt_wave_chains<1, false>)
+                            : (S.flat ? k_mlt_wave_chains<4, true> : k_mlt_wave_chains<4, false>);
+    hipLaunchKernelGGL(run, dim3(min(n, grid)), dim3(64), lds, st, S, M, p, film, B.spill, B.spill_stride, n, mutations,
+                       nx, max_depth, rr_depth);
 }
 
 }  // namespace bnd

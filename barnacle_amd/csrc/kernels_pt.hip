@@ -81,7 +81,8 @@ struct Work<true> {
     const RoundHeader* hdr;
     const RoundItem* items;
     const DevScene* scenes;
-    bool flat() const { return false; }
+    bool list;                // every scene of the round has a DevScene::flat
+    bool flat() const { return list; }
     __device__ __forceinline__ int n() const { return hdr->n_items; }
     // item owning a path id (the round table is ordered by path_base)
     __device__ __forceinline__ int item_of_path(uint32_t id) const {
@@ -351,7 +352,7 @@ __device__ __forceinline__ int next_segment(const SegFetch& F, uint32_t pick, ui
     return -1;
 }
 
-template <bool ANY, bool COUNT, int K, bool FLAT, typename Setup, typename Init, typename Done>
+template <bool ANY, bool COUNT, bool BATCH, int K, bool FLAT, typename Setup, typename Init, typename Done>
 __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uint32_t* stk, uint32_t* spill,
                                                  size_t spill_stride, uint32_t refill, TraceCount& tc, Setup setup,
                                                  Init init, Done done) {
@@ -360,8 +361,8 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
     tr.st = LaneStack<K, 256>{stk + threadIdx.x, spill, (uint32_t)spill_stride, gid, 0};
     tr.clear();
     setup(tr);
-    __shared__ uint8_t order[FLAT ? sizeof(FlatScene::order) : 1];
-    if (FLAT) {
+    __shared__ uint8_t order[FLAT && !BATCH ? sizeof(FlatScene::order) : 1];
+    if (FLAT && !BATCH) {
         static_assert(sizeof(FlatScene::order) == 256, "a byte for each thread");
         order[threadIdx.x] = tr.G.flat->order[threadIdx.x / kFlatMax][threadIdx.x % kFlatMax];
         tr.order = order;
@@ -448,7 +449,7 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
         else ctl->q_count[1 - cur] = 0;
     }
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, COUNT, K, FLAT>(
+    persistent_trace<false, COUNT, BATCH, K, FLAT>(
         SegFetch{seg, kFetchSegs}, count, stk, spill, spill_stride, refill, tc,
         [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
         [&](Traversal<K, FLAT>& tr, uint32_t i) {
@@ -457,7 +458,8 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
             const int k = W.item_of(P, slot);
             W.bind_lane(tr.G, k);
             tr.start({xyz(o4), xyz(P.d[slot])}, kInf, W.scene(k).exact_only != 0);
-            if (FLAT) tr.take_instances(false);
+            if (FLAT && BATCH) tr.order = tr.G.flat->order[0];
+            if (FLAT) tr.template take_instances<BATCH>(false);
             else if (!COUNT) tr.take_tlas_root();
             // a placeholder path (padding pixel, max-depth 0) misses at once
             if (__float_as_int(o4.w) < 0) tr.empty();
@@ -869,7 +871,7 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = shq && par < 0 ? ctl->sh_count : ctl->shc[par];
     TraceCount tc{0, 0, 0};
-    persistent_trace<true, COUNT, K, FLAT>(
+    persistent_trace<true, COUNT, BATCH, K, FLAT>(
         SegFetch{seg, kShadowSegs}, count, stk, spill, spill_stride, refill, tc,
         [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
         [&](Traversal<K, FLAT>& tr, uint32_t i) {
@@ -878,7 +880,8 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
             const int k = shq ? W.item_of(P, slot) : (BATCH ? __float_as_int(d4.w) : 0);
             W.bind_lane(tr.G, k);
             tr.start({xyz(o4), xyz(d4)}, o4.w, W.scene(k).exact_only != 0);
-            if (FLAT) tr.take_instances(true);
+            if (FLAT && BATCH) tr.order = tr.G.flat->order[0];
+            if (FLAT) tr.template take_instances<BATCH>(true);
             else if (!COUNT) tr.take_tlas_root();
             // a NaN t max fails every slab test of the reference: empty traversal
             if (!(o4.w == o4.w)) tr.empty();
@@ -1126,14 +1129,14 @@ __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_trace_shadow
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = ctl->sh_count;
     TraceCount tc{0, 0, 0};
-    persistent_trace<true, false, K, FLAT>(
+    persistent_trace<true, false, false, K, FLAT>(
         SegFetch{seg, kShadowSegs}, count, stk, spill, spill_stride, refill, tc,
         [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
         [&](Traversal<K, FLAT>& tr, uint32_t i) {
             const uint32_t slot = shq[i];
             const float4 o4 = P.sh_o[slot];
             tr.start({xyz(o4), xyz(P.sh_d[slot])}, o4.w, W.S.exact_only != 0);
-            if (FLAT) tr.take_instances(true);
+            if (FLAT) tr.template take_instances<false>(true);
             else tr.take_tlas_root();
             if (!(o4.w == o4.w)) tr.empty();
         },
@@ -1348,7 +1351,7 @@ __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(De
     __shared__ uint32_t stk[K * 256];
     const uint32_t n = (uint32_t)width * (uint32_t)height;
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, false, K, FLAT>(
+    persistent_trace<false, false, false, K, FLAT>(
         SegFetch{fetch, segs}, n, stk, spill, spill_stride, 16u, tc,
         [&](Traversal<K, FLAT>& tr) { tr.G.set(S); },
         [&](Traversal<K, FLAT>& tr, uint32_t p) {
@@ -1358,7 +1361,7 @@ __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(De
             uPix.x = lcg(rng); uPix.y = lcg(rng);
             uLens.x = lcg(rng); uLens.y = lcg(rng);
             tr.start(camera_ray(S, x, y, uPix, uLens), kInf, S.exact_only != 0);
-            if (FLAT) tr.take_instances(false);
+            if (FLAT) tr.template take_instances<false>(false);
             else tr.take_tlas_root();
         },
         [&](Traversal<K, FLAT>& tr, uint32_t p, bool fin, bool) {
@@ -1382,6 +1385,7 @@ static Work<true> batch_work(const Launch& L) {
     w.hdr = L.hdr;
     w.items = L.items;
     w.scenes = L.scenes;
+    w.list = L.list;
     return w;
 }
 
@@ -1393,7 +1397,7 @@ static void launch_closest_t(bool count, int k, const Work<BATCH>& W, const Path
     hipLaunchKernelGGL((k_trace_closest<C, BATCH, KK, F>), dim3(grid), dim3(256), 0, st, W, P, ctl, cur, queue, \
                        B.spill, B.spill_stride, refill, B.stats, B.fetch_seg)
     if (count) { if (k == 16) BN_TC(true, 16, false); else BN_TC(true, 32, false); }
-    else if (W.flat()) { if (k == 16) BN_TC(false, 16, !BATCH); else BN_TC(false, 32, !BATCH); }
+    else if (W.flat()) { if (k == 16) BN_TC(false, 16, true); else BN_TC(false, 32, true); }
     else { if (k == 16) BN_TC(false, 16, false); else BN_TC(false, 32, false); }
 #undef BN_TC
 }
@@ -1409,7 +1413,7 @@ static void launch_shadow_t(bool count, int k, const Work<BATCH>& W, const PathB
     hipLaunchKernelGGL((k_trace_shadow<C, BATCH, KK, F>), dim3(grid), dim3(256), 0, st, W, P, ctl, shq, L_out, par, \
                        spill, B.spill_stride, refill, B.stats, seg)
     if (count) { if (k == 16) BN_TS(true, 16, false); else BN_TS(true, 32, false); }
-    else if (W.flat()) { if (k == 16) BN_TS(false, 16, !BATCH); else BN_TS(false, 32, !BATCH); }
+    else if (W.flat()) { if (k == 16) BN_TS(false, 16, true); else BN_TS(false, 32, true); }
     else { if (k == 16) BN_TS(false, 16, false); else BN_TS(false, 32, false); }
 #undef BN_TS
 }

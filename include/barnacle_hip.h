@@ -378,7 +378,7 @@ int bn_render_batch(bn_ctx* ctx, const bn_batch_item* items, int32_t n, float* c
  *   "bvh_small"            largest subtree (triangles, 128..512, default 128)
  *                          that one wave of the GPU build finishes alone; more
  *                          than 256 mean 256
- *   "mlt_wave_chains"      up to so many PSSMLT chains (default 20480) one wave
+ *   "mlt_wave_chains"      up to so many PSSMLT chains (default 28672) one wave
  *                          runs each chain's mutations; more advance together
  *                          as a wavefront.  The chains are the same either way.
  *   "overlap_shadow"       1 (default): path-tracing frames trace each bounce's

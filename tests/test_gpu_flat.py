@@ -12,8 +12,9 @@ from test_gpu_upload import reupload
 pytestmark = pytest.mark.gpu
 
 
-def cubes(n, fov):
+def cubes(n, fov, integrator=None):
     info = configs.cornell_box(27, 21, 3, 5, boxes=False)
+    info["integrator"] = integrator or info["integrator"]
     info["camera"]["fov"] = fov
     eye = info["transforms"][-1]["keyframes"][0]["translation"]
     info["primitives"].append({"type": "cube"})
@@ -106,3 +107,35 @@ def test_identity_instance_with_bounds_of_its_own(ctx, change):
     assert not same(walked, built.render_pt(p))
     up.release()
     built.release()
+
+
+@pytest.mark.parametrize("sizes", [(7, 20, 32), (7, 40, 20)])
+def test_mixed_batches_equal_plain_frames(ctx, sizes):
+    """A batch round binds each ray's scene: lists where all its scenes have
+    one, else trees; the same graph key must not stand for both."""
+    ds = [ctx.scene(cubes(n, 39.3)) for n in sizes]
+    ps = [d.sc.pt_params() for d in ds]
+    for pick in ((0, 1, 2), (0, 2), (1, 0), (0, 2)):
+        for k, film in zip(pick, ctx.render_batch([(ds[k], ps[k]) for k in pick])[0]):
+            assert same(film, ds[k].render_pt(ps[k], stats=True)[0])
+    for d in ds:
+        d.release()
+
+
+@pytest.mark.parametrize("n", [20, 40])
+def test_metropolis_waves_equal_the_wavefront(ctx, n):
+    caustics = configs.caustic_scene(width=27, height=21, spp=2, max_depth=5, freq=4, n_bootstrap=512, n_chains=37)
+    sc = cubes(n, 39.3, caustics["integrator"])
+    ds = ctx.scene(sc)
+    p = sc.mlt_params()
+    out = []
+    try:
+        for waves in (0, 1 << 20):
+            ctx.set_option("mlt_wave_chains", waves)
+            film, st = ds.render_pssmlt(p)
+            out.append((st["accepted"], ds.pssmlt_last(p)[1].copy(), film))
+    finally:
+        ctx.set_option("mlt_wave_chains", 20480)
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+    assert np.allclose(out[0][2], out[1][2], rtol=1e-4, atol=1e-5, equal_nan=True)
+    ds.release()
