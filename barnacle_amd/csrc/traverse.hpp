@@ -373,7 +373,7 @@ struct Traversal {
         const DevInst& I = G.insts[idx];
         bool in;
         if (FLAT) {
-            in = slab_fast(xyz(I.lo), xyz(I.hi), wo, winv, t);
+            in = any || slab_fast(xyz(I.lo), xyz(I.hi), wo, winv, t);   // t as in take_instances
             if (exact) in = slab(xyz(I.lo), xyz(I.hi), wo, winv, t);
         } else {
             in = box(xyz(I.lo), xyz(I.hi));
@@ -427,7 +427,7 @@ struct Traversal {
     // Extensions/Aggregate/BVH.fs:47-56 and Mesh.fs:233-240).  A child taken
     // next that is a leaf hands over its items at once (same items, same
     // order), without being popped first.
-    __device__ __forceinline__ void do_node() {
+    __device__ __forceinline__ void do_node(bool any) {
         uint32_t e = nxt;
         if (e == kNoNode) e = st.pop();
         nxt = kNoNode;
@@ -445,7 +445,10 @@ struct Traversal {
             const float4 ra = node_half(base, r, 0), rb = node_half(base, r, 1);
             const bool hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
             const bool hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));
-            const bool left_near = comp(cd, axis) > 0.0f;
+            // An any-hit query finds the same in any order, and t does not
+            // change on the way: left first saves it the axis (preview 1.02
+            // -> 0.97 ms, adjoint step 44.9 -> 43.0).
+            const bool left_near = any || comp(cd, axis) > 0.0f;
             if (hl && hr) st.push((uint32_t)(left_near ? r : l));
             const bool take_left = hl && (left_near || !hr);
             f = __float_as_uint(take_left ? lb.w : rb.w);
@@ -486,13 +489,15 @@ struct Traversal {
             cinv = sel(leave, winv, cinv);
         }
         if (FLAT ? left != 0 && nothing_in_blas() : blas_base < 0 && tl_cur < tl_end) do_inst(any, found);
-        if (bl_cur >= bl_end && (FLAT ? nxt != kNoNode || st.sp > 0
-                                      : (blas_base >= 0 || tl_cur >= tl_end) &&
-                                            (nxt != kNoNode || st.sp > (blas_base >= 0 ? blas_base : 0))))
-            do_node();
+        if (wants_node()) do_node(any);
         if (bl_cur < bl_end) do_tri(any, found);
         if (FLAT) return !found && (left != 0 || !nothing_in_blas());
         return !found && (tl_cur < tl_end || !nothing_in_blas());
+    }
+    __device__ __forceinline__ bool wants_node() const {
+        if (FLAT) return bl_cur >= bl_end && (nxt != kNoNode || st.sp > 0);
+        return bl_cur >= bl_end && (blas_base >= 0 || tl_cur >= tl_end) &&
+               (nxt != kNoNode || st.sp > (blas_base >= 0 ? blas_base : 0));
     }
     // FLAT: also no BLAS is being traversed; otherwise the TLAS stack is empty as well.
     __device__ __forceinline__ bool nothing_in_blas() const {
