@@ -219,6 +219,37 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
         apdf.insert(apdf.end(), b.alias.pdf.begin(), b.alias.pdf.end());
         aidx.insert(aidx.end(), b.alias.alias.begin(), b.alias.alias.end());
     }
+    // the interior nodes with their children's bounds (for scenes with a list
+    // of instances, whose triangles a reference can number)
+    const bool small = tris.size() / 9 < (1u << bnd::kRefBits) - 1;
+    std::vector<bnd::NodeRec> recs;
+    std::vector<uint32_t> ref(small ? nodes.size() : 0);
+    if (small) {
+        uint32_t n_recs = 0;
+        for (size_t i = 0; i < nodes.size(); ++i)
+            ref[i] = nodes[i].is_leaf ? bnd::kRefLeaf | (uint32_t)nodes[i].count << bnd::kRefBits |
+                                            (uint32_t)nodes[i].right_or_offset
+                                      : n_recs++;
+        recs.reserve(n_recs);
+        for (size_t i = 0; i < nodes.size(); ++i) {
+            if (nodes[i].is_leaf) continue;
+            const size_t right = (size_t)nodes[i].right_or_offset;
+            if (i + 1 >= nodes.size() || right >= nodes.size()) {       // a node that no other leads to
+                recs.push_back({});
+                continue;
+            }
+            const bn_bvh_node &l = nodes[i + 1], &r = nodes[right];
+            float lref, rref, axis;
+            const int ax = nodes[i].split_axis;
+            std::memcpy(&lref, &ref[i + 1], 4);
+            std::memcpy(&rref, &ref[right], 4);
+            std::memcpy(&axis, &ax, 4);
+            recs.push_back({make_float4(l.pmin[0], l.pmin[1], l.pmin[2], l.pmax[0]),
+                            make_float4(l.pmax[1], l.pmax[2], lref, axis),
+                            make_float4(r.pmin[0], r.pmin[1], r.pmin[2], r.pmax[0]),
+                            make_float4(r.pmax[1], r.pmax[2], rref, 0.0f)});
+        }
+    }
     std::vector<bnd::DevInst> di(insts.size());
     std::vector<int4> lrec;
     for (size_t i = 0; i < insts.size(); ++i) {
@@ -256,6 +287,9 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
                 d.aux.y = d.info.y + root.right_or_offset;
                 d.aux.z = d.aux.y + root.count;
             }
+            if (small) d.aux.w = (int)ref[d.info.x];
+            d.rlo = make_float4(root.pmin[0], root.pmin[1], root.pmin[2], 0.0f);
+            d.rhi = make_float4(root.pmax[0], root.pmax[1], root.pmax[2], 0.0f);
         }
         if (in.light >= 0) lrec.push_back(make_int4((int)i, d.info.y, ntri, in.light));
     }
@@ -271,7 +305,7 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
         boxes[i] = {{b[0], b[1], b[2]}, {b[3], b[4], b[5]}};
     }
     bnh::VisitOrder vo;
-    bool flat = bnh::visit_order(tlas, boxes, bnd::kFlatMax, vo);
+    bool flat = small && bnh::visit_order(tlas, boxes, bnd::kFlatMax, vo);
     bnd::FlatScene fs{};
     if (flat) {
         for (size_t i = 0; i < insts.size(); ++i) {
@@ -287,6 +321,8 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     }
     hipStream_t s = c->stream;
     sc.flat.upload(&fs, sizeof fs, s);
+    if (!flat) recs.clear();
+    sc.recs.upload(recs.data(), recs.size() * sizeof(bnd::NodeRec), s);
     sc.tlas.upload(tlas.data(), tlas.size() * sizeof(bn_bvh_node), s);
     sc.blas.upload(nodes.data(), nodes.size() * sizeof(bn_bvh_node), s);
     sc.tris.upload(tris.data(), tris.size() * sizeof(float), s);
@@ -330,8 +366,9 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     // the list traversal addresses the pools with 32-bit byte offsets
     flat = flat && finite && sc.blas.bytes < ((size_t)1 << 32) && sc.tris.bytes < ((size_t)1 << 32);
     sc.dev.flat = flat ? (const bnd::FlatScene*)sc.flat.p : nullptr;
+    sc.dev.recs = (const bnd::NodeRec*)sc.recs.p;
     sc.dev.n_insts = sc.n_insts;
-    sc.dev.n_tlas = (int)tlas.size();
+    sc.dev.n_tlas = flat ? vo.after[0] : (int)tlas.size();
     sc.live = true;
 }
 
@@ -802,7 +839,7 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
                           std::to_string(Lr.list);
         if (Lr.uniform) {
             const bnd::DevScene& d = Lr.scene;
-            for (const void* q : {(const void*)d.tlas, (const void*)d.flat, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
+            for (const void* q : {(const void*)d.tlas, (const void*)d.flat, (const void*)d.recs, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
                                   (const void*)d.mats})
                 key += ":" + std::to_string((uintptr_t)q);
             key += ":" + std::to_string(d.exact_only) + ":" + std::to_string(d.n_insts) + ":" +

@@ -44,7 +44,7 @@ struct BlasRec {
 
 struct SceneRec {
     bool live = false;
-    DevBuf tlas, flat, blas, tris, insts, mats, lightdefs, lrec, aprob, apdf, aidx;
+    DevBuf tlas, flat, recs, blas, tris, insts, mats, lightdefs, lrec, aprob, apdf, aidx;
     int n_lights = 0, n_insts = 0;
     bn_camera camera{};
     float c2w[16] = {};

@@ -120,7 +120,23 @@ struct DevInst {
     int4 info;      // x = BLAS root node (-1: sphere), y = first triangle, z = material, w = light (indices
                     // into the scene's pools, as are those inside the BLAS nodes)
     int4 aux;       // x = 1: w2o is the identity (entries 1 and zeros of either sign) and the world bounds are
-                    // the BLAS root's; y, z: first triangle and end of a BLAS that is one leaf, else y = -1
+                    // the BLAS root's; y, z: first triangle and end of a BLAS that is one leaf, else y = -1;
+                    // w: the root as a NodeRec reference
+    float4 rlo, rhi;   // bounds of the BLAS root
+};
+// An interior node with the bounds of its children, one memory round trip for a
+// node step where the node's second half and then two children took two
+// (config-1 frame 75.1 -> 69.7 ms, 2^20 Metropolis chains 109.5 -> 104.8; before
+// the traversal step was a third shorter it made no difference), and what they
+// are: interior (index of the child's record) or a leaf (kRefLeaf, count in the
+// seven bits below, first triangle in the low kRefBits).
+constexpr uint32_t kRefLeaf = 0x80000000u;
+constexpr int kRefBits = 24;
+struct NodeRec {
+    float4 llo;     // left child: min, max.x
+    float4 lhi;     // max.yz, reference, split axis
+    float4 rlo;     // right child
+    float4 rhi;     // max.yz, reference, unused
 };
 // A scene of few instances as a list (bnh::flat_instances): what a ray needs
 // to find the instances whose bounds it meets without the TLAS.
@@ -154,6 +170,7 @@ struct DevScene {
     int cam_kind;
     int exact_only;             // scene has non-finite geometry: exact slab tests only
     const FlatScene* flat;      // null: the scene is traversed through its TLAS
+    const NodeRec* recs;        // interior BLAS nodes (scenes with a list)
     int n_insts, n_tlas;
 };
 

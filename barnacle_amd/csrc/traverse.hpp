@@ -59,10 +59,11 @@ struct TraceScene {
     const float* tris;
     const DevInst* insts;
     const FlatScene* flat;
+    const NodeRec* recs;
     int n_insts, n_tlas;
     __device__ __forceinline__ void set(const DevScene& S) {
         tlas = S.tlas; blas = S.blas; tris = S.tris; insts = S.insts;
-        flat = S.flat; n_insts = S.n_insts; n_tlas = S.n_tlas;
+        flat = S.flat; recs = S.recs; n_insts = S.n_insts; n_tlas = S.n_tlas;
     }
 };
 
@@ -396,8 +397,12 @@ struct Traversal {
             co = wo;
             cd = wd;
             cinv = winv;
-            if (aux.y >= 0) { bl_cur = aux.y; bl_end = aux.z; }
-            nxt = aux.y >= 0 ? kNoNode : (uint32_t)info.x;
+            if (FLAT) {
+                take_ref((uint32_t)aux.w);
+            } else {
+                if (aux.y >= 0) { bl_cur = aux.y; bl_end = aux.z; }
+                nxt = aux.y >= 0 ? kNoNode : (uint32_t)info.x;
+            }
         }
         if (opaque(same)) return;
         const Xf w2o = I.w2o;
@@ -417,11 +422,16 @@ struct Traversal {
             co = oo; cd = od;
             cinv = {1.0f / od.x, 1.0f / od.y, 1.0f / od.z};
             exact = exact || !finite3(co) || !finite3(cinv);
-            take_root(G.blas, info.x, true);
+            if (FLAT) {
+                const float4 a = I.rlo, b = I.rhi;
+                if (box(xyz(a), xyz(b))) take_ref((uint32_t)aux.w);
+            } else {
+                take_root(G.blas, info.x, true);
+            }
         }
     }
 
-    // Expand the next node: a leaf sets its item range; an interior node
+    // Expand the next node (FLAT: record): a leaf sets its item range; an interior node
     // tests both children with the current t and keeps those that pass (the
     // near one in `nxt`, the far one on the stack, near first as in
     // Extensions/Aggregate/BVH.fs:47-56 and Mesh.fs:233-240).  A child taken
@@ -431,7 +441,11 @@ struct Traversal {
         uint32_t e = nxt;
         if (e == kNoNode) e = st.pop();
         nxt = kNoNode;
-        const bool in_blas = FLAT || blas_base >= 0;
+        if (FLAT) {
+            do_rec(e, any);
+            return;
+        }
+        const bool in_blas = blas_base >= 0;
         const float4* base = in_blas ? G.blas : G.tlas;
         const int node = (int)e;
         const float4 b = node_half(base, node, 1);
@@ -462,6 +476,29 @@ struct Traversal {
             if (in_blas) { bl_cur = word; bl_end = end; }
             if (!in_blas) { tl_cur = word; tl_end = end; }
         }
+    }
+
+    // FLAT: the reference of a record's child (nxt == kNoNode).
+    __device__ __forceinline__ void take_ref(uint32_t e) {
+        if (e & kRefLeaf) {
+            bl_cur = (int)(e & ((1u << kRefBits) - 1));
+            bl_end = bl_cur + (int)((e & ~kRefLeaf) >> kRefBits);
+        }
+        nxt = e & kRefLeaf ? kNoNode : e;
+    }
+    __device__ __forceinline__ void do_rec(uint32_t e, bool any) {
+        if (!(e & kRefLeaf)) {
+            const NodeRec& n = *(const NodeRec*)((const char*)G.recs + e * (uint32_t)sizeof(NodeRec));
+            const float4 la = n.llo, lb = n.lhi, ra = n.rlo, rb = n.rhi;
+            const bool hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
+            const bool hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));
+            const bool left_near = any || comp(cd, __float_as_int(lb.w)) > 0.0f;
+            const uint32_t l = __float_as_uint(lb.z), r = __float_as_uint(rb.z);
+            if (hl && hr) st.push(left_near ? r : l);
+            e = hl && (left_near || !hr) ? l : r;
+            if (!hl && !hr) e = kRefLeaf;            // a leaf of no triangles
+        }
+        take_ref(e);
     }
 
     // One step of the fast traversal: an instance, then a node, then a

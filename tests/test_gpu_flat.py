@@ -55,6 +55,29 @@ def test_few_instances_equal_the_tree_walk(ctx, orc, n, fov):
     ds.release()
 
 
+def test_nodes_that_no_other_leads_to(ctx):
+    from barnacle_amd.bvh_util import NODE_DTYPE
+    sc = cubes(9, 0.0)
+    built = ctx.scene(sc)
+    export, export_blas = built.export, built.export_blas
+    stray = np.zeros(1, NODE_DTYPE)
+    stray["split_axis"], stray["right_or_offset"] = 1, 1 << 28
+    leaf = np.zeros(1, NODE_DTYPE)
+    leaf["is_leaf"], leaf["count"], leaf["pmin"], leaf["pmax"] = 1, 9, -1e4, 1e4
+
+    def more(ex, key, node):
+        ex[key] = np.concatenate([ex[key], node])
+        return ex
+
+    built.export = lambda: more(export(), "tlas", leaf)
+    built.export_blas = lambda prim: more(export_blas(prim), "nodes", stray)
+    up, _ = reupload(ctx, sc, built)
+    p = sc.pt_params()
+    assert same(up.render_pt(p), built.render_pt(p))
+    up.release()
+    built.release()
+
+
 @pytest.mark.parametrize("shrink", [0, 1, 2])
 def test_tree_that_does_not_contain_its_instances(ctx, shrink):
     """An uploaded TLAS culls what its nodes leave out, whatever the bounds of
@@ -139,3 +162,36 @@ def test_metropolis_waves_equal_the_wavefront(ctx, n):
     assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
     assert np.allclose(out[0][2], out[1][2], rtol=1e-4, atol=1e-5, equal_nan=True)
     ds.release()
+
+
+def test_leaves_of_many_triangles(ctx):
+    """References of up to 127 triangles: an uploaded BLAS that is one leaf, and
+    one whose leaves hold none."""
+    from barnacle_amd.bvh_util import NODE_DTYPE
+    sc = cubes(9, 39.3)
+    built = ctx.scene(sc)
+    export_blas = built.export_blas
+
+    def one_leaf(prim):
+        b = export_blas(prim)
+        n = len(b["tri"].reshape(-1, 3))
+        root = b["nodes"][0].copy()
+        if n > 2:
+            root["is_leaf"], root["right_or_offset"], root["count"] = 1, 0, n
+            b["nodes"] = np.array([root], NODE_DTYPE)
+        else:
+            left = root.copy()
+            left["is_leaf"], left["right_or_offset"], left["count"] = 1, 0, 0
+            right = left.copy()
+            right["count"] = n
+            root["is_leaf"], root["right_or_offset"], root["split_axis"] = 0, 2, 1
+            b["nodes"] = np.array([root, left, right], NODE_DTYPE)
+        return b
+
+    built.export_blas = one_leaf
+    up, _ = reupload(ctx, sc, built)
+    p = sc.pt_params()
+    walked, _ = up.render_pt(p, stats=True)
+    assert same(up.render_pt(p), walked)
+    up.release()
+    built.release()
