@@ -188,6 +188,35 @@ std::vector<float4> pack_lights(const std::vector<bn_light>& lights) {
     return d;
 }
 
+// The records of the interior nodes, and the reference of every node.
+void node_records(const std::vector<bn_bvh_node>& nodes, std::vector<bnd::NodeRec>& recs, std::vector<uint32_t>& ref) {
+    uint32_t n_recs = 0;
+    ref.resize(nodes.size());
+    for (size_t i = 0; i < nodes.size(); ++i)
+        ref[i] = nodes[i].is_leaf ? bnd::kRefLeaf | (uint32_t)nodes[i].count << bnd::kRefBits |
+                                        (uint32_t)nodes[i].right_or_offset
+                                  : n_recs++;
+    recs.reserve(n_recs);
+    for (size_t i = 0; i < nodes.size(); ++i) {
+        if (nodes[i].is_leaf) continue;
+        const size_t right = (size_t)nodes[i].right_or_offset;
+        if (i + 1 >= nodes.size() || right >= nodes.size()) {           // a node that no other leads to
+            recs.push_back({});
+            continue;
+        }
+        const bn_bvh_node &l = nodes[i + 1], &r = nodes[right];
+        const int ax = nodes[i].split_axis;
+        float lref, rref, axis;
+        std::memcpy(&lref, &ref[i + 1], 4);
+        std::memcpy(&rref, &ref[right], 4);
+        std::memcpy(&axis, &ax, 4);
+        recs.push_back({make_float4(l.pmin[0], l.pmin[1], l.pmin[2], l.pmax[0]),
+                        make_float4(l.pmax[1], l.pmax[2], lref, axis),
+                        make_float4(r.pmin[0], r.pmin[1], r.pmin[2], r.pmax[0]),
+                        make_float4(r.pmax[1], r.pmax[2], rref, 0.0f)});
+    }
+}
+
 void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
                   const std::vector<bn_instance_upload>& insts, const std::vector<bn_material>& mats,
                   const std::vector<bn_light>& lights, const bn_camera& cam, const float* c2w) {
@@ -219,36 +248,14 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
         apdf.insert(apdf.end(), b.alias.pdf.begin(), b.alias.pdf.end());
         aidx.insert(aidx.end(), b.alias.alias.begin(), b.alias.alias.end());
     }
-    // the interior nodes with their children's bounds (for scenes with a list
-    // of instances, whose triangles a reference can number)
-    const bool small = tris.size() / 9 < (1u << bnd::kRefBits) - 1;
-    std::vector<bnd::NodeRec> recs;
-    std::vector<uint32_t> ref(small ? nodes.size() : 0);
+    // records, unless there are more items than a reference can number
+    constexpr size_t kMost = (1u << bnd::kRefBits) - 1;
+    const bool small = c->records && tris.size() / 9 < kMost && insts.size() < kMost;
+    std::vector<bnd::NodeRec> recs, trecs;
+    std::vector<uint32_t> ref, tref;
     if (small) {
-        uint32_t n_recs = 0;
-        for (size_t i = 0; i < nodes.size(); ++i)
-            ref[i] = nodes[i].is_leaf ? bnd::kRefLeaf | (uint32_t)nodes[i].count << bnd::kRefBits |
-                                            (uint32_t)nodes[i].right_or_offset
-                                      : n_recs++;
-        recs.reserve(n_recs);
-        for (size_t i = 0; i < nodes.size(); ++i) {
-            if (nodes[i].is_leaf) continue;
-            const size_t right = (size_t)nodes[i].right_or_offset;
-            if (i + 1 >= nodes.size() || right >= nodes.size()) {       // a node that no other leads to
-                recs.push_back({});
-                continue;
-            }
-            const bn_bvh_node &l = nodes[i + 1], &r = nodes[right];
-            float lref, rref, axis;
-            const int ax = nodes[i].split_axis;
-            std::memcpy(&lref, &ref[i + 1], 4);
-            std::memcpy(&rref, &ref[right], 4);
-            std::memcpy(&axis, &ax, 4);
-            recs.push_back({make_float4(l.pmin[0], l.pmin[1], l.pmin[2], l.pmax[0]),
-                            make_float4(l.pmax[1], l.pmax[2], lref, axis),
-                            make_float4(r.pmin[0], r.pmin[1], r.pmin[2], r.pmax[0]),
-                            make_float4(r.pmax[1], r.pmax[2], rref, 0.0f)});
-        }
+        node_records(nodes, recs, ref);
+        node_records(tlas, trecs, tref);
     }
     std::vector<bnd::DevInst> di(insts.size());
     std::vector<int4> lrec;
@@ -321,8 +328,8 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     }
     hipStream_t s = c->stream;
     sc.flat.upload(&fs, sizeof fs, s);
-    if (!flat) recs.clear();
     sc.recs.upload(recs.data(), recs.size() * sizeof(bnd::NodeRec), s);
+    sc.trecs.upload(trecs.data(), trecs.size() * sizeof(bnd::NodeRec), s);
     sc.tlas.upload(tlas.data(), tlas.size() * sizeof(bn_bvh_node), s);
     sc.blas.upload(nodes.data(), nodes.size() * sizeof(bn_bvh_node), s);
     sc.tris.upload(tris.data(), tris.size() * sizeof(float), s);
@@ -363,10 +370,11 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
     for (const auto& in : insts)
         for (int k = 0; k < 6; ++k) finite = finite && std::isfinite(in.bounds[k]);
     sc.dev.exact_only = finite ? 0 : 1;
-    // the list traversal addresses the pools with 32-bit byte offsets
-    flat = flat && finite && sc.blas.bytes < ((size_t)1 << 32) && sc.tris.bytes < ((size_t)1 << 32);
+    flat = flat && finite;
     sc.dev.flat = flat ? (const bnd::FlatScene*)sc.flat.p : nullptr;
     sc.dev.recs = (const bnd::NodeRec*)sc.recs.p;
+    sc.dev.trecs = (const bnd::NodeRec*)sc.trecs.p;
+    sc.dev.mode = flat ? bnd::kList : small ? bnd::kRecs : bnd::kNodes;
     sc.dev.n_insts = sc.n_insts;
     sc.dev.n_tlas = flat ? vo.after[0] : (int)tlas.size();
     sc.live = true;
@@ -836,10 +844,11 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
                           std::to_string((uintptr_t)c->b_items.p) + ":" + std::to_string((uintptr_t)c->b_scenes.p) +
                           ":" + std::to_string((uintptr_t)c->L_out.p) + ":" + std::to_string((int)L.octant_order) + ":" + std::to_string(L.skip_dark) +
                           ":" + std::to_string(whole ? n : 0) + ":" + std::to_string(Lr.stream2 != nullptr) + ":" +
-                          std::to_string(Lr.list);
+                          std::to_string(Lr.mode);
         if (Lr.uniform) {
             const bnd::DevScene& d = Lr.scene;
-            for (const void* q : {(const void*)d.tlas, (const void*)d.flat, (const void*)d.recs, (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
+            for (const void* q : {(const void*)d.tlas, (const void*)d.flat, (const void*)d.trecs, (const void*)d.recs,
+                                  (const void*)d.blas, (const void*)d.tris, (const void*)d.insts,
                                   (const void*)d.mats})
                 key += ":" + std::to_string((uintptr_t)q);
             key += ":" + std::to_string(d.exact_only) + ":" + std::to_string(d.n_insts) + ":" +
@@ -910,13 +919,13 @@ void render_batch(Ctx* c, const bn_batch_item* items, int n, float* const* films
         }
         int path = 0, pix = 0, round_depth = 0;
         L.uniform = true;
-        L.list = true;
+        L.mode = bnd::kList;
         int k0 = -1;
         for (int k = 0; k < n; ++k) {
             if (take[k] == 0) continue;
             if (k0 < 0) k0 = k;
             L.uniform = L.uniform && items[k].scene == items[k0].scene;
-            L.list = L.list && scenes[k].flat != nullptr;
+            L.mode = std::min(L.mode, scenes[k].mode);
             bnd::RoundItem it = base[k];
             it.s0 = next[k];
             it.ns = take[k];
@@ -1630,6 +1639,9 @@ extern "C" int bn_set_option(bn_ctx* ctx, const char* key, int64_t value) {
         } else if (k == "overlap_shadow") {
             if (value < 0 || value > 1) throw Error(BN_E_INVALID, "overlap_shadow must be 0 or 1");
             c->overlap_shadow = value != 0;
+        } else if (k == "records") {
+            if (value < 0 || value > 1) throw Error(BN_E_INVALID, "records must be 0 or 1");
+            c->records = value != 0;
         } else if (k == "mlt_wave_chains") {
             if (value < 0 || value > ((int64_t)1 << 26)) throw Error(BN_E_INVALID, "mlt_wave_chains out of range");
             c->mlt_wave_chains = (int)value;

@@ -44,7 +44,7 @@ struct BlasRec {
 
 struct SceneRec {
     bool live = false;
-    DevBuf tlas, flat, recs, blas, tris, insts, mats, lightdefs, lrec, aprob, apdf, aidx;
+    DevBuf tlas, flat, trecs, recs, blas, tris, insts, mats, lightdefs, lrec, aprob, apdf, aidx;
     int n_lights = 0, n_insts = 0;
     bn_camera camera{};
     float c2w[16] = {};
@@ -122,6 +122,7 @@ struct Ctx {
     // of 24576 chains: 52 to 56 ms against 62 to 66 of wavefronts; 32768: 71 to
     // 74 against 67 to 71; 65536: 150 against 84).
     int mlt_wave_chains = 28672;
+    bool records = true;                  // node records for the scenes uploaded from now on
     DevBuf m_inner, m_outer, m_state, m_bid, m_pix_new, m_pix_cur, m_Lcur, m_rad, m_acc, m_xs;
     DevBuf m_weights, m_aprob, m_aidx, m_accepted_out;
     // GPU BVH builder (bvh_gpu.hip): items (two buffers, then the output

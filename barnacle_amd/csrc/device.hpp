@@ -130,6 +130,9 @@ struct DevInst {
 // the traversal step was a third shorter it made no difference), and what they
 // are: interior (index of the child's record) or a leaf (kRefLeaf, count in the
 // seven bits below, first triangle in the low kRefBits).
+// How a scene is traversed: by the nodes of its trees, by their records, or by
+// its list of instances and the records of its BLAS.
+enum : int { kNodes = 0, kRecs = 1, kList = 2 };
 constexpr uint32_t kRefLeaf = 0x80000000u;
 constexpr int kRefBits = 24;
 struct NodeRec {
@@ -170,7 +173,8 @@ struct DevScene {
     int cam_kind;
     int exact_only;             // scene has non-finite geometry: exact slab tests only
     const FlatScene* flat;      // null: the scene is traversed through its TLAS
-    const NodeRec* recs;        // interior BLAS nodes (scenes with a list)
+    const NodeRec *trecs, *recs;   // interior nodes of the TLAS and of the BLAS
+    int mode;                   // kNodes: more items than a reference can number; kRecs; kList: flat is set
     int n_insts, n_tlas;
 };
 

@@ -101,7 +101,7 @@ struct Launch {
     // its compact rounds launch the single-scene trace kernels (the scene
     // bound once per launch) on grid_uniform blocks.
     bool uniform;
-    bool list;                // batch mode: every scene of the round has a DevScene::flat
+    int mode;                 // batch mode: the least DevScene::mode of the round's scenes
     int grid_uniform;
     uint32_t refill;
     hipStream_t stream;

@@ -508,19 +508,19 @@ constexpr int kMltWaveK = 16;
 // WAVES per SIMD: alone on its SIMD a wave may use every register; where there
 // are more chains than SIMDs four waves share one, at 128 VGPRs, with spills
 // (1024 chains: 63.5 ms alone, 67.9 ms with four; 16384: 47.1 and 36.6 ms).
-template <int WAVES, bool FLAT>
+template <int WAVES, int MODE>
 __global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBuf M, MltParamsDev p, float* film,
                                                            uint32_t* spill, size_t spill_stride, int n,
                                                            int mutations, int nx, int max_depth, int rr_depth) {
     extern __shared__ float4 xs[];
     __shared__ uint32_t stk[kMltWaveK * 64];
     const int lane = (int)lane_id();
-    Traversal<kMltWaveK, FLAT, 64> tr;
+    Traversal<kMltWaveK, MODE, 64> tr;
     tr.st = LaneStack<kMltWaveK, 64>{stk + lane, spill, (uint32_t)spill_stride, blockIdx.x * 64u + (uint32_t)lane, 0};
     tr.clear();
     tr.G.set(S);
-    __shared__ uint8_t order[FLAT ? sizeof(FlatScene::order) : 1];
-    if (FLAT) {
+    __shared__ uint8_t order[MODE == kList ? sizeof(FlatScene::order) : 1];
+    if (MODE == kList) {
         for (int k = lane; k < (int)sizeof order; k += 64) order[k] = S.flat->order[k / kFlatMax][k % kFlatMax];
         tr.order = order;
         wave_sync();
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBu
     // a whole traversal of one ray, the same in every lane
     auto trace = [&](const Ray& r, float tmax, bool any) {
         tr.start(r, tmax, S.exact_only != 0);
-        if (FLAT) tr.take_instances_wave(any);
+        if (MODE == kList) tr.take_instances_wave(any);
         else tr.take_tlas_root();
         if (!(tmax == tmax)) tr.empty();
         bool found = false;
@@ -668,8 +668,10 @@ void launch_mlt_wave_chains(const DevScene& S, const MltBuf& M, const MltParamsD
                             hipStream_t st) {
     const int nx = 4 + 7 * max_depth;
     const size_t lds = (size_t)nx * sizeof(float4);
-    auto* run = n <= n_simd ? (S.flat ? k_mlt_wave_chains<1, true> : k_mlt_wave_chains<1, false>)
-                            : (S.flat ? k_mlt_wave_chains<4, true> : k_mlt_wave_chains<4, false>);
+    const bool alone = n <= n_simd;
+    auto* run = alone ? k_mlt_wave_chains<1, kNodes> : k_mlt_wave_chains<4, kNodes>;
+    if (S.mode == kRecs) run = alone ? k_mlt_wave_chains<1, kRecs> : k_mlt_wave_chains<4, kRecs>;
+    if (S.mode == kList) run = alone ? k_mlt_wave_chains<1, kList> : k_mlt_wave_chains<4, kList>;
     hipLaunchKernelGGL(run, dim3(min(n, grid)), dim3(64), lds, st, S, M, p, film, B.spill, B.spill_stride, n, mutations,
                        nx, max_depth, rr_depth);
 }

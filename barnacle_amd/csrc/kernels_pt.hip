@@ -63,7 +63,7 @@ template <>
 struct Work<false> {
     DevScene S;
     RoundItem it;
-    bool flat() const { return S.flat != nullptr; }
+    int mode() const { return S.mode; }
     __device__ __forceinline__ int n() const { return 1; }
     __device__ __forceinline__ int item_of_path(uint32_t) const { return 0; }
     __device__ __forceinline__ int item_of(const PathBuf&, uint32_t) const { return 0; }
@@ -81,8 +81,8 @@ struct Work<true> {
     const RoundHeader* hdr;
     const RoundItem* items;
     const DevScene* scenes;
-    bool list;                // every scene of the round has a DevScene::flat
-    bool flat() const { return list; }
+    int round_mode;           // the least DevScene::mode of the round
+    int mode() const { return round_mode; }
     __device__ __forceinline__ int n() const { return hdr->n_items; }
     // item owning a path id (the round table is ordered by path_base)
     __device__ __forceinline__ int item_of_path(uint32_t id) const {
@@ -352,17 +352,17 @@ __device__ __forceinline__ int next_segment(const SegFetch& F, uint32_t pick, ui
     return -1;
 }
 
-template <bool ANY, bool COUNT, bool BATCH, int K, bool FLAT, typename Setup, typename Init, typename Done>
+template <bool ANY, bool COUNT, bool BATCH, int K, int MODE, typename Setup, typename Init, typename Done>
 __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uint32_t* stk, uint32_t* spill,
                                                  size_t spill_stride, uint32_t refill, TraceCount& tc, Setup setup,
                                                  Init init, Done done) {
     const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
-    Traversal<K, FLAT> tr;
+    Traversal<K, MODE> tr;
     tr.st = LaneStack<K, 256>{stk + threadIdx.x, spill, (uint32_t)spill_stride, gid, 0};
     tr.clear();
     setup(tr);
-    __shared__ uint8_t order[FLAT && !BATCH ? sizeof(FlatScene::order) : 1];
-    if (FLAT && !BATCH) {
+    __shared__ uint8_t order[MODE == kList && !BATCH ? sizeof(FlatScene::order) : 1];
+    if (MODE == kList && !BATCH) {
         static_assert(sizeof(FlatScene::order) == 256, "a byte for each thread");
         order[threadIdx.x] = tr.G.flat->order[threadIdx.x / kFlatMax][threadIdx.x % kFlatMax];
         tr.order = order;
@@ -437,7 +437,7 @@ __device__ __forceinline__ void persistent_trace(SegFetch F, uint32_t count, uin
 // rays are queue[i], or position i of a compact round (queue null).
 // Eight blocks' 16-entry LDS stack windows fit a CU; the register budget is set
 // for eight waves per SIMD, seven in batches.
-template <bool COUNT, bool BATCH, int K, bool FLAT>
+template <bool COUNT, bool BATCH, int K, int MODE>
 __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_closest(Work<BATCH> W, PathBuf P, Ctl* ctl, int cur,
                                                        const uint32_t* queue, uint32_t* spill, size_t spill_stride,
                                                        uint32_t refill, unsigned long long* stats, uint32_t* seg) {
@@ -449,22 +449,22 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
         else ctl->q_count[1 - cur] = 0;
     }
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, COUNT, BATCH, K, FLAT>(
+    persistent_trace<false, COUNT, BATCH, K, MODE>(
         SegFetch{seg, kFetchSegs}, count, stk, spill, spill_stride, refill, tc,
-        [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
-        [&](Traversal<K, FLAT>& tr, uint32_t i) {
+        [&](Traversal<K, MODE>& tr) { W.bind(tr.G); },
+        [&](Traversal<K, MODE>& tr, uint32_t i) {
             const uint32_t slot = queue ? queue[i] : i;
             const float4 o4 = P.o[slot];
             const int k = W.item_of(P, slot);
             W.bind_lane(tr.G, k);
             tr.start({xyz(o4), xyz(P.d[slot])}, kInf, W.scene(k).exact_only != 0);
-            if (FLAT && BATCH) tr.order = tr.G.flat->order[0];
-            if (FLAT) tr.template take_instances<BATCH>(false);
+            if (MODE == kList && BATCH) tr.order = tr.G.flat->order[0];
+            if (MODE == kList) tr.template take_instances<BATCH>(false);
             else if (!COUNT) tr.take_tlas_root();
             // a placeholder path (padding pixel, max-depth 0) misses at once
             if (__float_as_int(o4.w) < 0) tr.empty();
         },
-        [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool) {
+        [&](Traversal<K, MODE>& tr, uint32_t i, bool fin, bool) {
             if (fin) {
                 const uint32_t slot = queue ? queue[i] : i;
                 int bin = -1, prim = -1;
@@ -863,7 +863,7 @@ __global__ __launch_bounds__(256, 3) void k_shade_c(Work<BATCH> W, PathBuf X, Pa
 // an unoccluded ray adds beta*f * Le/(pdf_b + pdf_l) to L.  Slot rounds: the
 // rays of the slots in shq, added to the slot's L.  Compact rounds (shq
 // null): ray i, added to L_out[path id] (nee_a.w).
-template <bool COUNT, bool BATCH, int K, bool FLAT>
+template <bool COUNT, bool BATCH, int K, int MODE>
 __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWaves) : 1) void k_trace_shadow(Work<BATCH> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                       float4* L_out, int par,
                                                       uint32_t* spill, size_t spill_stride, uint32_t refill,
@@ -871,22 +871,22 @@ __global__ __launch_bounds__(256, K == 16 ? (BATCH ? kTraceWavesBatch : kTraceWa
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = shq && par < 0 ? ctl->sh_count : ctl->shc[par];
     TraceCount tc{0, 0, 0};
-    persistent_trace<true, COUNT, BATCH, K, FLAT>(
+    persistent_trace<true, COUNT, BATCH, K, MODE>(
         SegFetch{seg, kShadowSegs}, count, stk, spill, spill_stride, refill, tc,
-        [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
-        [&](Traversal<K, FLAT>& tr, uint32_t i) {
+        [&](Traversal<K, MODE>& tr) { W.bind(tr.G); },
+        [&](Traversal<K, MODE>& tr, uint32_t i) {
             const uint32_t slot = shq ? shq[i] : i;
             const float4 o4 = P.sh_o[slot], d4 = P.sh_d[slot];
             const int k = shq ? W.item_of(P, slot) : (BATCH ? __float_as_int(d4.w) : 0);
             W.bind_lane(tr.G, k);
             tr.start({xyz(o4), xyz(d4)}, o4.w, W.scene(k).exact_only != 0);
-            if (FLAT && BATCH) tr.order = tr.G.flat->order[0];
-            if (FLAT) tr.template take_instances<BATCH>(true);
+            if (MODE == kList && BATCH) tr.order = tr.G.flat->order[0];
+            if (MODE == kList) tr.template take_instances<BATCH>(true);
             else if (!COUNT) tr.take_tlas_root();
             // a NaN t max fails every slab test of the reference: empty traversal
             if (!(o4.w == o4.w)) tr.empty();
         },
-        [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool found) {
+        [&](Traversal<K, MODE>& tr, uint32_t i, bool fin, bool found) {
             if (fin && !found) {
                 const uint32_t slot = shq ? shq[i] : i;
                 const float4 a = P.nee_a[slot];
@@ -1122,25 +1122,25 @@ __global__ __launch_bounds__(LDS ? kGradLdsThreads : 256) void k_shade_adj(
 // The shadow rays of a replayed bounce only record their visibility (in
 // nee_a.w): gradient sums belong in a kernel whose lanes are all busy, not in
 // the traversal loop.
-template <int K, bool FLAT>
+template <int K, int MODE>
 __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_trace_shadow_vis(Work<false> W, PathBuf P, Ctl* ctl, const uint32_t* shq,
                                                           uint32_t* spill, size_t spill_stride, uint32_t refill,
                                                           uint32_t* seg) {
     __shared__ uint32_t stk[K * 256];
     const uint32_t count = ctl->sh_count;
     TraceCount tc{0, 0, 0};
-    persistent_trace<true, false, false, K, FLAT>(
+    persistent_trace<true, false, false, K, MODE>(
         SegFetch{seg, kShadowSegs}, count, stk, spill, spill_stride, refill, tc,
-        [&](Traversal<K, FLAT>& tr) { W.bind(tr.G); },
-        [&](Traversal<K, FLAT>& tr, uint32_t i) {
+        [&](Traversal<K, MODE>& tr) { W.bind(tr.G); },
+        [&](Traversal<K, MODE>& tr, uint32_t i) {
             const uint32_t slot = shq[i];
             const float4 o4 = P.sh_o[slot];
             tr.start({xyz(o4), xyz(P.sh_d[slot])}, o4.w, W.S.exact_only != 0);
-            if (FLAT) tr.template take_instances<false>(true);
+            if (MODE == kList) tr.template take_instances<false>(true);
             else tr.take_tlas_root();
             if (!(o4.w == o4.w)) tr.empty();
         },
-        [&](Traversal<K, FLAT>& tr, uint32_t i, bool fin, bool found) {
+        [&](Traversal<K, MODE>& tr, uint32_t i, bool fin, bool found) {
             if (fin) P.nee_a[shq[i]].w = found ? 0.0f : 1.0f;
         });
 }
@@ -1344,27 +1344,27 @@ __global__ void k_shade_direct(Work<false> W, PathBuf P, Ctl* ctl, const uint32_
 }
 
 // First hit of one sample per pixel: (instance, primitive, t) in pixel order.
-template <int K, bool FLAT>
+template <int K, int MODE>
 __global__ __launch_bounds__(256, K == 16 ? kTraceWaves : 1) void k_first_hit(DevScene S, int width, int height, int sample_id, int spp,
                                                    int frame_id, int* out_inst, int* out_prim, float* out_t,
                                                    uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs) {
     __shared__ uint32_t stk[K * 256];
     const uint32_t n = (uint32_t)width * (uint32_t)height;
     TraceCount tc{0, 0, 0};
-    persistent_trace<false, false, false, K, FLAT>(
+    persistent_trace<false, false, false, K, MODE>(
         SegFetch{fetch, segs}, n, stk, spill, spill_stride, 16u, tc,
-        [&](Traversal<K, FLAT>& tr) { tr.G.set(S); },
-        [&](Traversal<K, FLAT>& tr, uint32_t p) {
+        [&](Traversal<K, MODE>& tr) { tr.G.set(S); },
+        [&](Traversal<K, MODE>& tr, uint32_t p) {
             const int x = (int)(p % (uint32_t)width), y = (int)(p / (uint32_t)width);
             uint32_t rng = xxhash3((uint32_t)x, (uint32_t)y, (uint32_t)(frame_id * spp + sample_id));
             V2 uPix, uLens;
             uPix.x = lcg(rng); uPix.y = lcg(rng);
             uLens.x = lcg(rng); uLens.y = lcg(rng);
             tr.start(camera_ray(S, x, y, uPix, uLens), kInf, S.exact_only != 0);
-            if (FLAT) tr.template take_instances<false>(false);
+            if (MODE == kList) tr.template take_instances<false>(false);
             else tr.take_tlas_root();
         },
-        [&](Traversal<K, FLAT>& tr, uint32_t p, bool fin, bool) {
+        [&](Traversal<K, MODE>& tr, uint32_t p, bool fin, bool) {
             if (fin) {
                 out_inst[p] = tr.hit_inst;
                 out_prim[p] = tr.hit_inst >= 0 ? tr.prim_of(S.insts[tr.hit_inst].info) : -1;
@@ -1385,7 +1385,7 @@ static Work<true> batch_work(const Launch& L) {
     w.hdr = L.hdr;
     w.items = L.items;
     w.scenes = L.scenes;
-    w.list = L.list;
+    w.round_mode = L.mode;
     return w;
 }
 
@@ -1396,9 +1396,11 @@ static void launch_closest_t(bool count, int k, const Work<BATCH>& W, const Path
 #define BN_TC(C, KK, F)                                                                                            \
     hipLaunchKernelGGL((k_trace_closest<C, BATCH, KK, F>), dim3(grid), dim3(256), 0, st, W, P, ctl, cur, queue, \
                        B.spill, B.spill_stride, refill, B.stats, B.fetch_seg)
-    if (count) { if (k == 16) BN_TC(true, 16, false); else BN_TC(true, 32, false); }
-    else if (W.flat()) { if (k == 16) BN_TC(false, 16, true); else BN_TC(false, 32, true); }
-    else { if (k == 16) BN_TC(false, 16, false); else BN_TC(false, 32, false); }
+    const int mode = W.mode();
+    if (count) { if (k == 16) BN_TC(true, 16, kNodes); else BN_TC(true, 32, kNodes); }
+    else if (mode == kList) { if (k == 16) BN_TC(false, 16, kList); else BN_TC(false, 32, kList); }
+    else if (mode == kRecs) { if (k == 16) BN_TC(false, 16, kRecs); else BN_TC(false, 32, kRecs); }
+    else { if (k == 16) BN_TC(false, 16, kNodes); else BN_TC(false, 32, kNodes); }
 #undef BN_TC
 }
 // par: the parity of a compact round's iteration (its shadow count and fetch
@@ -1412,9 +1414,11 @@ static void launch_shadow_t(bool count, int k, const Work<BATCH>& W, const PathB
 #define BN_TS(C, KK, F)                                                                                            \
     hipLaunchKernelGGL((k_trace_shadow<C, BATCH, KK, F>), dim3(grid), dim3(256), 0, st, W, P, ctl, shq, L_out, par, \
                        spill, B.spill_stride, refill, B.stats, seg)
-    if (count) { if (k == 16) BN_TS(true, 16, false); else BN_TS(true, 32, false); }
-    else if (W.flat()) { if (k == 16) BN_TS(false, 16, true); else BN_TS(false, 32, true); }
-    else { if (k == 16) BN_TS(false, 16, false); else BN_TS(false, 32, false); }
+    const int mode = W.mode();
+    if (count) { if (k == 16) BN_TS(true, 16, kNodes); else BN_TS(true, 32, kNodes); }
+    else if (mode == kList) { if (k == 16) BN_TS(false, 16, kList); else BN_TS(false, 32, kList); }
+    else if (mode == kRecs) { if (k == 16) BN_TS(false, 16, kRecs); else BN_TS(false, 32, kRecs); }
+    else { if (k == 16) BN_TS(false, 16, kNodes); else BN_TS(false, 32, kNodes); }
 #undef BN_TS
 }
 
@@ -1565,8 +1569,10 @@ static void iterations_t(const Work<BATCH>& W, Integrator kind, const Launch& L,
                   } }
                 { Bracket b(hook, "trace_shadow", st);
                   uint32_t* seg = B.fetch_seg + kFetchSegs * kSegStride;
-                  auto* vis = W.flat() ? (B.stack_k == 16 ? k_trace_shadow_vis<16, true> : k_trace_shadow_vis<32, true>)
-                                       : (B.stack_k == 16 ? k_trace_shadow_vis<16, false> : k_trace_shadow_vis<32, false>);
+                  const bool k16 = B.stack_k == 16;
+                  auto* vis = k16 ? k_trace_shadow_vis<16, kNodes> : k_trace_shadow_vis<32, kNodes>;
+                  if (W.mode() == kRecs) vis = k16 ? k_trace_shadow_vis<16, kRecs> : k_trace_shadow_vis<32, kRecs>;
+                  if (W.mode() == kList) vis = k16 ? k_trace_shadow_vis<16, kList> : k_trace_shadow_vis<32, kList>;
                   hipLaunchKernelGGL(vis, dim3(L.grid_trace), dim3(256), 0, st, W, P, ctl, B.shq, B.spill,
                                      B.spill_stride, L.refill, seg); }
                 { Bracket b(hook, "nee_adj", st);
@@ -1662,8 +1668,9 @@ void launch_trace_shadow(bool count, const DevScene& S, const PathBuf& P, Ctl* c
 void launch_first_hit(const DevScene& S, int w, int h, int sample_id, int spp, int frame_id, int* inst, int* prim,
                       float* t, uint32_t* spill, size_t spill_stride, uint32_t* fetch, int segs, int stack_k, int grid,
                       hipStream_t st) {
-    auto* hit = S.flat ? (stack_k == 16 ? k_first_hit<16, true> : k_first_hit<32, true>)
-                       : (stack_k == 16 ? k_first_hit<16, false> : k_first_hit<32, false>);
+    auto* hit = stack_k == 16 ? k_first_hit<16, kNodes> : k_first_hit<32, kNodes>;
+    if (S.mode == kRecs) hit = stack_k == 16 ? k_first_hit<16, kRecs> : k_first_hit<32, kRecs>;
+    if (S.mode == kList) hit = stack_k == 16 ? k_first_hit<16, kList> : k_first_hit<32, kList>;
     hipLaunchKernelGGL(hit, dim3(grid), dim3(256), 0, st, S, w, h, sample_id, spp, frame_id, inst, prim, t, spill,
                        spill_stride, fetch, segs);
 }

@@ -59,11 +59,11 @@ struct TraceScene {
     const float* tris;
     const DevInst* insts;
     const FlatScene* flat;
-    const NodeRec* recs;
+    const NodeRec *trecs, *recs;
     int n_insts, n_tlas;
     __device__ __forceinline__ void set(const DevScene& S) {
         tlas = S.tlas; blas = S.blas; tris = S.tris; insts = S.insts;
-        flat = S.flat; recs = S.recs; n_insts = S.n_insts; n_tlas = S.n_tlas;
+        flat = S.flat; trecs = S.trecs; recs = S.recs; n_insts = S.n_insts; n_tlas = S.n_tlas;
     }
 };
 
@@ -86,8 +86,9 @@ __device__ __forceinline__ Scalar<T>* scalar(const T* p) { return (Scalar<T>*)(u
 // of 38 busy lanes of a wave step stood at a TLAS node or at an instance they
 // then missed, and the traversal is bound by instruction issue.  Config-1 frame
 // 109 -> 89 ms, 1024x768 frame of analytic spheres 11.7 -> 8.8 ms.
-template <int K, bool FLAT, int PITCH = 256>
+template <int K, int MODE, int PITCH = 256>
 struct Traversal {
+    static constexpr bool FLAT = MODE == kList, RECS = MODE != kNodes;
     TraceScene G;
     // world ray and the ray of the current space (world, or object inside a BLAS)
     V3 wo, wd, winv;
@@ -108,12 +109,12 @@ struct Traversal {
     // The primitive of the hit as the reference numbers it: a mesh's triangle.
     __device__ __forceinline__ int prim_of(int4 info) const { return hit_prim - (info.x >= 0 ? info.y : 0); }
 
-    // Half of a node.  FLAT scenes have pools of less than 4 GiB: an offset of
+    // Half of a node.  With records the pools have less than 4 GiB: an offset of
     // 32 bits to a base in scalar registers takes no 64-bit address arithmetic.
     // (With indices into the pools in the nodes, so that a lane holds no BLAS
     // root or first triangle, and the order in LDS: config-1 frame 89 -> 84 ms.)
     __device__ __forceinline__ static float4 node_half(const float4* nodes, int i, int half) {
-        if (FLAT) return *(const float4*)((const char*)nodes + ((uint32_t)i * 32u + 16u * half));
+        if (RECS) return *(const float4*)((const char*)nodes + ((uint32_t)i * 32u + 16u * half));
         return nodes[2 * i + half];
     }
     __device__ __forceinline__ static Tri load_tri32(const float* tris, int i) {
@@ -350,7 +351,7 @@ struct Traversal {
     // One triangle of the current BLAS leaf.
     __device__ __forceinline__ void do_tri(bool any, bool& found) {
         const int idx = bl_cur++;
-        const Tri tr = FLAT ? load_tri32(G.tris, idx) : load_tri(G.tris, idx);
+        const Tri tr = RECS ? load_tri32(G.tris, idx) : load_tri(G.tris, idx);
         if (box_tri(tr)) {
             float tt;
             if (tri_hit(tr, co, cd, t, tt)) {
@@ -397,7 +398,7 @@ struct Traversal {
             co = wo;
             cd = wd;
             cinv = winv;
-            if (FLAT) {
+            if (RECS) {
                 take_ref((uint32_t)aux.w);
             } else {
                 if (aux.y >= 0) { bl_cur = aux.y; bl_end = aux.z; }
@@ -422,7 +423,7 @@ struct Traversal {
             co = oo; cd = od;
             cinv = {1.0f / od.x, 1.0f / od.y, 1.0f / od.z};
             exact = exact || !finite3(co) || !finite3(cinv);
-            if (FLAT) {
+            if (RECS) {
                 const float4 a = I.rlo, b = I.rhi;
                 if (box(xyz(a), xyz(b))) take_ref((uint32_t)aux.w);
             } else {
@@ -431,7 +432,7 @@ struct Traversal {
         }
     }
 
-    // Expand the next node (FLAT: record): a leaf sets its item range; an interior node
+    // Expand the next node (RECS: record): a leaf sets its item range; an interior node
     // tests both children with the current t and keeps those that pass (the
     // near one in `nxt`, the far one on the stack, near first as in
     // Extensions/Aggregate/BVH.fs:47-56 and Mesh.fs:233-240).  A child taken
@@ -441,7 +442,7 @@ struct Traversal {
         uint32_t e = nxt;
         if (e == kNoNode) e = st.pop();
         nxt = kNoNode;
-        if (FLAT) {
+        if (RECS) {
             do_rec(e, any);
             return;
         }
@@ -478,17 +479,19 @@ struct Traversal {
         }
     }
 
-    // FLAT: the reference of a record's child (nxt == kNoNode).
+    // RECS: the reference of a record's child, or of a root (nxt == kNoNode).
+    // (Adjoint step over 8000 instances: 43.3 ms by nodes, 41.7 by records.)
     __device__ __forceinline__ void take_ref(uint32_t e) {
-        if (e & kRefLeaf) {
-            bl_cur = (int)(e & ((1u << kRefBits) - 1));
-            bl_end = bl_cur + (int)((e & ~kRefLeaf) >> kRefBits);
-        }
+        const int first = (int)(e & ((1u << kRefBits) - 1)), end = first + (int)((e & ~kRefLeaf) >> kRefBits);
+        const bool in_blas = FLAT || blas_base >= 0;
+        if ((e & kRefLeaf) && in_blas) { bl_cur = first; bl_end = end; }
+        if ((e & kRefLeaf) && !in_blas) { tl_cur = first; tl_end = end; }
         nxt = e & kRefLeaf ? kNoNode : e;
     }
     __device__ __forceinline__ void do_rec(uint32_t e, bool any) {
         if (!(e & kRefLeaf)) {
-            const NodeRec& n = *(const NodeRec*)((const char*)G.recs + e * (uint32_t)sizeof(NodeRec));
+            const NodeRec* base = FLAT || blas_base >= 0 ? G.recs : G.trecs;
+            const NodeRec& n = *(const NodeRec*)((const char*)base + e * (uint32_t)sizeof(NodeRec));
             const float4 la = n.llo, lb = n.lhi, ra = n.rlo, rb = n.rhi;
             const bool hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
             const bool hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));

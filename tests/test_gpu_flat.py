@@ -1,5 +1,5 @@
-"""Scenes of at most 32 instances are traversed through a list of their bounds
-in place of the TLAS: the same films and hits as the walk of the reference's
+"""Scenes are traversed by records of their nodes, those of at most 32 instances
+through a list of their bounds in place of the TLAS: the same films and hits as the walk of the reference's
 tree (the counting kernels), on both sides of the limit, for rays with zero
 direction components (whose slab tests see NaNs: bounds in the plane of the
 origin) and for a tree whose nodes do not contain their instances."""
@@ -39,10 +39,15 @@ def same(a, b):
 
 @pytest.mark.parametrize("fov", [39.3, 0.0])
 @pytest.mark.parametrize("n", [6, 7, 20, 31, 32, 33, 40])
-def test_few_instances_equal_the_tree_walk(ctx, orc, n, fov):
-    print(f"{n} instances, fov {fov}", flush=True)
+@pytest.mark.parametrize("records", [1, 0])
+def test_few_instances_equal_the_tree_walk(ctx, orc, n, fov, records):
+    print(f"{n} instances, fov {fov}, records {records}", flush=True)
     sc = cubes(n, fov)
-    ds = ctx.scene(sc)
+    ctx.set_option("records", records)
+    try:
+        ds = ctx.scene(sc)
+    finally:
+        ctx.set_option("records", 1)
     p = sc.pt_params()
     walked, _ = ds.render_pt(p, stats=True)
     assert same(ds.render_pt(p), walked)
@@ -137,8 +142,13 @@ def test_mixed_batches_equal_plain_frames(ctx, sizes):
     """A batch round binds each ray's scene: lists where all its scenes have
     one, else trees; the same graph key must not stand for both."""
     ds = [ctx.scene(cubes(n, 39.3)) for n in sizes]
+    ctx.set_option("records", 0)
+    try:
+        ds.append(ctx.scene(cubes(11, 39.3)))
+    finally:
+        ctx.set_option("records", 1)
     ps = [d.sc.pt_params() for d in ds]
-    for pick in ((0, 1, 2), (0, 2), (1, 0), (0, 2)):
+    for pick in ((0, 1, 2), (0, 2), (1, 0), (0, 2), (0, 3), (0, 2)):
         for k, film in zip(pick, ctx.render_batch([(ds[k], ps[k]) for k in pick])[0]):
             assert same(film, ds[k].render_pt(ps[k], stats=True)[0])
     for d in ds:
