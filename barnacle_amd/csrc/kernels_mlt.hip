@@ -531,6 +531,8 @@ __global__ __launch_bounds__(64, WAVES) void k_mlt_wave_chains(DevScene S, MltBu
         if (MODE == kList) tr.take_instances_wave(any);
         else tr.take_tlas_root();
         if (!(tmax == tmax)) tr.empty();
+        if constexpr (MODE == kList)
+            if (any) return tr.any_hit_wave(stk, kMltWaveK * 64);
         bool found = false;
         while (tr.step_fast(any, found)) {}
         if (any) tr.clear();

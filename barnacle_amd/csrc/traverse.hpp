@@ -539,6 +539,67 @@ struct Traversal {
         return bl_cur >= bl_end && (blas_base >= 0 || tl_cur >= tl_end) &&
                (nxt != kNoNode || st.sp > (blas_base >= 0 ? blas_base : 0));
     }
+    // The any-hit query of a ray that all lanes of the wave hold (kList, after
+    // start() and take_instances_wave()).  It finds the same in any order, so
+    // the lanes take up to 64 of the open nodes at a time: a ray needs about
+    // as many steps as a BLAS has levels, not as many as it visits nodes.
+    // The open references are a stack of `cap` words in LDS; a step takes m of
+    // them and puts back at most 2 m, and only one at a time (a depth-first
+    // walk, which adds one a level) when fewer than 64 + 64 would stay free.
+    // 300 mutations of 1024 Metropolis chains: 39.8 -> 35.4 ms.
+    __device__ __forceinline__ bool any_hit_wave(uint32_t* open, int cap) {
+        const int lane = (int)lane_id();
+        bool found = false;
+        while (left != 0 && !found) {
+            bl_cur = bl_end = 0;
+            nxt = kNoNode;
+            do_inst(true, found);
+            if (found) break;
+            // the triangles of a BLAS of one leaf
+            for (int k = bl_cur + lane; k < bl_end; k += 64) found = found || hits(k);
+            if (nxt != kNoNode) {
+                int n = 1;
+                if (lane == 0) open[0] = nxt;
+                wave_sync();
+                while (n > 0 && __ballot(found) == 0) {
+                    const int m = min(min(n, 64), max(1, cap - 128 - n));
+                    n -= m;
+                    uint32_t l = 0, r = 0;
+                    bool hl = false, hr = false;
+                    if (lane < m) {
+                        const uint32_t e = open[n + lane];
+                        if (e & kRefLeaf) {
+                            const int first = (int)(e & ((1u << kRefBits) - 1));
+                            const int end = first + (int)((e & ~kRefLeaf) >> kRefBits);
+                            for (int k = first; k < end; ++k) found = found || hits(k);
+                        } else {
+                            const NodeRec& rec = *(const NodeRec*)((const char*)G.recs + e * (uint32_t)sizeof(NodeRec));
+                            const float4 la = rec.llo, lb = rec.lhi, ra = rec.rlo, rb = rec.rhi;
+                            hl = box(mk(la.x, la.y, la.z), mk(la.w, lb.x, lb.y));
+                            hr = box(mk(ra.x, ra.y, ra.z), mk(ra.w, rb.x, rb.y));
+                            l = __float_as_uint(lb.z);
+                            r = __float_as_uint(rb.z);
+                        }
+                    }
+                    const uint64_t ml = __ballot(hl), mr = __ballot(hr);
+                    wave_sync();
+                    if (hl) open[n + (int)mbcnt(ml)] = l;
+                    n += __popcll(ml);
+                    if (hr) open[n + (int)mbcnt(mr)] = r;
+                    n += __popcll(mr);
+                    wave_sync();
+                }
+            }
+            found = __ballot(found) != 0;
+        }
+        clear();
+        return found;
+    }
+    __device__ __forceinline__ bool hits(int triangle) const {
+        const Tri tr = load_tri32(G.tris, triangle);
+        float tt;
+        return box_tri(tr) && tri_hit(tr, co, cd, t, tt);
+    }
     // FLAT: also no BLAS is being traversed; otherwise the TLAS stack is empty as well.
     __device__ __forceinline__ bool nothing_in_blas() const {
         return bl_cur >= bl_end && nxt == kNoNode && st.sp == 0;
