@@ -607,10 +607,14 @@ __device__ __forceinline__ bool dark_term(float a, float b) {
 // are returned in v.
 __device__ __forceinline__ void stage_shadow(ShadeStage* stage, int slot, const float4& o, const float4& d,
                                              const float4& a, const float4& b);
+struct VertexIn { float4 o, d, beta; uint32_t rng; };
+__device__ __forceinline__ VertexIn load_vertex(const PathBuf& P, uint32_t at) {
+    return {P.o[at], P.d[at], P.beta[at], P.rng[at]};
+}
 __device__ __forceinline__ void shade_vertex(const DevScene& S, const RoundItem& it, const PathBuf& P, uint32_t at,
-                                             int4 h, Vertex& v, float4* Lacc = nullptr, ShadeStage* stage = nullptr,
-                                             int slot = 0, bool skip_dark = false) {
-    const float4 o4 = P.o[at], d4 = P.d[at];
+                                             const VertexIn& in, int4 h, Vertex& v, float4* Lacc = nullptr,
+                                             ShadeStage* stage = nullptr, int slot = 0, bool skip_dark = false) {
+    const float4 o4 = in.o, d4 = in.d;
     const Ray r = {xyz(o4), xyz(d4)};
     const float prev_pdf = d4.w;
     const int depth = __float_as_int(o4.w);
@@ -618,7 +622,7 @@ __device__ __forceinline__ void shade_vertex(const DevScene& S, const RoundItem&
     const int4 info = S.insts[h.x].info;
     V3 L = Lacc ? V3{0.0f, 0.0f, 0.0f} : xyz(P.L[at]);
     // a camera path starts with beta = 1 (regen_c does not store it)
-    V3 beta = depth == 0 ? V3{1.0f, 1.0f, 1.0f} : xyz(P.beta[at]);
+    V3 beta = depth == 0 ? V3{1.0f, 1.0f, 1.0f} : xyz(in.beta);
     v.cont = false;
     v.shadow = false;
     if (info.w >= 0) {
@@ -630,7 +634,7 @@ __device__ __forceinline__ void shade_vertex(const DevScene& S, const RoundItem&
         else L = fma3(beta, Le * w, L);
     }
     if (info.z >= 0) {
-        uint32_t rng = P.rng[at];
+        uint32_t rng = in.rng;
         const Mat m = load_mat(S, info.z);
         const V3 wo = -r.d;
         const V3 wo_l = to_local(g, wo);
@@ -696,7 +700,7 @@ __global__ __launch_bounds__(256) void k_shade(Work<BATCH> W, PathBuf P, Ctl* ct
             while (i >= start[b + 1]) ++b;
             slot = bins[(size_t)b * bin_cap + (i - start[b])];
             const int k = W.item_of(P, slot);
-            shade_vertex(W.scene(k), W.item(k), P, slot, P.hit[slot], v);
+            shade_vertex(W.scene(k), W.item(k), P, slot, load_vertex(P, slot), P.hit[slot], v);
             if (v.shadow) {
                 P.sh_o[slot] = v.sh_o;
                 P.sh_d[slot] = v.sh_d;
@@ -755,12 +759,18 @@ __device__ __forceinline__ void shade_tile(const Work<BATCH>& W, const PathBuf& 
         pid = X.pid[i];
         k = W.item_of(X, i);
         const int4 h = X.hit[i];
+        // The path's state is on its way while the hit decides whether it is
+        // needed (nearly always).  With its loads behind that branch, one
+        // after the other, the kernel takes 20 VGPRs more and waits longer:
+        // config-1 frame 69.4 -> 67.8 ms, 1024x768 lens frame 7.53 -> 7.28.
+        VertexIn in = load_vertex(X, i);
+        pin(in.o.x); pin(in.d.x); pin(in.beta.x); pin(in.rng);
         Vertex v;
         v.cont = false;
         v.shadow = false;
         if (h.x >= 0) {
             ++shaded;
-            shade_vertex(W.scene(k), W.item(k), X, i, h, v, &L_out[pid], &sg, t, skip_dark);
+            shade_vertex(W.scene(k), W.item(k), X, i, in, h, v, &L_out[pid], &sg, t, skip_dark);
         }
         cont = v.cont;
         shadow = v.shadow;
@@ -1449,13 +1459,13 @@ static void compact_iterations_t(const Work<BATCH>& W, const Launch& L, const Pa
     // round over one scene traces with the single-scene kernels.
     const bool one_scene = BATCH && L.uniform;
     // regen_c and shade_c run one resident set of blocks (three 256-thread
-    // blocks per CU, shade_c's launch bound: 139 VGPRs, no spills), each
+    // blocks per CU, shade_c's launch bound: 145 VGPRs, no spills), each
     // striding over the tiles of positions.  With twice as many blocks the
     // traversal of the next bounce, which reads the positions in the order
     // the blocks appended them, was measured 1.6% (config 1) to 3.6%
     // (32-scene batch) slower; four blocks per CU at four waves per SIMD
-    // (6 VGPRs spilled) made shade_c 0.7 ms faster per config-1 frame but
-    // the two-stream frame 2.4 ms slower.
+    // (16 VGPRs spilled) make a config-1 frame take 68.6 ms, not 67.6, and
+    // the 256x256 box frame 1.26, not 1.18.
     const int grid_c = L.grid_shade * 3 / 8;
     // With a second stream, the shadow rays of iteration i are traced while
     // regen, prep and trace_closest of iteration i + 1 run: shade_c(i + 1)

@@ -15,6 +15,9 @@ __device__ __forceinline__ int opaque(int v) {
     asm volatile("" : "+v"(v));
     return v;
 }
+// v, loaded by now: a load whose value is pinned is not moved to a later place.
+__device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
 // Orders the wave's LDS accesses: what its lanes wrote before is what any of
 // them reads after.
 __device__ __forceinline__ void wave_sync() {
