@@ -598,7 +598,8 @@ def main():
         with open(path) as fh:
             return json.load(fh)
     prof = load_profile("counters_config1.json").get("kernels", {})
-    names = {"trace_closest": "k_trace_closest<false, false, 16>", "trace_shadow": "k_trace_shadow<false, false, 16>",
+    names = {"trace_closest": "k_trace_closest<false, false, 16, 2>",
+             "trace_shadow": "k_trace_shadow<false, false, 16, 2>",
              "shade_c": "k_shade_c<false, true>"}
     traffic_of = {k: prof.get(v, {}).get("hbm_bytes_per_launch") for k, v in names.items()}
     l2 = {k: {"l2_hit_rate": prof.get(v, {}).get("l2_hit_rate")} for k, v in names.items()}
@@ -619,10 +620,12 @@ def main():
             r["traffic_frac"] = r["traffic_gbs"] / HBM_PEAK_GBS
         return r
     rl_closest = roofline("trace_closest", "trace_closest", closest_bytes(st_tr))
-    # The closest-hit traversal keeps 87% of its VALU issue slots busy
-    # (profiles/trace_config1_sq_counters.md): the byte roofline is the
-    # contract's yardstick, instruction issue is what limits it.
-    rl_closest["limiter"] = "VALU instruction issue (87% of issue slots, profiles/trace_config1_sq_counters.md)"
+    # The closest-hit traversal issues in 65% of its VALU slots, launches of
+    # all sizes averaged (profiles/trace_config1_sq_counters.md): the byte
+    # roofline is the contract's yardstick, instruction issue and the latency
+    # of a step are what limits it.
+    rl_closest["limiter"] = ("VALU instruction issue (65% of issue slots, profiles/trace_config1_sq_counters.md) and "
+                             "the latency of a step")
 
     out = {
         "metric": "Mrays/s (batched vs plain, %HBM peak) + adjoint iters/s at RMSE<=1e-3 vs CPU",
