@@ -39,6 +39,7 @@
 namespace bvhg {
 
 constexpr int kBins = 12, kLeaf = 4, kMaxDepth = 64;        // BVHBuildConfig (Util/BVH.fs:99-107)
+constexpr int kLeafMost = 127;                              // what a node's int8 count holds
 constexpr int kThreads = 256, kIpt = 4;
 constexpr int kChunk = kThreads * kIpt;                     // items per chunk block
 constexpr int kWavesPerBlock = kThreads / 64;
@@ -445,6 +446,10 @@ __global__ void __launch_bounds__(kThreads) k_task_split(Bufs B, int level) {
                 child_task[side] = k;
                 child_chunk0[side] = c0;
                 code[side] = u;
+            } else if (t.depth + 1 >= kMaxDepth && l - f > kLeafMost) {
+                // a leaf that its count cannot hold (and a task that k_small's
+                // LDS may not): the host gives up before the subtrees are built
+                atomicOr(&B.ctl->err, kErrLeaf);
             } else {
                 const int k = atomicAdd(&B.ctl->n_small, 1);
                 if (k >= B.small_cap) { atomicOr(&B.ctl->err, kErrCapacity); continue; }
@@ -533,6 +538,7 @@ __device__ __forceinline__ bn_bvh_node make_node(const DBox& b, int32_t word, bo
 // like this, 0.26 ms for tasks of up to 128 items), and the SAH sweep runs in 22 lanes, one per prefix and suffix.
 constexpr int kPer = 4;
 constexpr int kSmallMax = 64 * kPer;
+static_assert(kSmallMax >= kLeafMost, "a task at the depth limit fits, whatever the option says");
 constexpr int kRow = kSmallMax + 4;               // the two sides' rows start in different banks
 struct SmallLds {
     float f[6][kRow];
@@ -638,8 +644,8 @@ __global__ void __launch_bounds__(kThreads) k_small(Bufs B, int n_small) {
         }
         wave_union6(bb, lanes);
         if (cnt <= kLeaf || depth >= kMaxDepth) {
-            if (cnt > 127) {
-                if (lane == 0) atomicOr(&B.ctl->err, 1);
+            if (cnt > kLeafMost) {
+                if (lane == 0) atomicOr(&B.ctl->err, kErrLeaf);
             } else if (lane == 0) {
                 region[me] = make_node(dbox(bb), task.first + first - off, true, 0, cnt);
             }
@@ -937,6 +943,7 @@ GpuBvh bvh_build_gpu(Ctx* c, const std::vector<const float*>& sets, const std::v
         hip_check(hipStreamSynchronize(st), "bvh level");
         if (ctl.err & kErrFinite) throw Error(BN_E_INVALID, "GPU BVH build needs finite bounds (bn_bvh_build takes any)");
         if (ctl.err & kErrCapacity) throw Error(BN_E_CAPACITY, "GPU BVH build: task capacity exceeded");
+        if (ctl.err & kErrLeaf) throw Error(BN_E_CAPACITY, "BVH leaf larger than the int8 count field");
     };
     // Levels: as many as an even tree has and three more, then four at a time
     // while there are tasks left.  A level holds at most twice the tasks of

@@ -1,0 +1,56 @@
+"""The GPU BVH build at the edges of what it takes: trees as deep as the depth
+limit, whose last leaf holds what a node's int8 count can hold and no more."""
+import numpy as np
+import pytest
+
+from barnacle_amd import configs, native, scene
+
+pytestmark = pytest.mark.gpu
+BN_E_CAPACITY = -5
+
+
+def point_boxes(x):
+    p = np.zeros((len(x), 3), np.float32)
+    p[:, 0] = x
+    return np.concatenate([p, p], 1)
+
+
+def peeled(kind, n):
+    """n points that stay together in the leaf at depth 64, behind 64 that leave one a level."""
+    if kind == "powers_of_13":                  # the 67 points 13^-33 .. 13^33: the last three stay too
+        return point_boxes(np.concatenate([13.0 ** np.arange(-33, 34), np.zeros(n - 3)]))
+    return point_boxes(np.concatenate([np.zeros(n), 2.0 ** (-120 + 3.75 * np.arange(64))]))
+
+
+@pytest.mark.parametrize("small", [128, 512])
+@pytest.mark.parametrize("kind", ["powers_of_13", "powers_of_2"])
+@pytest.mark.parametrize("n", [100, 127, 128, 256, 257, 300, 3003, 5000])
+def test_leaf_at_the_depth_limit(ctx, kind, n, small):
+    b = peeled(kind, n)
+    print(f"{kind} {n}, bvh_small {small}", flush=True)
+    ctx.set_option("bvh_small", small)
+    try:
+        if n <= 127:
+            hn, hp = native.bvh_build(b)
+            gn, gp = ctx.bvh_build(b)
+            assert gn.tobytes() == hn.tobytes() and np.array_equal(gp, hp)
+            assert gn["count"][gn["is_leaf"] != 0].max() == n
+        else:
+            for build in (native.bvh_build, ctx.bvh_build):
+                with pytest.raises(native.BarnacleError, match="int8 count") as e:
+                    build(b)
+                assert e.value.code == BN_E_CAPACITY
+        after = point_boxes(np.arange(1000.0))
+        assert ctx.bvh_build(after)[0].tobytes() == native.bvh_build(after)[0].tobytes()
+    finally:
+        ctx.set_option("bvh_small", 128)
+
+
+def test_scene_with_such_a_mesh_is_refused(ctx):
+    x = peeled("powers_of_13", 3003)[:, :3]
+    info = configs.cornell_box(16, 16, 1, 2)
+    info["primitives"][0] = {"type": "mesh", "vertices": x.reshape(-1),
+                             "indices": np.repeat(np.arange(len(x), dtype=np.int32), 3)}
+    with pytest.raises(native.BarnacleError, match="int8 count") as e:
+        ctx.scene(scene.load_scene(info))
+    assert e.value.code == BN_E_CAPACITY
