@@ -619,7 +619,9 @@ __global__ void __launch_bounds__(kThreads) k_small(Bufs B, int n_small) {
         const int me = nodes++;
         if (parent >= 0 && lane == 0) region[parent].right_or_offset = me;
         const int cnt = last - first;
-        const int per = (cnt + 63) >> 6;                  // at most kPer
+        // at most kPer; a node has no items where the centroids' extent is
+        // infinite, which puts all of its parent's in bin 0
+        const int per = max(1, (cnt + 63) >> 6);
         const int lanes = (cnt + per - 1) / per;          // lanes with items
         const int b = min(first + lane * per, last), n = min(b + per, last) - b;
         Box6 its[kPer], bb = empty6(), cb = empty6();

@@ -54,3 +54,32 @@ def test_scene_with_such_a_mesh_is_refused(ctx):
     with pytest.raises(native.BarnacleError, match="int8 count") as e:
         ctx.scene(scene.load_scene(info))
     assert e.value.code == BN_E_CAPACITY
+
+
+def one_far_away(n):
+    """Finite boxes, of which one has a centroid that overflows: the extent of
+    the centroids is infinite, all items of a node fall in its first bin, and
+    every node down to the depth limit has a right child without items."""
+    rng = np.random.default_rng(n)
+    lo = rng.uniform(-9, 9, (n, 3))
+    b = np.concatenate([lo, lo + 1], 1).astype(np.float32)
+    b[n // 2, [0, 3]] = 3e38
+    return b
+
+
+@pytest.mark.parametrize("n", [4, 65, 100, 127])
+def test_nodes_without_items(ctx, n):
+    b = one_far_away(n)
+    print(f"{n} boxes", flush=True)
+    hn, hp = native.bvh_build(b)
+    gn, gp = ctx.bvh_build(b)
+    assert gn.tobytes() == hn.tobytes() and np.array_equal(gp, hp)
+    assert len(gn) == (1 if n == 4 else 2 * 64 + 1)
+
+
+@pytest.mark.parametrize("n", [128, 129, 3000])
+def test_more_such_boxes_than_a_leaf_holds(ctx, n):
+    for build in (native.bvh_build, ctx.bvh_build):
+        with pytest.raises(native.BarnacleError, match="int8 count") as e:
+            build(one_far_away(n))
+        assert e.value.code == BN_E_CAPACITY
