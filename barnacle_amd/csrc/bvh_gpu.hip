@@ -614,6 +614,11 @@ __global__ void __launch_bounds__(kThreads) k_small(Bufs B, int n_small) {
     bnd::wave_sync();
     int sp = 1, nodes = 0;
     while (sp > 0) {
+        // nodes without items are the only way past the region's 2 * total
+        if (nodes >= 2 * total) {
+            if (lane == 0) atomicOr(&B.ctl->err, kErrCount);
+            break;
+        }
         const int4 f = S.frames[--sp];
         const int first = sreg(f.x), last = sreg(f.y), depth = sreg(f.z), parent = sreg(f.w);
         const int me = nodes++;

@@ -83,3 +83,15 @@ def test_more_such_boxes_than_a_leaf_holds(ctx, n):
         with pytest.raises(native.BarnacleError, match="int8 count") as e:
             build(one_far_away(n))
         assert e.value.code == BN_E_CAPACITY
+
+
+@pytest.mark.parametrize("n", [5, 20, 63, 64])
+def test_trees_of_more_nodes_than_two_an_item(ctx, n):
+    """129 nodes for at most 64 items: the GPU build has room for two nodes an
+    item, refuses, and is as good as new."""
+    with pytest.raises(native.BarnacleError, match="node count"):
+        ctx.bvh_build(one_far_away(n))
+    after = np.concatenate([one_far_away(4), point_boxes(np.arange(300.0))])
+    with pytest.raises(native.BarnacleError, match="int8 count"):
+        ctx.bvh_build(after)
+    assert ctx.bvh_build(after[4:])[0].tobytes() == native.bvh_build(after[4:])[0].tobytes()
