@@ -248,9 +248,8 @@ void upload_scene(Ctx* c, SceneRec& sc, const std::vector<bn_bvh_node>& tlas,
         apdf.insert(apdf.end(), b.alias.pdf.begin(), b.alias.pdf.end());
         aidx.insert(aidx.end(), b.alias.alias.begin(), b.alias.alias.end());
     }
-    // records, unless there are more items than a reference can number
-    constexpr size_t kMost = (1u << bnd::kRefBits) - 1;
-    const bool small = c->records && tris.size() / 9 < kMost && insts.size() < kMost;
+    // records, where they can stand for the nodes
+    const bool small = c->records && bnd::records_reach(tris.size() / 9, nodes.size(), insts.size(), tlas.size());
     std::vector<bnd::NodeRec> recs, trecs;
     std::vector<uint32_t> ref, tref;
     if (small) {

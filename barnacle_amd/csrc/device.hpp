@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "node_ref.hpp"
 #include "trig.hpp"
 
 namespace bnd {
@@ -124,23 +125,21 @@ struct DevInst {
                     // w: the root as a NodeRec reference
     float4 rlo, rhi;   // bounds of the BLAS root
 };
+// How a scene is traversed: by the nodes of its trees, by their records, or by
+// its list of instances and the records of its BLAS.
+enum : int { kNodes = 0, kRecs = 1, kList = 2 };
 // An interior node with the bounds of its children, one memory round trip for a
 // node step where the node's second half and then two children took two
 // (config-1 frame 75.1 -> 69.7 ms, 2^20 Metropolis chains 109.5 -> 104.8; before
 // the traversal step was a third shorter it made no difference), and what they
-// are: interior (index of the child's record) or a leaf (kRefLeaf, count in the
-// seven bits below, first triangle in the low kRefBits).
-// How a scene is traversed: by the nodes of its trees, by their records, or by
-// its list of instances and the records of its BLAS.
-enum : int { kNodes = 0, kRecs = 1, kList = 2 };
-constexpr uint32_t kRefLeaf = 0x80000000u;
-constexpr int kRefBits = 24;
+// are (node_ref.hpp).
 struct NodeRec {
     float4 llo;     // left child: min, max.x
     float4 lhi;     // max.yz, reference, split axis
     float4 rlo;     // right child
     float4 rhi;     // max.yz, reference, unused
 };
+static_assert(sizeof(NodeRec) == kRecBytes, "records_reach counts in records of this size");
 // A scene of few instances as a list (bnh::flat_instances): what a ray needs
 // to find the instances whose bounds it meets without the TLAS.
 // 32: the bits of one register hold a ray's instances; testing all of them
@@ -174,7 +173,7 @@ struct DevScene {
     int exact_only;             // scene has non-finite geometry: exact slab tests only
     const FlatScene* flat;      // null: the scene is traversed through its TLAS
     const NodeRec *trecs, *recs;   // interior nodes of the TLAS and of the BLAS
-    int mode;                   // kNodes: more items than a reference can number; kRecs; kList: flat is set
+    int mode;                   // kNodes: more than records can stand for (records_reach); kRecs; kList: flat is set
     int n_insts, n_tlas;
 };
 
@@ -236,7 +235,7 @@ __device__ __forceinline__ bool sphere_hit(float radius, V3 o, V3 d, float t, fl
 
 struct NodeView { V3 lo, hi; int word; int leaf, axis, count; };
 __device__ __forceinline__ NodeView load_node(const float4* nodes, int i) {
-    float4 a = nodes[2 * i], b = nodes[2 * i + 1];
+    float4 a = nodes[node_at(i, 0)], b = nodes[node_at(i, 1)];
     NodeView n;
     n.lo = {a.x, a.y, a.z};
     n.hi = {a.w, b.x, b.y};

@@ -115,7 +115,7 @@ struct Traversal {
     // root or first triangle, and the order in LDS: config-1 frame 89 -> 84 ms.)
     __device__ __forceinline__ static float4 node_half(const float4* nodes, int i, int half) {
         if (RECS) return *(const float4*)((const char*)nodes + ((uint32_t)i * 32u + 16u * half));
-        return nodes[2 * i + half];
+        return nodes[node_at(i, half)];
     }
     __device__ __forceinline__ static Tri load_tri32(const float* tris, int i) {
         const float* p = (const float*)((const char*)tris + ((uint32_t)i * 32u + (uint32_t)i * 4u));

@@ -380,8 +380,8 @@ int bn_render_batch(bn_ctx* ctx, const bn_batch_item* items, int32_t n, float* c
  *                          than 256 mean 256
  *   "records"              1 (default): scenes uploaded from now on are traversed
  *                          by records of their nodes; 0: by the nodes, as
- *                          scenes of 2^24 - 1 triangles or instances and more
- *                          are.  Hits are the same.
+ *                          scenes of 2^24 - 1 triangles or instances, or of
+ *                          more than 2^26 nodes, are.  Hits are the same.
  *   "mlt_wave_chains"      up to so many PSSMLT chains (default 28672) one wave
  *                          runs each chain's mutations; more advance together
  *                          as a wavefront.  The chains are the same either way.
