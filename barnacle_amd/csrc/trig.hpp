@@ -49,6 +49,7 @@ __host__ __device__ inline void sincos_f(float xf, float& s, float& c) {
     s = n & 1 ? fc : fs;
     c = n & 1 ? fs : fc;
     s = n & 2 ? -s : s;
+    s = xf == 0.0f ? xf : s;                                         // -0 is its own sine
     c = (n + 1) & 2 ? -c : c;
 }
 
