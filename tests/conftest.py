@@ -19,6 +19,19 @@ def orc():
     return oracle.Oracle()
 
 
+# Default of the option "mlt_wave_chains" (Ctx::mlt_wave_chains).
+MLT_WAVE_CHAINS = 28672
+
+
+@pytest.fixture(autouse=True)
+def shipped_chain_limit(request):
+    """Whatever a test sets it to, the next one gets the session's context with
+    the number of chains up to which a wave runs each as it is shipped."""
+    yield
+    if "ctx" in request.fixturenames:
+        request.getfixturevalue("ctx").set_option("mlt_wave_chains", MLT_WAVE_CHAINS)
+
+
 @pytest.fixture(scope="session")
 def ctx():
     from barnacle_amd import native
