@@ -12,19 +12,21 @@
 //  * Bin counts, partition counts and positions are integers; the partition
 //    is the reference's: left items in order from `first`, right items in
 //    order from `last - 1` downwards (Util/BVH.fs:205-217).
-//  * The SAH sweep of a node runs in one thread in the reference's order.
+//  * The SAH sweep of a node folds each prefix and suffix of its bins in a lane
+//    of its own, in the reference's order.
 //
 // Schedule: a task is a node's item range.  Tasks of more than `small` items
 // run level by level over chunks of kChunk items: bounds, bins and the scatter
 // by one block per chunk, the decisions (split axis; split and children) by one
 // wave or block per task.  Task and chunk counts stay on the device: the levels
 // are launched for the most they can have, several levels at a time.  A task of
-// at most `small` items (or at depth 64) is built whole by one wave into a node
-// region of its own.  One block numbers the upper nodes and regions in
-// pre-order, and a last pass writes the flattened nodes.  A level takes 55 us
-// for 240,000 items; with decisions by one thread per task, a copy of the
-// counters and a host synchronisation it took 120, and with the decisions in
-// the block that finishes a task's last chunk 90 (the fences).
+// at most `small` items (or at depth 64, where more than 127 are refused) is
+// built whole by one wave into a node region of its own, of two nodes an item.
+// One block numbers the upper nodes and regions in pre-order, and a last pass
+// writes the flattened nodes.  A level takes 55 us for 240,000 items; with
+// decisions by one thread per task, a copy of the counters and a host
+// synchronisation it took 120, and with the decisions in the block that finishes
+// a task's last chunk 90 (the fences).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -535,7 +537,8 @@ __device__ __forceinline__ bn_bvh_node make_node(const DBox& b, int32_t word, bo
 // folded by 48 lanes, one per bin, side and half of the items, each walking
 // the items in order (24 x 7 values through six lane-reduction steps took the
 // same time for every node: the kernel ran 2.6 ms for 240,000 items, 0.50 ms
-// like this, 0.26 ms for tasks of up to 128 items), and the SAH sweep runs in 22 lanes, one per prefix and suffix.
+// like this, 0.26 ms for tasks of up to 128 items), and the SAH sweep runs in 22
+// lanes, one per prefix and suffix.
 constexpr int kPer = 4;
 constexpr int kSmallMax = 64 * kPer;
 static_assert(kSmallMax >= kLeafMost, "a task at the depth limit fits, whatever the option says");

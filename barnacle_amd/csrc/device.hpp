@@ -140,7 +140,7 @@ struct NodeRec {
     float4 rhi;     // max.yz, reference, unused
 };
 static_assert(sizeof(NodeRec) == kRecBytes, "records_reach counts in records of this size");
-// A scene of few instances as a list (bnh::flat_instances): what a ray needs
+// A scene of few instances as a list (bnh::visit_order): what a ray needs
 // to find the instances whose bounds it meets without the TLAS.
 // 32: the bits of one register hold a ray's instances; testing all of them
 // costs a refill about two wave steps then, and a walk takes more.

@@ -107,8 +107,8 @@ struct Launch {
     hipStream_t stream;
     // Compact path-tracing rounds with stream2 set trace the shadow rays of
     // iteration i on stream2 while stream runs regen, prep and trace_closest
-    // of iteration i + 1; ev_shade / ev_shadow order the two streams.  Not
-    // for rounds captured into a graph.
+    // of iteration i + 1; ev_shade / ev_shadow order the two streams (in a
+    // captured round too: its fork and join are part of the graph).
     hipStream_t stream2;
     hipEvent_t ev_shade, ev_shadow;
     // Compact shading groups each block's continuing paths and shadow rays

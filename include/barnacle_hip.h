@@ -214,9 +214,12 @@ int bn_bvh_build(const float* item_bounds, int32_t n_items,
 
 /* BVHNode.Build (Util/BVH.fs:128-247) on the context's GPU: the same nodes,
  * node order and permutation as bn_bvh_build, bit for bit, for finite item
- * bounds (BN_E_INVALID otherwise; bn_bvh_build takes any).  bn_scene_build
- * builds the BLAS of every mesh with finite triangle bounds this way unless
- * the option "bvh_gpu" is 0. */
+ * bounds (BN_E_INVALID otherwise; bn_bvh_build takes any).  Refused as well:
+ * a leaf of more than 127 items at the depth limit (BN_E_CAPACITY, as by
+ * bn_bvh_build), and a tree of more than 2*n nodes, which a few items with
+ * overflowing centroids can have (BN_E_DEVICE).  bn_scene_build builds the
+ * BLAS of every mesh with finite triangle bounds this way unless the option
+ * "bvh_gpu" is 0. */
 int bn_bvh_build_gpu(bn_ctx* ctx, const float* item_bounds, int32_t n_items,
                      bn_bvh_node* out_nodes, int32_t* out_n_nodes, int32_t* out_perm);
 
